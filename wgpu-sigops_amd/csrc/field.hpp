@@ -50,6 +50,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
+#include <initializer_list>
 #else
 #define SIGOPS_BOUNDS 0
 #endif

@@ -19,6 +19,7 @@
 //     for the careful path, which redoes the item with complete, branching formulas.
 #pragma once
 #include "inv.hpp"
+#include "sfield.hpp"
 
 namespace sigops {
 
@@ -146,6 +147,73 @@ DEV jac jmadd(const jac& P, const fe& x2, const fe& y2, bool& exc) {
   const fe rVX = mont_mul<F>(r, fsub_nr<F, 2, 1>(V, R.X));
   R.Y = fnorm_red<F>(fsub_nr<F, 2, 1>(rVX, mont_mul<F>(fscale_nr(P.Y, 2), J)));
   R.Z = mont_mul<F>(P.Z, fscale_nr(H, 2));                  // (Z1 + H)^2 - Z1Z1 - HH = 2 Z1 H
+  return R;
+}
+
+// ---- the ladder's formulas, on signed arithmetic (sfield.hpp) ----
+// Points carry W = 2Y in place of Y: the doubling's 4XY^2 = X W^2 and 8Y^4 = W^4 / 2 then need no
+// scaling, and W3 = 2 M (S - X3) - W^4 is a difference of two products that takes one reduction, as
+// the addition's W3 = 2 (r (V - X3) - W1 J) is. The subtractions of X3 and the factors 2 and 3 are
+// part of the products' carry chains. VALU instructions (secp256k1): doubling 1,015 against jdbl's
+// 1,280, mixed addition 1,760 against jmadd's 2,018.
+struct jacs {
+  sfe X, W, Z;
+};
+
+// 3M + 4S (a = 0) or 4M + 4S (a = -3), one reduction less: S = X W^2, M = 3X^2 + aZ^4,
+// X3 = M^2 - 2S, W3 = 2 M (S - X3) - W^4, Z3 = W Z
+template <class C>
+DEV jacs sdbl(const jacs& P) {
+  typedef typename C::Fp F;
+  const sfe WW = s_sqr<F>(P.W);
+  const sfe S = s_mul<F>(P.X, WW);
+  sfe Mn;
+  if constexpr (C::A_IS_M3)
+    Mn = s_sqr_diff<F, 3>(P.X, s_sqr<F>(P.Z));  // 3 (X^2 - Z^4)
+  else
+    Mn = s_sqr<F, 3>(P.X);
+  jacs R;
+  R.X = s_sqr_sub<F, 2>(Mn, S);
+  R.W = s_dot_sqr<F>(Mn, s_dbl(s_sub(S, R.X)), WW);
+  R.Z = s_mul<F>(P.W, P.Z);
+  return R;
+}
+
+// madd-2007-bl on (X, W, Z) with the affine (x2, w2 = 2 y2), 8M + 3S with one reduction less:
+// r = w2 Z1^3 - W1. exc is set when H == 0 (P == +-Q). za: the Z that x2 and w2 are scaled by (P.Z,
+// or P.Z times the factor between the accumulator's curve and the table's).
+template <class C>
+DEV jacs smadd_z(const jacs& P, const sfe& za, const sfe& x2, const sfe& w2, bool& exc) {
+  typedef typename C::Fp F;
+  const sfe ZZ = s_sqr<F>(za);
+  const sfe U2 = s_mul<F>(x2, ZZ);
+  const sfe S2 = s_mul<F>(s_mul<F>(w2, za), ZZ);
+  const sfe H = s_sub(U2, P.X);
+  const sfe HH2 = s_sqr<F, 2>(H);
+  exc = exc || s_sqr_maybe_zero<F, 2>(HH2);
+  const sfe J = s_mul<F, 2>(H, HH2);    // 4 H^3
+  const sfe V = s_mul<F, 2>(P.X, HH2);  // 4 X1 H^2
+  const sfe r = s_sub(S2, P.W);
+  jacs R;
+  R.X = s_fold<F>(s_sqr_sub<F, 1>(r, s_add(J, s_dbl(V))));
+  R.W = s_dot<F, 2>(r, s_sub(V, R.X), s_neg(P.W), J);
+  R.Z = s_mul<F, 2>(P.Z, H);
+  return R;
+}
+template <class C>
+DEV jacs smadd(const jacs& P, const sfe& x2, const sfe& w2, bool& exc) {
+  return smadd_z<C>(P, P.Z, x2, w2, exc);
+}
+
+// (X, W, Z) -> (X, Y, Z) of the same point in field.hpp's form: Y = W / 2, so scaled by 2:
+// (4X, 4W, 2Z)
+template <class C>
+DEV jac s_to_jac(const jacs& P) {
+  typedef typename C::Fp F;
+  jac R;
+  R.X = fnorm_red<F>(fscale_nr(s_to_fe<F, 4>(P.X), 4));
+  R.Y = fnorm_red<F>(fscale_nr(s_to_fe<F, 4>(P.W), 4));
+  R.Z = fnorm_red<F>(fscale_nr(s_to_fe<F, 4>(P.Z), 2));
   return R;
 }
 
@@ -469,257 +537,246 @@ DEV u32 digit9(const u32* c, int j) {
 constexpr int GLV_BG9 = 135;  // G streams of secp256k1: 15 windows of 9 bits
 constexpr int R1_BG9 = 261;   // the G stream of P-256: 29 windows of 9 bits
 
-// acc + the odd multiple of the G table's point that 9-bit digit d spells (negated per digit and
-// stream sign); PHI: the entry read as phi(entry) = (beta x, y)
-template <class C, bool PHI, class GTab>
-DEV jac g_add9(const jac& acc, const GTab& gt, u32 d, bool neg_stream, bool& exc) {
+// acc + the entry of the per-lane table that the 4-bit digit d spells (negated per digit and stream
+// sign); PHI: phi(entry) = (beta x, y). e: the entry, loaded ahead by r_load.
+struct r_entry {
+  fe x, w;
+};
+template <bool PHI, class Tab>
+DEV r_entry r_load(const Tab& tab, u32 d) {
+  r_entry e;
+  const u32 idx = ((d < 8) ? ~d : d) & 7u;
+  if constexpr (PHI)
+    tab.load_affine_phi(idx, e.x, e.w);
+  else
+    tab.load_affine(idx, e.x, e.w);
+  return e;
+}
+template <class C>
+DEV jacs r_add(const jacs& acc, const r_entry& e, bool neg, bool& exc) {
   typedef typename C::Fp F;
+  return smadd<C>(acc, s_unraw<F>(e.x), s_neg_if(neg, s_unraw<F>(e.w)), exc);
+}
+
+// acc + the odd multiple of the G table's point that the digit d of WGB bits spells; zeta: the
+// accumulator's coordinates are those of the curve isomorphic by zeta (secp_build_table)
+template <class C, int WGB, bool PHI, class GTab>
+DEV jacs g_add(const jacs& acc, const GTab& gt, u32 d, bool neg_stream, const sfe& zeta, bool& exc) {
+  typedef typename C::Fp F;
+  constexpr u32 HALF = 1u << (WGB - 1);
   fe gx, gy;
-  const u32 idx = ((d < 256) ? ~d : d) & 255u;
+  const u32 idx = ((d < HALF) ? ~d : d) & (HALF - 1u);
   if constexpr (PHI)
     gt.load_phi(idx, gx, gy);
   else
     gt.load(idx, gx, gy);
-  return jmadd<C>(acc, gx, fneg_if<F>((d < 256) != neg_stream, gy), exc);
+  const sfe w = s_neg_if((d < HALF) != neg_stream, s_dbl(s_from(gy)));
+  if constexpr (C::GLV) return smadd_z<C>(acc, s_mul<F>(acc.Z, zeta), s_from(gx), w, exc);
+  return smadd<C>(acc, s_from(gx), w, exc);
 }
 
-// GLV ladder with 9-bit G windows (see secp_ladder_glv): one doubling per iteration over bits
-// 127..0; the R digits enter at multiples of 4, the G digits at multiples of 9
-template <class C, class Tab, class GTab>
-DEV jac secp_ladder_glv9(const secp_pro& o, Tab& tab, const GTab& gt, bool& exc) {
-  typedef typename C::Fp F;
-  u32 cg1[5], cg2[5];
-#pragma unroll
-  for (int i = 0; i < 5; i++) {
-    cg1[i] = o.cg1[i];
-    cg2[i] = o.cg2[i];
-  }
-  // marker bit GLV_BG - 1 = 135 -> GLV_BG9 - 1 = 134 (the halves are below 2^130)
-  cg1[4] = (cg1[4] & ~(1u << 7)) | (1u << 6);
-  cg2[4] = (cg2[4] & ~(1u << 7)) | (1u << 6);
-  jac acc;
-  {
-    fe x, y;
-    tab.load_affine(nibble(o.cr1, 32) - 8, x, y);
-    acc.X = fnorm_red<F>(x);
-    acc.Y = fnorm_red<F>(fneg_if<F>(o.sr1, y));
-    acc.Z = fe_from_const(F::ONE);
-  }
-  {
-    fe bx, ey;
-    tab.load_affine_phi(nibble(o.cr2, 32) - 8, bx, ey);
-    acc = jmadd<C>(acc, bx, fneg_if<F>(o.sr2, ey), exc);
-  }
-  fe x1, y1;
-  u32 c1 = 0;
-#pragma unroll 1
-  for (int p = 127; p >= 0; p--) {
-    if ((p & 3) == 3) {  // the window's first table entry, loaded ahead of its four doublings
-      c1 = nibble(o.cr1, p >> 2);
-      tab.load_affine((c1 < 8 ? ~c1 : c1) & 7u, x1, y1);
-    }
-    acc = jdbl<C>(acc);
-    if ((p & 3) == 0) {
-      const u32 c2 = nibble(o.cr2, p >> 2);
-      fe x2, y2;
-      tab.load_affine_phi((c2 < 8 ? ~c2 : c2) & 7u, x2, y2);  // x2 = beta x
-      acc = jmadd<C>(acc, x1, fneg_if<F>((c1 < 8) != o.sr1, y1), exc);
-      acc = jmadd<C>(acc, x2, fneg_if<F>((c2 < 8) != o.sr2, y2), exc);
-    }
-    if (p % 9 == 0) {
-      acc = g_add9<C, false>(acc, gt, digit9(cg1, p / 9), o.sg1, exc);
-      acc = g_add9<C, true>(acc, gt, digit9(cg2, p / 9), o.sg2, exc);
-    }
-  }
-  return acc;
-}
-
-// P-256 ladder with 9-bit G windows (see secp_ladder): one doubling per iteration over bits
-// 251..0; the R digits enter at multiples of 4, the G digits at multiples of 9 (the top one, at
-// bit 252, with the top R digit)
-template <class C, class Tab, class GTab>
-DEV jac secp_ladder9(const secp_pro& o, Tab& tab, const GTab& gt, bool& exc) {
-  typedef typename C::Fp F;
-  u32 cg[9];
-#pragma unroll
-  for (int i = 0; i < 8; i++) cg[i] = o.c1[i];
-  cg[7] &= 0x7fffffffu;  // marker bit 255 -> R1_BG9 - 1 = 260 (u1 < n < 2^256)
-  cg[8] = 1u << (R1_BG9 - 1 - 256);
-  jac acc;
-  {
-    fe x, y;
-    tab.load_affine(nibble(o.c2, 63) - 8, x, y);
-    acc.X = fnorm_red<F>(x);
-    acc.Y = fnorm_red<F>(y);
-    acc.Z = fe_from_const(F::ONE);
-  }
-  acc = g_add9<C, false>(acc, gt, digit9(cg, 28), o.g_neg, exc);
-  fe ex, ey;
-  u32 c = 0;
-#pragma unroll 1
-  for (int p = 251; p >= 0; p--) {
-    if ((p & 3) == 3) {
-      c = nibble(o.c2, p >> 2);
-      tab.load_affine((c < 8 ? ~c : c) & 7u, ex, ey);
-    }
-    acc = jdbl<C>(acc);
-    if ((p & 3) == 0) acc = jmadd<C>(acc, ex, fneg_if<F>(c < 8, ey), exc);
-    if (p % 9 == 0) acc = g_add9<C, false>(acc, gt, digit9(cg, p / 9), o.g_neg, exc);
-  }
-  return acc;
-}
-
-// GLV ladder (secp256k1): Q = h1 G + h2 phi(G) + h3 R + h4 phi(R) on one doubling chain of 132
-// bits, with phi(x, y) = (beta x, y): both tables store beta x beside x (Tab::load_affine_phi,
-// GTab::load_phi read (beta x, y)). R streams use 33
-// windows of 4 bits over the per-lane table of odd multiples of R; G streams 17 windows of 8 bits
-// over the table of odd multiples of G, added at every second R window.
-template <class C, class Tab, class GTab>
-DEV jac secp_ladder_glv(const secp_pro& o, Tab& tab, const GTab& gt, bool& exc) {
-  typedef typename C::Fp F;
-  // top windows: every stream's top digit is positive; only the stream signs apply
-  // the accumulator enters jmadd as a subtrahend, so its coordinates are folded to < (1 + 2^-19) M
-  jac acc;
-  {
-    fe x, y;
-    tab.load_affine(nibble(o.cr1, 32) - 8, x, y);
-    acc.X = fnorm_red<F>(x);
-    acc.Y = fnorm_red<F>(fneg_if<F>(o.sr1, y));
-    acc.Z = fe_from_const(F::ONE);
-  }
-  {
-    fe bx, ey;
-    tab.load_affine_phi(nibble(o.cr2, 32) - 8, bx, ey);
-    acc = jmadd<C>(acc, bx, fneg_if<F>(o.sr2, ey), exc);
-  }
-#pragma unroll 1
-  for (int i = 32; i >= 0; i--) {
-    if (i < 32) {
-      // the first table load is issued before the doublings and the second before the first
-      // addition; each is hidden behind that work without keeping both entries live
-      const u32 c1 = nibble(o.cr1, i), c2 = nibble(o.cr2, i);
-      fe x1, y1, x2, y2;
-      tab.load_affine((c1 < 8 ? ~c1 : c1) & 7u, x1, y1);
-#pragma unroll 1
-      for (int d = 0; d < 4; d++) acc = jdbl<C>(acc);
-      tab.load_affine_phi((c2 < 8 ? ~c2 : c2) & 7u, x2, y2);  // x2 = beta x
-      acc = jmadd<C>(acc, x1, fneg_if<F>((c1 < 8) != o.sr1, y1), exc);
-      acc = jmadd<C>(acc, x2, fneg_if<F>((c2 < 8) != o.sr2, y2), exc);
-    }
-    if ((i & 1) == 0) {
-      fe gx, gy;
-      const u32 b1 = byte8(o.cg1, i >> 1), b2 = byte8(o.cg2, i >> 1);
-      gt.load(((b1 < 128) ? ~b1 : b1) & 127u, gx, gy);
-      gy = fneg_if<F>((b1 < 128) != o.sg1, gy);
-      acc = jmadd<C>(acc, gx, gy, exc);
-      gt.load_phi(((b2 < 128) ? ~b2 : b2) & 127u, gx, gy);  // gx = beta x
-      gy = fneg_if<F>((b2 < 128) != o.sg2, gy);
-      acc = jmadd<C>(acc, gx, gy, exc);
-    }
-  }
-  return acc;
-}
-
-// Per-lane table of the odd multiples (2e + 1) P, e = 0..7, made affine with one inversion
-// (Montgomery's simultaneous inversion), so that the ladder adds its entries with the mixed formula
-// (8M + 3S instead of 11M + 5S per addition). The entries are built in Jacobian form with the
-// running product of the Z coordinates before them stored alongside; one inversion of the full
-// product then yields every 1/Z on the way back down, and each entry is rewritten in place as
-// (x, y). Tab: store_full(e, jac, before) / load_full(e, jac&, before&) and store_affine(e, x, y)
-// / load_affine(e, x&, y&).
+// Per-lane table of the odd multiples (2e + 1) P, e = 0..7, as affine (x, w = 2y) on a curve where
+// all of them are, so that the ladder adds its entries with the mixed formula (8M + 3S instead of
+// 11M + 5S per addition).
 // The entries are built on an isomorphic curve where 2P is affine, so the seven additions are
-// mixed ones too: with 2P = (X2, Y2, Z2), the map (x, y) -> (Z2^2 x, Z2^3 y) takes the curve to
-// y^2 = x^3 + a Z2^4 x + b Z2^6, 2P to the affine (X2, Y2) and P to (Z2^2 x, Z2^3 y). The
-// addition formulas do not involve a or b. A Jacobian (X, Y, Z) there is (X, Y, Z Z2) on the
-// curve, so Z2 joins the product that is inverted.
+// mixed ones too: with 2P = (X2, W2, Z2), the map (x, y) -> (Z2^2 x, Z2^3 y) takes the curve to
+// y^2 = x^3 + a Z2^4 x + b Z2^6, 2P to the affine (X2, W2) and P to (Z2^2 x, Z2^3 y). The addition
+// formulas do not involve a or b. A Jacobian (X, W, Z) there is (X, W, Z Z2) on the curve.
+// Then, from the last entry down, with the factors zr_e = Z_e / Z_(e-1) that the additions give:
+//   * a = 0 (secp256k1): the entries are scaled to the last one's Z, (X rho^2, W rho^3) with
+//     rho = Z_7 / Z_e, which makes them affine on the curve isomorphic by zeta = Z2 Z_7. The ladder
+//     runs there (the doubling does not involve b) and multiplies its Z by zeta at the end, so no
+//     inversion is needed (a divstep inversion is 20,000 instructions, 7% of an item). beta x is
+//     stored beside each entry for the phi(R) stream.
+//   * a = -3 (P-256): the doubling needs a, so the entries are made affine on the curve itself by
+//     one inversion of Z2 Z_7 (Montgomery's trick, with the same factors).
+// Tab: store_full(e, (X, W, zr), unused) / load_full and store_affine(e, x, w) / load_affine (and
+// the _phi forms with beta x). Returns zeta (1 for P-256).
 template <class C, class Tab>
-DEV void secp_build_table(const secp_pro& o, Tab& tab, bool& exc) {
+DEV sfe secp_build_table(const secp_pro& o, Tab& tab, bool& exc) {
   typedef typename C::Fp F;
-  jac P;
-  P.X = o.rx;
-  P.Y = o.ry;
-  P.Z = fe_from_const(F::ONE);
-  const jac P2 = jdbl<C>(P);
-  // secp256k1 (GLV): beta x beside each entry, for the phi(R) stream
-  const fe beta = C::GLV ? fe_from_const(K1_BETA) : fe_zero();
-  if constexpr (C::GLV)
-    tab.store_affine_phi(0, P.X, P.Y, mont_mul<F>(P.X, beta));
-  else
-    tab.store_affine(0, P.X, P.Y);
-  // P on the isomorphic curve; the accumulator enters jmadd as a subtrahend, so it is folded
-  const fe zz = mont_sqr<F>(P2.Z);
-  jac T;
-  T.X = fnorm_red<F>(mont_mul<F>(P.X, zz));
-  T.Y = fnorm_red<F>(mont_mul<F>(P.Y, mont_mul<F>(zz, P2.Z)));
+  jacs P;
+  P.X = s_from(o.rx);
+  P.W = s_from(fnorm_red<F>(fscale_nr(o.ry, 2)));
+  P.Z = s_from(fe_from_const(F::ONE));
+  const jacs P2 = sdbl<C>(P);
+  const sfe beta = s_from(C::GLV ? fe_from_const(K1_BETA) : fe_zero());
+  const sfe zz = s_sqr<F>(P2.Z);
+  jacs T;
+  T.X = s_mul<F>(P.X, zz);
+  T.W = s_mul<F>(P.W, s_mul<F>(zz, P2.Z));
   T.Z = P.Z;
-  fe before = P.Z;  // Z_1 * ... * Z_(e-1), isomorphic-curve Z coordinates
+  tab.store_full(0, jac{s_raw(T.X), s_raw(T.W), s_raw(T.Z)}, fe_zero());
 #pragma unroll 1
   for (int e = 1; e < 8; e++) {
-    T = jmadd<C>(T, P2.X, P2.Y, exc);
-    tab.store_full(e, T, before);
-    before = mont_mul<F>(before, T.Z);
+    // smadd with Z1 = 1 tracked apart: Z_e = Z_(e-1) zr_e with zr_e = 2H
+    const sfe ZZ = s_sqr<F>(T.Z);
+    const sfe H = s_sub(s_mul<F>(P2.X, ZZ), T.X);
+    const sfe r = s_sub(s_mul<F>(s_mul<F>(P2.W, T.Z), ZZ), T.W);
+    const sfe HH2 = s_sqr<F, 2>(H);
+    exc = exc || s_sqr_maybe_zero<F, 2>(HH2);
+    const sfe J = s_mul<F, 2>(H, HH2);
+    const sfe V = s_mul<F, 2>(T.X, HH2);
+    // 2H as a normalised value: 2H times R times R^-1
+    const sfe zr = s_mul<F, 2>(H, P.Z);
+    T.X = s_fold<F>(s_sqr_sub<F, 1>(r, s_add(J, s_dbl(V))));
+    T.W = s_dot<F, 2>(r, s_sub(V, T.X), s_neg(T.W), J);
+    T.Z = s_mul<F>(T.Z, zr);
+    tab.store_full(e, jac{s_raw(T.X), s_raw(T.W), s_raw(zr)}, fe_zero());
   }
-  fe inv = finv<F>(mont_mul<F>(before, P2.Z));  // 1 / (Z2 * Z_1 * ... * Z_7)
+  sfe zeta = s_mul<F>(T.Z, P2.Z);  // Z2 Z_7
+  sfe rho;
+  if constexpr (C::GLV)
+    rho = P.Z;
+  else
+    rho = s_from(finv<F>(s_to_fe<F, 4>(zeta)));  // 1 / (Z2 Z_7)
 #pragma unroll 1
-  for (int e = 7; e >= 1; e--) {
-    jac E;
-    fe b;
-    tab.load_full(e, E, b);
-    const fe zi = mont_mul<F>(inv, b);  // 1 / (Z2 * Z_e), the curve's 1 / Z
-    inv = mont_mul<F>(inv, E.Z);        // 1 / (Z2 * Z_1 * ... * Z_(e-1))
-    const fe zi2 = mont_sqr<F>(zi);
-    const fe ax = mont_mul<F>(E.X, zi2), ay = mont_mul<F>(E.Y, mont_mul<F>(zi2, zi));
+  for (int e = 7; e >= 0; e--) {
+    jac E;  // (X, W, zr)
+    fe unused;
+    tab.load_full(e, E, unused);
+    const sfe r2 = s_sqr<F>(rho);
+    const sfe ax = s_mul<F>(s_unraw<F>(E.X), r2);
+    const sfe aw = s_mul<F>(s_unraw<F>(E.Y), s_mul<F>(r2, rho));
+    rho = s_mul<F>(rho, s_unraw<F>(E.Z));
     if constexpr (C::GLV)
-      tab.store_affine_phi(e, ax, ay, mont_mul<F>(ax, beta));
+      tab.store_affine_phi(e, s_raw(ax), s_raw(aw), s_raw(s_mul<F>(ax, beta)));
     else
-      tab.store_affine(e, ax, ay);
+      tab.store_affine(e, s_raw(ax), s_raw(aw));
   }
+  return zeta;
 }
 
-// R-table stored per lane (secp_build_table). GTab provides load(idx, fe& x, fe& y) for the odd
-// multiples (2 idx + 1) G: 128 of them for fixed-base windows of WGB = 8 bits, 256 for 9.
-template <class C, int WGB = 8, class Tab, class GTab>
-DEV jac secp_ladder(const secp_pro& o, Tab& tab, const GTab& gt, bool& exc) {
+// the ladder's first point: the entry of the top digit (always positive), with the stream's sign
+template <class C, class Tab>
+DEV jacs r_first(const Tab& tab, u32 d, bool neg) {
   typedef typename C::Fp F;
-  static_assert(WGB == 8 || WGB == 9, "fixed-base windows of 8 or 9 bits");
-  secp_build_table<C>(o, tab, exc);
-  if constexpr (WGB == 9) {
-    if constexpr (C::GLV)
-      return secp_ladder_glv9<C>(o, tab, gt, exc);
-    else
-      return secp_ladder9<C>(o, tab, gt, exc);
-  }
-  if constexpr (C::GLV) return secp_ladder_glv<C>(o, tab, gt, exc);
-  // top R digit is always positive (C's bit 255 is set); the accumulator enters jmadd as a
-  // subtrahend, so its coordinates are folded to < (1 + 2^-19) M
-  jac acc;
-  {
-    fe x, y;
-    tab.load_affine(nibble(o.c2, 63) - 8, x, y);
-    acc.X = fnorm_red<F>(x);
-    acc.Y = fnorm_red<F>(y);
-    acc.Z = fe_from_const(F::ONE);
-  }
+  fe x, w;
+  tab.load_affine(d - 8, x, w);
+  return jacs{s_unraw<F>(x), s_carry(s_neg_if(neg, s_unraw<F>(w))), s_from(fe_from_const(F::ONE))};
+}
+
+// Q = h1 G + h2 phi(G) + h3 R + h4 phi(R) on one doubling chain of 132 bits (secp256k1; phi(x, y) =
+// (beta x, y), both tables store beta x beside x), or u1 G + u2 R on one of 256 bits (P-256). R
+// streams: 33 (64) windows of 4 bits over the per-lane table of odd multiples of R. G streams: WGB
+// = 8 or 9 bits over the table gt of odd multiples of G, or WGB = 0: none, the caller adds u1 G
+// (secp_comb). Every window adds exactly one entry.
+template <class C, int WGB, class Tab, class GTab>
+DEV jacs secp_ladder_s(const secp_pro& o, Tab& tab, const GTab& gt, bool& exc) {
+  typedef typename C::Fp F;
+  static_assert(WGB == 0 || WGB == 8 || WGB == 9, "fixed-base windows of 8 or 9 bits, or none");
+  const sfe zeta = secp_build_table<C>(o, tab, exc);
+  jacs acc;
+  if constexpr (C::GLV) {
+    u32 cg1[5], cg2[5];
+#pragma unroll
+    for (int i = 0; i < 5; i++) {
+      cg1[i] = o.cg1[i];
+      cg2[i] = o.cg2[i];
+    }
+    if constexpr (WGB == 9) {  // marker bit GLV_BG - 1 = 135 -> GLV_BG9 - 1 = 134 (the halves are below 2^130)
+      cg1[4] = (cg1[4] & ~(1u << 7)) | (1u << 6);
+      cg2[4] = (cg2[4] & ~(1u << 7)) | (1u << 6);
+    }
+    acc = r_first<C>(tab, nibble(o.cr1, 32), o.sr1);
+    {
+      const u32 d = nibble(o.cr2, 32);
+      acc = r_add<C>(acc, r_load<true>(tab, d), o.sr2, exc);
+    }
+    if constexpr (WGB == 8) {
+      acc = g_add<C, WGB, false>(acc, gt, byte8(cg1, 16), o.sg1, zeta, exc);
+      acc = g_add<C, WGB, true>(acc, gt, byte8(cg2, 16), o.sg2, zeta, exc);
+    }
+    // the first table load of a window is issued before its doublings and the second before the
+    // first addition; each is hidden behind that work without keeping both entries live
+    if constexpr (WGB == 9) {  // one doubling per trip: R digits at multiples of 4, G digits at multiples of 9
+      r_entry e1;
+      u32 c1 = 0;
 #pragma unroll 1
-  for (int i = 62; i >= 0; i--) {
-    // issue the HBM load of this window's table entry before the doublings, which hide its latency
-    const u32 c = nibble(o.c2, i);
-    const bool neg = c < 8;
-    fe ex, ey;
-    tab.load_affine((neg ? ~c : c) & 7u, ex, ey);
+      for (int p = 127; p >= 0; p--) {
+        if ((p & 3) == 3) {
+          c1 = nibble(o.cr1, p >> 2);
+          e1 = r_load<false>(tab, c1);
+        }
+        acc = sdbl<C>(acc);
+        if ((p & 3) == 0) {
+          const u32 c2 = nibble(o.cr2, p >> 2);
+          const r_entry e2 = r_load<true>(tab, c2);
+          acc = r_add<C>(acc, e1, (c1 < 8) != o.sr1, exc);
+          acc = r_add<C>(acc, e2, (c2 < 8) != o.sr2, exc);
+        }
+        if (p % 9 == 0) {
+          acc = g_add<C, WGB, false>(acc, gt, digit9(cg1, p / 9), o.sg1, zeta, exc);
+          acc = g_add<C, WGB, true>(acc, gt, digit9(cg2, p / 9), o.sg2, zeta, exc);
+        }
+      }
+    } else {
 #pragma unroll 1
-    for (int d = 0; d < 4; d++) acc = jdbl<C>(acc);
-    acc = jmadd<C>(acc, ex, fneg_if<F>(neg, ey), exc);
-    if ((i & 1) == 0) {
-      const u32 cg = byte8(o.c1, i >> 1);
-      const bool gneg = (cg < 128) != o.g_neg;
-      fe gx, gy;
-      gt.load(((cg < 128) ? ~cg : cg) & 127u, gx, gy);
-      gy = fneg_if<F>(gneg, gy);
-      acc = jmadd<C>(acc, gx, gy, exc);
+      for (int i = 31; i >= 0; i--) {
+        const u32 c1 = nibble(o.cr1, i), c2 = nibble(o.cr2, i);
+        const r_entry e1 = r_load<false>(tab, c1);
+#pragma unroll 1
+        for (int d = 0; d < 4; d++) acc = sdbl<C>(acc);
+        const r_entry e2 = r_load<true>(tab, c2);
+        acc = r_add<C>(acc, e1, (c1 < 8) != o.sr1, exc);
+        acc = r_add<C>(acc, e2, (c2 < 8) != o.sr2, exc);
+        if constexpr (WGB == 8) {
+          if ((i & 1) == 0) {
+            acc = g_add<C, WGB, false>(acc, gt, byte8(cg1, i >> 1), o.sg1, zeta, exc);
+            acc = g_add<C, WGB, true>(acc, gt, byte8(cg2, i >> 1), o.sg2, zeta, exc);
+          }
+        }
+      }
+    }
+    acc.Z = s_mul<F>(acc.Z, zeta);
+  } else {
+    u32 cg[9];
+#pragma unroll
+    for (int i = 0; i < 8; i++) cg[i] = o.c1[i];
+    cg[8] = 0;
+    if constexpr (WGB == 9) {
+      cg[7] &= 0x7fffffffu;  // marker bit 255 -> R1_BG9 - 1 = 260 (u1 < n < 2^256)
+      cg[8] = 1u << (R1_BG9 - 1 - 256);
+    }
+    acc = r_first<C>(tab, nibble(o.c2, 63), false);
+    if constexpr (WGB == 9) {
+      acc = g_add<C, WGB, false>(acc, gt, digit9(cg, 28), o.g_neg, zeta, exc);
+      r_entry e;
+      u32 c = 0;
+#pragma unroll 1
+      for (int p = 251; p >= 0; p--) {
+        if ((p & 3) == 3) {
+          c = nibble(o.c2, p >> 2);
+          e = r_load<false>(tab, c);
+        }
+        acc = sdbl<C>(acc);
+        if ((p & 3) == 0) acc = r_add<C>(acc, e, c < 8, exc);
+        if (p % 9 == 0) acc = g_add<C, WGB, false>(acc, gt, digit9(cg, p / 9), o.g_neg, zeta, exc);
+      }
+    } else {
+#pragma unroll 1
+      for (int i = 62; i >= 0; i--) {
+        // the HBM load of this window's entry is issued before the doublings, which hide its latency
+        const u32 c = nibble(o.c2, i);
+        const r_entry e = r_load<false>(tab, c);
+#pragma unroll 1
+        for (int d = 0; d < 4; d++) acc = sdbl<C>(acc);
+        acc = r_add<C>(acc, e, c < 8, exc);
+        if constexpr (WGB == 8) {
+          if ((i & 1) == 0) acc = g_add<C, WGB, false>(acc, gt, byte8(cg, i >> 1), o.g_neg, zeta, exc);
+        }
+      }
     }
   }
   return acc;
+}
+
+// secp_ladder_s with its result in field.hpp's form. R-table stored per lane (secp_build_table).
+// GTab provides load(idx, fe& x, fe& y) for the odd multiples (2 idx + 1) G: 128 of them for
+// fixed-base windows of WGB = 8 bits, 256 for 9.
+template <class C, int WGB = 8, class Tab, class GTab>
+DEV jac secp_ladder(const secp_pro& o, Tab& tab, const GTab& gt, bool& exc) {
+  return s_to_jac<C>(secp_ladder_s<C, WGB>(o, tab, gt, exc));
 }
 
 // careful path: Q = u1*G + u2*R by double-and-add with the complete law (slow, branching)
