@@ -1,0 +1,90 @@
+"""Every path a plain call can take by its size: four lanes per item up to 16,384 items, one lane per
+item with shared inversions above, around the sizes where the path, the workgroups or the stages'
+lanes change. Each call holds the edge cases and corrupted generated items, repeated to the size, and
+every result is compared with the oracle's."""
+import numpy as np
+import pytest
+
+import edge_cases
+import oracle_lib as O
+from sigops_pkg import sigops
+
+pytestmark = pytest.mark.gpu
+SIZES = [1, 15, 16, 17, 1000, 16384, 16385, 65537]
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = sigops.Context()
+    yield c
+    c.close()
+
+
+def _bytes(rows, width):
+    return np.frombuffer(b"".join(rows), np.uint8).reshape(-1, width)
+
+
+def _at(n, count, seed):
+    """n positions in a list of count items: all of them in order (as many as fit), then random ones"""
+    rng = np.random.default_rng(seed)
+    return np.concatenate([np.arange(min(n, count)), rng.integers(0, count, max(0, n - count))])
+
+
+@pytest.mark.parametrize("curve", [0, 1])
+def test_recover_sizes(ctx, curve):
+    cases = edge_cases.secp_cases(curve)
+    exp = edge_cases.secp_expected(curve, cases)
+    s, d, _, _ = O.gen_secp(curve, 31, 300, corrupt_ppm=200000)
+    o, t = O.recover_batch(curve, s, d)
+    sigs = np.concatenate([_bytes([c[1] for c in cases], 64), s])
+    digs = np.concatenate([_bytes([c[2] for c in cases], 32), d])
+    out = np.concatenate([_bytes([e[1] for e in exp], 64), o])
+    st = np.concatenate([np.array([e[0] for e in exp], np.uint8), t])
+    fn = ctx.secp256k1_recover if curve == 0 else ctx.secp256r1_recover
+    for n in SIZES:
+        print(f"recover curve={curve} n={n}", flush=True)
+        at = _at(n, len(st), n)
+        got, gst = fn(sigs[at], digs[at])
+        assert np.array_equal(gst, st[at]) and np.array_equal(got, out[at]), n
+
+
+@pytest.mark.parametrize("curve", [0, 1])
+def test_verify_sizes(ctx, curve):
+    cases = edge_cases.secp_verify_cases(curve)
+    s, d, p, _ = O.gen_secp(curve, 32, 300, corrupt_ppm=200000)
+    st = np.concatenate([np.array(edge_cases.secp_verify_expected(curve, cases), np.uint8),
+                         O.secp_verify_batch(curve, s, d, p)])
+    sigs = np.concatenate([_bytes([c[1] for c in cases], 64), s])
+    digs = np.concatenate([_bytes([c[2] for c in cases], 32), d])
+    pubs = np.concatenate([_bytes([c[3] for c in cases], 64), p])
+    fn = ctx.secp256k1_verify if curve == 0 else ctx.secp256r1_verify
+    for n in SIZES:
+        print(f"verify curve={curve} n={n}", flush=True)
+        at = _at(n, len(st), n)
+        valid, gst = fn(sigs[at], digs[at], pubs[at])
+        assert np.array_equal(gst, st[at]) and np.array_equal(valid, st[at] == 0), n
+
+
+@pytest.mark.parametrize("strict", [False, True])
+def test_ed25519_sizes(ctx, strict):
+    # name, signature, key, message
+    cases = edge_cases.ed_cases() + edge_cases.ed_strict_cases()
+    oracle = O.ed25519_verify_strict if strict else O.ed25519_verify
+    good = np.array([bool(oracle(c[1], c[2], c[3])) for c in cases])
+    sigs, keys = [c[1] for c in cases], [c[2] for c in cases]
+    msgs = [bytes(c[3]) for c in cases]
+    off = np.concatenate([[0], np.cumsum(np.arange(300) * 7 % 500)]).astype(np.uint64)
+    s, k, m, _ = O.gen_ed25519(33, 300, off, corrupt_ppm=200000)
+    good = np.concatenate([good, (O.verify_strict_batch if strict else O.verify_batch)(s, k, m, off).astype(bool)])
+    sigs = np.concatenate([_bytes(sigs, 64), s])
+    keys = np.concatenate([_bytes(keys, 32), k])
+    msgs += [m[int(off[i]):int(off[i + 1])].tobytes() for i in range(300)]
+    lens = np.array([len(x) for x in msgs])
+    for n in SIZES:
+        print(f"ed25519 strict={strict} n={n}", flush=True)
+        at = _at(n, len(good), n)
+        moff = np.concatenate([[0], np.cumsum(lens[at])]).astype(np.uint64)
+        data = np.frombuffer(b"".join(msgs[i] for i in at), np.uint8)
+        valid, st = ctx.ed25519_verify(sigs[at], keys[at], data, moff, strict=strict)
+        assert np.array_equal(valid, good[at]), n
+        assert np.array_equal(st == 0, good[at]), n

@@ -6,10 +6,12 @@
 //      Ed25519 by SHA-512 block count, so the lanes of a wavefront hash equally long messages), each
 //      bucket padded to whole tiles; the buckets are processed in the context's order (its rank
 //      table: secp256r1, secp256k1, then Ed25519 by decreasing block count);
-//   2. k_batch_run is persistent: every wavefront pulls the next tile (64 x tile_rounds items of
+//   2. k_batch_scalars computes u1 and u2 of the secp items, several per lane with one inversion;
+//   3. k_batch_run is persistent: every wavefront pulls the next tile (64 x tile_rounds items of
 //      one bucket) from an atomic counter, so the scheme is uniform across the wavefront and load
 //      balances dynamically; it runs the same per-item code as the plain kernels;
-//   3. k_batch_careful finishes secp items whose fast ladder met an exceptional addition.
+//   4. k_batch_finish makes the recovered keys affine, again several per lane with one inversion;
+//   5. k_batch_careful finishes secp items whose fast ladder met an exceptional addition.
 // The batch's buffers and n are read from device memory (BatchIO), so the captured graph of these
 // launches replays for any buffers and any n up to the context capacity.
 #include "kernels_impl.hpp"
@@ -37,6 +39,7 @@ struct BatchArgs {
   u32* pend_count;
   const u8* rank;   // bucket -> processing rank
   u32 tile_items;   // 64 * tile_rounds
+  ItemScratch sc;   // secp items, by position in `order`
 };
 
 // Every kernel starts with bind_io: the per-call buffers come from device memory (written on the
@@ -154,15 +157,56 @@ DEV void store16(uint4* p, const u32 o[16]) {
   for (int c = 0; c < 4; c++) p[c] = make_uint4(o[4 * c], o[4 * c + 1], o[4 * c + 2], o[4 * c + 3]);
 }
 
-template <class C, int WGB, class GT>
-DEV void batch_secp_item(const BatchArgs& a, u32 i, STabDev& tab, const GT& gt) {
-  u32 sr[16], dr[8], o[16];
+// a secp item up to its Jacobian result in the scratch (k_batch_finish makes it affine)
+template <class C>
+DEV void batch_secp_item(const BatchArgs& a, u32 i, u32 pos, STabDev& tab, const CombDev& comb) {
+  u32 sr[16];
   load_words(a.sigs + 4 * (u64)i, sr, 4);
-  load_words(a.aux + 2 * (u64)i, dr, 2);
-  const u32 st = secp_item<C, WGB>(sr, dr, tab, gt, o);
-  if (st == ST_PENDING) a.pend_list[atomicAdd(a.pend_count, 1u)] = i;
-  store16(a.out + 4 * (u64)i, o);
-  a.status[i] = (u8)st;
+  if (secp_recover_point<C>(sr, pos, a.sc, tab, comb) == ST_PENDING) a.pend_list[atomicAdd(a.pend_count, 1u)] = i;
+}
+
+// the positions of one curve's tiles as items of the stages around the persistent kernel
+struct OrderItems {
+  const BatchArgs& a;
+  DEV bool sig(u32 p, u32* w) const {
+    const u32 i = a.order[p];
+    if (i == DUMMY) return false;
+    load_words(a.sigs + 4 * (u64)i, w, 4);
+    return true;
+  }
+  DEV bool digest(u32 p, u32* w) const {
+    const u32 i = a.order[p];
+    if (i == DUMMY) return false;
+    load_words(a.aux + 2 * (u64)i, w, 2);
+    return true;
+  }
+  DEV uint4* out(u32 p) const {
+    const u32 i = a.order[p];
+    return i == DUMMY ? nullptr : a.out + 4 * (u64)i;
+  }
+  DEV void status(u32 p, u32 st) const { a.status[a.order[p]] = (u8)st; }
+};
+
+// u1, u2 of every secp item (secp_scalars_lane), after the bucketing
+__global__ __launch_bounds__(256, SIGOPS_WAVES_PER_EU) void k_batch_scalars(BatchArgs a) {
+  bind_io(a);
+  const u32 id = blockIdx.x * blockDim.x + threadIdx.x, lanes = gridDim.x * blockDim.x;
+  const u32 rk = a.rank[BUCKET_K1], rr = a.rank[BUCKET_R1];
+  secp_scalars_lane<CurveK1, false>(a.tile_start[rk] * a.tile_items + id, lanes, a.tile_start[rk + 1] * a.tile_items,
+                                    OrderItems{a}, a.sc);
+  secp_scalars_lane<CurveR1, false>(a.tile_start[rr] * a.tile_items + id, lanes, a.tile_start[rr + 1] * a.tile_items,
+                                    OrderItems{a}, a.sc);
+}
+
+// affine keys and statuses of every secp item, after the persistent kernel
+__global__ __launch_bounds__(256, SIGOPS_WAVES_PER_EU) void k_batch_finish(BatchArgs a) {
+  bind_io(a);
+  const u32 id = blockIdx.x * blockDim.x + threadIdx.x, lanes = gridDim.x * blockDim.x;
+  const u32 rk = a.rank[BUCKET_K1], rr = a.rank[BUCKET_R1];
+  secp_finish_lane<CurveK1>(a.tile_start[rk] * a.tile_items + id, lanes, a.tile_start[rk + 1] * a.tile_items,
+                            OrderItems{a}, a.sc);
+  secp_finish_lane<CurveR1>(a.tile_start[rr] * a.tile_items + id, lanes, a.tile_start[rr + 1] * a.tile_items,
+                            OrderItems{a}, a.sc);
 }
 
 // The schemes a persistent launch serves (template mask): the mixed batch serves all three; the
@@ -174,24 +218,18 @@ constexpr u32 RUN_MIXED = RUN_K1 | RUN_R1 | RUN_ED;
 // WAVES: waves per SIMD the kernel is built for, which sets its register budget per lane (512 /
 // WAVES): 2 by default (256 registers, some values spilled to scratch memory); 1 lets the
 // compiler keep them in registers (accumulation registers included) with half the waves to hide
-// latencies. WGB: the secp streams' fixed-base window, 8 bits (128 odd multiples of G staged in
-// LDS) or 9 (256: 63.5 KB of LDS per workgroup, still two per CU). The autotuner measures them.
-template <u32 MASK, int WAVES = SIGOPS_WAVES_PER_EU, int WGB = 8>
-__global__ __launch_bounds__(256, WAVES) void k_batch_run(BatchArgs a, const uint4* __restrict__ gk1,
-                                                   const uint4* __restrict__ gr1, const uint4* __restrict__ gb,
+// latencies. The autotuner measures them.
+template <u32 MASK, int WAVES = SIGOPS_WAVES_PER_EU>
+__global__ __launch_bounds__(256, WAVES) void k_batch_run(BatchArgs a, const uint4* __restrict__ comb_k1,
+                                                   const uint4* __restrict__ comb_r1, const uint4* __restrict__ gb,
                                                    uint4* __restrict__ lane_tab, u32 slots) {
   static_assert(!((MASK & RUN_ED) && (MASK & RUN_ED_STRICT)), "one Ed25519 rule set per launch");
   constexpr bool K1 = MASK & RUN_K1, R1 = MASK & RUN_R1, ED = MASK & (RUN_ED | RUN_ED_STRICT);
-  constexpr u32 GN = WGB == 9 ? GTAB9_ENTRIES : GTAB_ENTRIES;
   // the kernels that serve only Ed25519 run the lattice-reduced check (both fixed-base tables)
   constexpr bool LAT = ED && !K1 && !R1;
   constexpr u32 BN = LAT ? BTAB_UINT4 : BTAB_ENTRIES * 7;
   bind_io(a);
-  __shared__ uint4 s_k1[K1 ? GN * gtab_chunks<CurveK1>() : 1];
-  __shared__ uint4 s_r1[R1 ? GN * gtab_chunks<CurveR1>() : 1];
   __shared__ uint4 s_b[ED ? BN : 1];
-  if constexpr (K1) stage_gtab<CurveK1, GN>(s_k1, gk1);
-  if constexpr (R1) stage_gtab<CurveR1, GN>(s_r1, gr1);
   if constexpr (ED)
     for (int t = threadIdx.x; t < BN; t += blockDim.x) s_b[t] = gb[t];
   __syncthreads();
@@ -218,12 +256,13 @@ __global__ __launch_bounds__(256, WAVES) void k_batch_run(BatchArgs a, const uin
       if (a.rank[q] == r) b = q;
     b = __builtin_amdgcn_readfirstlane(b);
     for (u32 k = 0; k < a.tile_items; k += 64) {
-      const u32 i = a.order[(u64)t * a.tile_items + k + lane];
+      const u32 pos = t * a.tile_items + k + lane;
+      const u32 i = a.order[pos];
       if (i == DUMMY) continue;
       if (K1 && b == BUCKET_K1) {
-        if constexpr (K1) batch_secp_item<CurveK1, WGB>(a, i, jt, GTabOf<CurveK1>{s_k1});
+        if constexpr (K1) batch_secp_item<CurveK1>(a, i, pos, jt, CombDev{comb_k1});
       } else if (R1 && b == BUCKET_R1) {
-        if constexpr (R1) batch_secp_item<CurveR1, WGB>(a, i, jt, GTabOf<CurveR1>{s_r1});
+        if constexpr (R1) batch_secp_item<CurveR1>(a, i, pos, jt, CombDev{comb_r1});
       } else if constexpr (ED) {
         // the challenge is hashed here, inside the persistent kernel: the tile's items have equal
         // SHA-512 block counts (bucketed), and the hash's memory latency hides behind the other
@@ -295,6 +334,7 @@ static BatchArgs batch_args(const BatchLaunch& L) {
   a.order = L.order;
   a.rank = L.rank;
   a.tile_items = 64u * L.tile_rounds;
+  a.sc = ItemScratch{(uint4*)L.scratch, L.scratch_stride};
   return a;
 }
 
@@ -330,15 +370,14 @@ hipError_t launch_batch(const BatchLaunch& L, hipStream_t s) {
   // (the Ed25519 challenges are hashed inside k_batch_run; the stage stays empty, so that the
   // stage indices of earlier measurements keep their meaning)
   if ((e = mark(2)) != hipSuccess) return e;
+  k_batch_scalars<<<L.stage_grid, 256, 0, s>>>(a);
   if (L.waves == 1)
-    k_batch_run<RUN_MIXED, 1><<<L.grid, 256, 0, s>>>(a, (const uint4*)L.gk1, (const uint4*)L.gr1, (const uint4*)L.gb,
-                                                    (uint4*)L.lane_tab, L.slots);
-  else if (L.g_window == 9)
-    k_batch_run<RUN_MIXED, 2, 9><<<L.grid, 256, 0, s>>>(a, (const uint4*)L.gk1, (const uint4*)L.gr1,
-                                                       (const uint4*)L.gb, (uint4*)L.lane_tab, L.slots);
+    k_batch_run<RUN_MIXED, 1><<<L.grid, 256, 0, s>>>(a, (const uint4*)L.comb_k1, (const uint4*)L.comb_r1,
+                                                    (const uint4*)L.gb, (uint4*)L.lane_tab, L.slots);
   else
-    k_batch_run<RUN_MIXED><<<L.grid, 256, 0, s>>>(a, (const uint4*)L.gk1, (const uint4*)L.gr1, (const uint4*)L.gb,
-                                                 (uint4*)L.lane_tab, L.slots);
+    k_batch_run<RUN_MIXED><<<L.grid, 256, 0, s>>>(a, (const uint4*)L.comb_k1, (const uint4*)L.comb_r1,
+                                                 (const uint4*)L.gb, (uint4*)L.lane_tab, L.slots);
+  k_batch_finish<<<L.stage_grid, 256, 0, s>>>(a);
   if ((e = mark(3)) != hipSuccess) return e;
   k_batch_careful<<<64, 64, 0, s>>>(a, (const uint4*)L.gk1, (const uint4*)L.gr1);
   if ((e = mark(4)) != hipSuccess) return e;

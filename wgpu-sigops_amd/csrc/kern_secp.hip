@@ -10,45 +10,55 @@
 
 namespace sigops {
 
-hipError_t SIGOPS_CAT(launch_secp_recover_, SIGOPS_CURVE)(const void* sigs, const void* digs, void* out, void* status,
-                                                         u32 n, const void* gtab, void* rtab, u32 slots,
-                                                         u32* pend_list, u32* pend_count, u32 grid, u32 g_window,
-                                                         hipStream_t s) {
+static constexpr int CURVE_ID = std::is_same<SIGOPS_CURVE, CurveK1>::value ? 0 : 1;
+
+// lanes of the stages that share an inversion: one per item up to STAGE_LANES
+static u32 stage_blocks(u32 n) { return ((n < STAGE_LANES ? n : STAGE_LANES) + 255) / 256; }
+
+hipError_t SIGOPS_CAT(launch_secp_recover_, SIGOPS_CURVE)(const SecpLaunch& L, const void* sigs, const void* digs,
+                                                         void* out, void* status, u32 n, hipStream_t s) {
   if (n == 0) return hipSuccess;
   const u32 want = (n + 255) / 256;
-  const u32 g = want < grid ? want : grid;
-  k_fill_u32<<<1, 64, 0, s>>>(pend_count, 0u, 1u);
-  if (g_window == 9)
-    k_secp_recover<SIGOPS_CURVE, 9><<<g, 256, 0, s>>>((const uint4*)sigs, (const uint4*)digs, (uint4*)out,
-                                                     (u8*)status, n, (const uint4*)gtab, (uint4*)rtab, slots,
-                                                     pend_list, pend_count);
-  else
-    k_secp_recover<SIGOPS_CURVE, 8><<<g, 256, 0, s>>>((const uint4*)sigs, (const uint4*)digs, (uint4*)out,
-                                                     (u8*)status, n, (const uint4*)gtab, (uint4*)rtab, slots,
-                                                     pend_list, pend_count);
+  const u32 g = want < L.grid ? want : L.grid;
+  const bool quad = !L.gtab8 && n <= QUAD_MAX_ITEMS;
+  if (!quad) k_fill_u32<<<1, 64, 0, s>>>(L.pend_count, 0u, 1u);
+  if (quad) {
+    const hipError_t e = launch_quad_secp(CURVE_ID, false, L, sigs, digs, nullptr, out, status, n, s);
+    if (e != hipSuccess) return e;
+  } else if (L.gtab8) {
+    k_secp_recover<SIGOPS_CURVE><<<g, 256, 0, s>>>((const uint4*)sigs, (const uint4*)digs, (uint4*)out, (u8*)status, n,
+                                                  (const uint4*)L.gtab8, (uint4*)L.lane_tab, L.slots, L.pend_list,
+                                                  L.pend_count);
+  } else {
+    const ItemScratch sc{(uint4*)L.scratch, L.scratch_stride};
+    k_secp_scalars<SIGOPS_CURVE, false><<<stage_blocks(n), 256, 0, s>>>((const uint4*)sigs, (const uint4*)digs, n, sc);
+    k_secp_points<SIGOPS_CURVE><<<g, 256, 0, s>>>((const uint4*)sigs, n, sc, (const uint4*)L.comb, (uint4*)L.lane_tab,
+                                                 L.slots, L.pend_list, L.pend_count);
+    k_secp_finish<SIGOPS_CURVE><<<stage_blocks(n), 256, 0, s>>>((uint4*)out, (u8*)status, n, sc);
+  }
   k_secp_careful<SIGOPS_CURVE><<<64, 64, 0, s>>>((const uint4*)sigs, (const uint4*)digs, (uint4*)out, (u8*)status,
-                                                (const uint4*)gtab, pend_list, pend_count);
+                                                (const uint4*)(L.gtab8 ? L.gtab8 : L.gtab), L.pend_list, L.pend_count);
   return hipGetLastError();
 }
 
-hipError_t SIGOPS_CAT(launch_secp_verify_, SIGOPS_CURVE)(const void* sigs, const void* digs, const void* pubs,
-                                                        void* status, u32 n, const void* gtab, void* rtab, u32 slots,
-                                                        u32* pend_list, u32* pend_count, u32 grid, u32 g_window,
-                                                        hipStream_t s) {
+hipError_t SIGOPS_CAT(launch_secp_verify_, SIGOPS_CURVE)(const SecpLaunch& L, const void* sigs, const void* digs,
+                                                        const void* pubs, void* status, u32 n, hipStream_t s) {
   if (n == 0) return hipSuccess;
   const u32 want = (n + 255) / 256;
-  const u32 g = want < grid ? want : grid;
-  k_fill_u32<<<1, 64, 0, s>>>(pend_count, 0u, 1u);
-  if (g_window == 9)
-    k_secp_verify<SIGOPS_CURVE, 9><<<g, 256, 0, s>>>((const uint4*)sigs, (const uint4*)digs, (const uint4*)pubs,
-                                                    (u8*)status, n, (const uint4*)gtab, (uint4*)rtab, slots,
-                                                    pend_list, pend_count);
-  else
-    k_secp_verify<SIGOPS_CURVE, 8><<<g, 256, 0, s>>>((const uint4*)sigs, (const uint4*)digs, (const uint4*)pubs,
-                                                    (u8*)status, n, (const uint4*)gtab, (uint4*)rtab, slots,
-                                                    pend_list, pend_count);
+  const u32 g = want < L.grid ? want : L.grid;
+  if (n <= QUAD_MAX_ITEMS) {
+    const hipError_t e = launch_quad_secp(CURVE_ID, true, L, sigs, digs, pubs, nullptr, status, n, s);
+    if (e != hipSuccess) return e;
+  } else {
+  const ItemScratch sc{(uint4*)L.scratch, L.scratch_stride};
+  k_fill_u32<<<1, 64, 0, s>>>(L.pend_count, 0u, 1u);
+  k_secp_scalars<SIGOPS_CURVE, true><<<stage_blocks(n), 256, 0, s>>>((const uint4*)sigs, (const uint4*)digs, n, sc);
+  k_secp_verify<SIGOPS_CURVE><<<g, 256, 0, s>>>((const uint4*)sigs, (const uint4*)pubs, (u8*)status, n, sc,
+                                               (const uint4*)L.comb, (uint4*)L.lane_tab, L.slots, L.pend_list,
+                                               L.pend_count);
+  }
   k_secp_verify_careful<SIGOPS_CURVE><<<64, 64, 0, s>>>((const uint4*)sigs, (const uint4*)digs, (const uint4*)pubs,
-                                                       (u8*)status, (const uint4*)gtab, pend_list, pend_count);
+                                                       (u8*)status, (const uint4*)L.gtab, L.pend_list, L.pend_count);
   return hipGetLastError();
 }
 

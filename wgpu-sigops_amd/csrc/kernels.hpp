@@ -8,30 +8,66 @@ namespace sigops {
 typedef uint8_t u8;
 
 constexpr uint32_t GTAB_ENTRIES = 1u << (8 - 1);  // odd multiples 1..255 of G
-constexpr uint32_t GTAB9_ENTRIES = 1u << (9 - 1);  // odd multiples 1..511 of G (9-bit windows; the HBM table's size)
 constexpr uint32_t BTAB_ENTRIES = 1u << (8 - 1);  // odd multiples 1..255 of B (and as many of [2^136] B)
 // the Ed25519 fixed-base tables as held in HBM and LDS: odd multiples of B, then of [2^136] B,
 // 7 uint4 per entry
 constexpr uint32_t BTAB_UINT4 = 2 * BTAB_ENTRIES * 7;
-constexpr uint32_t SECP_LANE_TAB_BYTES = 8 * 9 * 16;  // 8 entries x 9 uint4 (Jacobian + Z product, then affine)
+constexpr uint32_t SECP_LANE_TAB_BYTES = 8 * 7 * 16;  // 8 entries x 7 uint4 (Jacobian, then affine)
 constexpr uint32_t ED_LANE_TAB_BYTES = 16 * 9 * 16;   // 16 cached entries (-A, then -R) x 9 uint4
 
-// g_window: the fixed-base window, 8 or 9 bits (9 needs a table of 256 odd multiples of G: the
-// resident one)
-hipError_t launch_secp_recover_CurveK1(const void* sigs, const void* digs, void* out, void* status, uint32_t n,
-                                      const void* gtab, void* rtab, uint32_t slots, uint32_t* pend_list,
-                                      uint32_t* pend_count, uint32_t grid, uint32_t g_window, hipStream_t s);
-hipError_t launch_secp_recover_CurveR1(const void* sigs, const void* digs, void* out, void* status, uint32_t n,
-                                      const void* gtab, void* rtab, uint32_t slots, uint32_t* pend_list,
-                                      uint32_t* pend_count, uint32_t grid, uint32_t g_window, hipStream_t s);
+constexpr uint32_t ITEM_SCRATCH_BYTES = 7 * 16;       // per position of a secp call (ItemScratch)
 
-// verification with a known public key (64 bytes X || Y per item); status only
-hipError_t launch_secp_verify_CurveK1(const void* sigs, const void* digs, const void* pubs, void* status, uint32_t n,
-                                     const void* gtab, void* rtab, uint32_t slots, uint32_t* pend_list,
-                                     uint32_t* pend_count, uint32_t grid, uint32_t g_window, hipStream_t s);
-hipError_t launch_secp_verify_CurveR1(const void* sigs, const void* digs, const void* pubs, void* status, uint32_t n,
-                                     const void* gtab, void* rtab, uint32_t slots, uint32_t* pend_list,
-                                     uint32_t* pend_count, uint32_t grid, uint32_t g_window, hipStream_t s);
+// what the secp launches use of a context. gtab8: a caller's converted table (128 odd multiples), or
+// null for the resident tables: the wide ones (comb) and, for the careful pass, gtab.
+struct SecpLaunch {
+  const void* gtab;
+  const void* gtab8;
+  const void* comb;
+  void* scratch;
+  uint32_t scratch_stride;  // positions the scratch holds, at least n
+  void* lane_tab;
+  uint32_t slots, grid;
+  uint32_t* pend_list;
+  uint32_t* pend_count;
+};
+hipError_t launch_secp_recover_CurveK1(const SecpLaunch& L, const void* sigs, const void* digs, void* out,
+                                      void* status, uint32_t n, hipStream_t s);
+hipError_t launch_secp_recover_CurveR1(const SecpLaunch& L, const void* sigs, const void* digs, void* out,
+                                      void* status, uint32_t n, hipStream_t s);
+
+// verification with a known public key (64 bytes X || Y per item); status only; resident tables
+hipError_t launch_secp_verify_CurveK1(const SecpLaunch& L, const void* sigs, const void* digs, const void* pubs,
+                                     void* status, uint32_t n, hipStream_t s);
+hipError_t launch_secp_verify_CurveR1(const SecpLaunch& L, const void* sigs, const void* digs, const void* pubs,
+                                     void* status, uint32_t n, hipStream_t s);
+
+// Small calls (kern_quad.hpp) take four lanes per item: up to this many items the point waves are at
+// most one per SIMD, and the call is as long as one item. Measured (us per device call, four lanes
+// against one lane per item): secp256k1 recovery 473 / 807 at 1,000 items, 551 / 812 at 16,384, 1,015
+// / 812 at 20,011; secp256r1 verification 563 / 1,140, 656 / 1,148, 1,255 / 1,148; Ed25519 with
+// messages up to 200 bytes 320 / 990, 543 / 1,000 (one lane per item with its bucketing).
+constexpr uint32_t QUAD_MAX_ITEMS = 16384;
+// pend_count is cleared; the careful pass is the caller's (launch_secp_*_careful)
+hipError_t launch_quad_secp(int curve, bool verify, const SecpLaunch& L, const void* sigs, const void* digs,
+                            const void* pubs, void* out, void* status, uint32_t n, hipStream_t s);
+struct EdQuadLaunch {
+  const void* sigs;
+  const void* keys;
+  const void* msgs;
+  const uint64_t* msg_off;
+  void* status;
+  const void* comb;
+  const void* gb;     // resident table, for the full-length check
+  void* lane_tab;
+  uint32_t slots;     // at least QUAD_MAX_ITEMS / 16 * 128
+};
+hipError_t launch_quad_ed(bool strict, const EdQuadLaunch& L, uint32_t n, hipStream_t s);
+
+// the wide fixed-base table of a curve (0 secp256k1, 1 secp256r1, 2 Ed25519) from its resident table; tmp:
+// comb_tmp_bytes() that may be freed once the stream has passed the launch
+size_t comb_bytes(int curve);
+size_t comb_tmp_bytes();
+hipError_t launch_comb_build(int curve, const void* gtab, void* comb, void* tmp, hipStream_t s);
 
 // ---- mixed batch ----
 constexpr uint32_t BUCKET_K1 = 0, BUCKET_R1 = 1, BUCKET_ED0 = 2;
@@ -64,10 +100,14 @@ struct BatchLaunch {
   const void* gk1;
   const void* gr1;
   const void* gb;
+  const void* comb_k1;
+  const void* comb_r1;
+  void* scratch;            // ItemScratch of the secp items, by position in `order`
+  uint32_t scratch_stride;  // its positions: the capacity of `order`
   void* lane_tab;
   uint32_t slots, grid, aux_grid, tile_rounds;
+  uint32_t stage_grid;   // blocks of the stages that share an inversion between items
   uint32_t waves;        // mixed batch: waves per SIMD the persistent kernel is built for (1 or 2)
-  uint32_t g_window;     // mixed batch: fixed-base window of the secp streams, 8 or 9 bits (9: waves 2 only)
   hipEvent_t* stage_ev;  // null, or 5 events recorded before, between and after the 4 stages
 };
 
@@ -112,14 +152,15 @@ struct StreamLaunch {
   uint32_t* ctr;         // device: STREAM_CTR_BYTES of counters and polling state (cleared by the launch)
   uint32_t* pend_list;   // device: position lanes (position * 64 + lane) the careful pass redoes
   uint32_t pend_cap;     // entries pend_list holds (further pending lanes are not recorded)
-  const void* gk1;
+  const void* gk1;       // resident tables, for the careful pass
   const void* gr1;
   const void* gb;
+  const void* comb_k1;   // wide tables
+  const void* comb_r1;
   void* lane_tab;
   uint32_t slots;        // tiles a wavefront may take at most
   uint32_t base, mask;   // see qpos (a batch: 0 and ~0)
   uint32_t seq, lane_slots, grid;
-  uint32_t g_window;     // fixed-base window of the secp items, 8 or 9 bits
   uint64_t poll_ticks;   // wall-clock ticks between reads of the pinned count (device-wide)
   uint64_t limit_ticks;  // a wave that waits this long for a tile gives up
 };
@@ -139,9 +180,10 @@ struct RingResources {
   const void* gk1;
   const void* gr1;
   const void* gb;
+  const void* comb_k1;
+  const void* comb_r1;
   void* lane_tab;
   uint32_t lane_slots, grid;
-  uint32_t g_window;             // fixed-base window of the secp items, 8 or 9 bits
   const uint32_t* bucket_order;  // processing rank -> bucket, NBUCKETS entries
   hipStream_t stream;
 };

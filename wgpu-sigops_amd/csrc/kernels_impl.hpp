@@ -136,52 +136,53 @@ struct LaneTab {
   }
 };
 
-// secp R-table (secp_build_table): while building, entry e holds a Jacobian point and the running
-// product of the Z coordinates before it (36 words, 9 chunks); afterwards its first 5 chunks hold
-// the affine (x, y) the ladder reads, and for secp256k1 chunks 4..6 also hold beta * x, so that
-// the phi(R) stream reads (beta x, y) from chunks 2..6 (five loads, as for (x, y))
-struct STabDev : LaneTab<9> {
-  DEV void store_full(int e, const jac& p, const fe& before) {
-    u32 w[36];
+// secp R-table (secp_build_table): while building, entry e holds a Jacobian point (X, W) and the
+// factor between its Z and the one before (27 words, 7 chunks); afterwards its first 5 chunks hold
+// the affine (x, w) the ladder reads, and for secp256k1 chunks 4..6 also hold beta * x, so that
+// the phi(R) stream reads (beta x, w) from chunks 2..6 (five loads, as for (x, w))
+struct STabDev : LaneTab<7> {
+  DEV void store_full(int e, const jac& p, const fe&) {
+    u32 w[28];
 #pragma unroll
     for (int k = 0; k < NL; k++) {
-      w[k] = p.X.v[k]; w[9 + k] = p.Y.v[k]; w[18 + k] = p.Z.v[k]; w[27 + k] = before.v[k];
+      w[k] = p.X.v[k]; w[9 + k] = p.Y.v[k]; w[18 + k] = p.Z.v[k];
     }
+    w[27] = 0;
     put(e, w);
   }
-  DEV void load_full(u32 e, jac& p, fe& before) const {
-    u32 w[36];
+  DEV void load_full(u32 e, jac& p, fe&) const {
+    u32 w[28];
     get(e, w);
 #pragma unroll
     for (int k = 0; k < NL; k++) {
-      p.X.v[k] = w[k]; p.Y.v[k] = w[9 + k]; p.Z.v[k] = w[18 + k]; before.v[k] = w[27 + k];
+      p.X.v[k] = w[k]; p.Y.v[k] = w[9 + k]; p.Z.v[k] = w[18 + k];
     }
   }
-  DEV void store_affine(int e, const fe& x, const fe& y) {
+  DEV void store_affine(int e, const fe& x, const fe& w2) {
     u32 w[20];
 #pragma unroll
-    for (int k = 0; k < NL; k++) { w[k] = x.v[k]; w[9 + k] = y.v[k]; }
+    for (int k = 0; k < NL; k++) { w[k] = x.v[k]; w[9 + k] = w2.v[k]; }
     w[18] = w[19] = 0;
     put_n<5>(e, w);
   }
-  DEV void load_affine(u32 e, fe& x, fe& y) const {
+  DEV void load_affine(u32 e, fe& x, fe& w2) const {
     u32 w[20];
     get_n<5>(e, w);
 #pragma unroll
-    for (int k = 0; k < NL; k++) { x.v[k] = w[k]; y.v[k] = w[9 + k]; }
+    for (int k = 0; k < NL; k++) { x.v[k] = w[k]; w2.v[k] = w[9 + k]; }
   }
-  DEV void store_affine_phi(int e, const fe& x, const fe& y, const fe& bx) {
+  DEV void store_affine_phi(int e, const fe& x, const fe& w2, const fe& bx) {
     u32 w[28];
 #pragma unroll
-    for (int k = 0; k < NL; k++) { w[k] = x.v[k]; w[9 + k] = y.v[k]; w[18 + k] = bx.v[k]; }
+    for (int k = 0; k < NL; k++) { w[k] = x.v[k]; w[9 + k] = w2.v[k]; w[18 + k] = bx.v[k]; }
     w[27] = 0;
-    put_n<7>(e, w);
+    put(e, w);
   }
-  DEV void load_affine_phi(u32 e, fe& bx, fe& y) const {
+  DEV void load_affine_phi(u32 e, fe& bx, fe& w2) const {
     u32 w[28];
     get_range<2, 5>(e, w);
 #pragma unroll
-    for (int k = 0; k < NL; k++) { y.v[k] = w[9 + k]; bx.v[k] = w[18 + k]; }
+    for (int k = 0; k < NL; k++) { w2.v[k] = w[9 + k]; bx.v[k] = w[18 + k]; }
   }
 };
 
@@ -203,6 +204,40 @@ struct CTabDev : LaneTab<9> {  // cached Edwards point: 36 words
       p.ypx.v[k] = w[k]; p.ymx.v[k] = w[9 + k]; p.z.v[k] = w[18 + k]; p.t2d.v[k] = w[27 + k];
     }
     return p;
+  }
+};
+
+// the wide fixed-base table of one curve in HBM: entry j of window i at 4 (i COMB_ENTRIES + j)
+struct CombDev {
+  const uint4* t;
+  DEV void load(int i, u32 j, comb_entry& e) const {
+    const uint4* p = t + 4 * ((u64)i * COMB_ENTRIES + j);
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      const uint4 q = p[c];
+      e.v[4 * c] = q.x; e.v[4 * c + 1] = q.y; e.v[4 * c + 2] = q.z; e.v[4 * c + 3] = q.w;
+    }
+  }
+};
+
+// Per-item scratch between the stages of a secp call, chunk c of position p at base[c * stride + p]:
+// first u1 and u2 (4 chunks), then the Jacobian result and its status (7 chunks)
+struct ItemScratch {
+  uint4* base;
+  u32 stride;
+  template <int N>
+  DEV void put(u32 p, const u32* w) const {
+#pragma unroll
+    for (int c = 0; c < N; c++)
+      base[(u64)c * stride + p] = make_uint4(w[4 * c], w[4 * c + 1], w[4 * c + 2], w[4 * c + 3]);
+  }
+  template <int N, int A = 0>
+  DEV void get(u32 p, u32* w) const {
+#pragma unroll
+    for (int c = A; c < A + N; c++) {
+      const uint4 q = base[(u64)c * stride + p];
+      w[4 * c] = q.x; w[4 * c + 1] = q.y; w[4 * c + 2] = q.z; w[4 * c + 3] = q.w;
+    }
   }
 };
 
@@ -231,19 +266,267 @@ DEV void load_words(const uint4* p, u32* w, int nq) {
   }
 }
 
+// ---- stages of a secp call on the wide tables ----
+// A recovery inverts r modulo n and the result's Z modulo p, 20,000 VALU instructions each, of about
+// 400,000 for the item. Both are shared: a lane of the stages before and after the ladder takes
+// every lanes-th item, inverts the product of their values once and multiplies back (Montgomery's
+// trick: 3 products of 170-220 instructions per item). The stages pass 64 and 112 bytes per item
+// through HBM (ItemScratch).
+constexpr u32 STAGE_LANES = 65536;  // lanes of those stages: one wavefront per SIMD
+
+// u1, u2 of the positions first, first + step, ... below end. Src: sig(p, words) and digest(p,
+// words), sig false where the position holds no item. VERIFY: u1 = z/s, u2 = r/s; else -z/r, s/r.
+template <class C, bool VERIFY, class Src>
+DEV void secp_scalars_lane(u32 first, u32 step, u32 end, const Src& src, const ItemScratch& sc) {
+  typedef typename C::Fn Fn;
+  if (first >= end) return;
+  const fe one = fe_from_const(Fn::ONE);
+  auto denominator = [&](u32 p, secp_sig& g) {
+    u32 sr[16];
+    if (!src.sig(p, sr) || secp_decode_sig<C>(sr, g) != ST_OK) return one;
+    return to_mont<Fn>(fe_from_words(VERIFY ? g.s : g.r));
+  };
+  fe run = one;
+  u32 p = first;
+#pragma unroll 1
+  for (;;) {
+    u32 w[12];
+#pragma unroll
+    for (int k = 0; k < NL; k++) w[k] = run.v[k];
+    w[9] = w[10] = w[11] = 0;
+    sc.put<3>(p, w);
+    secp_sig g;
+    run = mont_mul<Fn>(run, denominator(p, g));
+    if (end - p <= step) break;
+    p += step;
+  }
+  fe inv = finv<Fn>(run);
+#pragma unroll 1
+  for (;;) {
+    u32 w[16], dr[8];
+    sc.get<3>(p, w);
+    fe before;
+#pragma unroll
+    for (int k = 0; k < NL; k++) before.v[k] = w[k];
+    secp_sig g;
+    const fe d = denominator(p, g);
+    const fe di = mont_mul<Fn>(inv, before);
+    inv = mont_mul<Fn>(inv, d);
+    if (src.digest(p, dr)) {
+      secp_decode_digest<C>(dr, g);
+      const fe zd = mont_mul<Fn>(to_mont<Fn>(fe_from_words(g.z)), di);
+      const fe u1m = VERIFY ? zd : fneg<Fn>(zd);
+      const fe u2m = mont_mul<Fn>(to_mont<Fn>(fe_from_words(VERIFY ? g.r : g.s)), di);
+      fe_to_words(from_mont<Fn>(u1m), w);
+      fe_to_words(from_mont<Fn>(u2m), w + 8);
+      sc.put<4>(p, w);
+    }
+    if (p == first) break;
+    p -= step;
+  }
+}
+
+// Q = u1 G + u2 P of position p (u1, u2 from secp_scalars_lane)
+template <class C>
+DEV jac secp_point(u32 p, const fe& x, const fe& y, const ItemScratch& sc, STabDev& tab, const CombDev& comb,
+                   bool& exc) {
+  u32 w[16];
+  sc.get<4>(p, w);
+  secp_pro pro;
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    pro.u1[k] = w[k];
+    pro.u2[k] = w[8 + k];
+  }
+  secp_carriers<C, true>(pro, x, y);
+  const jacs Q = secp_ladder_s<C, 0>(pro, tab, comb, exc);
+  return s_to_jac<C>(secp_comb<C>(Q, pro, comb, exc));
+}
+
+// the recovery at position p up to its Jacobian result, left in the scratch with the status
+template <class C>
+DEV u32 secp_recover_point(const u32 sr[16], u32 p, const ItemScratch& sc, STabDev& tab, const CombDev& comb) {
+  secp_sig g;
+  u32 st = secp_decode_sig<C>(sr, g);
+  u32 w[28];
+  if (st == ST_OK) {
+    fe x, y;
+    if (!secp_lift<C>(g.r, g.y_odd, x, y)) st = ST_NO_POINT;
+    if (st == ST_OK) {
+      bool exc = false;
+      const jac Q = secp_point<C>(p, x, y, sc, tab, comb, exc);
+      if (exc) st = ST_PENDING;
+#pragma unroll
+      for (int k = 0; k < NL; k++) {
+        w[k] = Q.X.v[k]; w[9 + k] = Q.Y.v[k]; w[18 + k] = Q.Z.v[k];
+      }
+    }
+  }
+  w[27] = st;
+  sc.put<7>(p, w);
+  return st;
+}
+
+// affine keys of the positions first, first + step, ... below end, from the scratch. Dst: out(p),
+// the item's 64 output bytes (null where the position holds no item; they carry the running products
+// in between), and status(p, st).
+template <class C, class Dst>
+DEV void secp_finish_lane(u32 first, u32 step, u32 end, const Dst& dst, const ItemScratch& sc) {
+  typedef typename C::Fp F;
+  if (first >= end) return;
+  auto z_of = [&](const u32* w) {
+    fe z = fe_from_const(F::ONE);
+    if (w[27] == ST_OK) {
+#pragma unroll
+      for (int k = 0; k < NL; k++) z.v[k] = w[18 + k];
+    }
+    return z;
+  };
+  fe run = fe_from_const(F::ONE);
+  u32 p = first;
+#pragma unroll 1
+  for (;;) {
+    uint4* o = dst.out(p);
+    if (o) {
+      u32 w[28];
+      sc.get<3, 4>(p, w);
+      o[0] = make_uint4(run.v[0], run.v[1], run.v[2], run.v[3]);
+      o[1] = make_uint4(run.v[4], run.v[5], run.v[6], run.v[7]);
+      o[2] = make_uint4(run.v[8], 0, 0, 0);
+      run = mont_mul<F>(run, z_of(w));
+    }
+    if (end - p <= step) break;
+    p += step;
+  }
+  fe inv = finv<F>(run);
+#pragma unroll 1
+  for (;;) {
+    uint4* o = dst.out(p);
+    if (o) {
+      u32 w[28], res[16];
+      sc.get<7>(p, w);
+      fe before;
+      const uint4 b0 = o[0], b1 = o[1], b2 = o[2];
+      before.v[0] = b0.x; before.v[1] = b0.y; before.v[2] = b0.z; before.v[3] = b0.w;
+      before.v[4] = b1.x; before.v[5] = b1.y; before.v[6] = b1.z; before.v[7] = b1.w;
+      before.v[8] = b2.x;
+      const fe zi = mont_mul<F>(inv, before);
+      inv = mont_mul<F>(inv, z_of(w));
+      fe X, Y;
+#pragma unroll
+      for (int k = 0; k < NL; k++) { X.v[k] = w[k]; Y.v[k] = w[9 + k]; }
+      secp_store_affine<C>(X, Y, zi, res);
+      const u32 keep = lane_mask(w[27] == ST_OK);
+#pragma unroll
+      for (int c = 0; c < 4; c++)
+        o[c] = make_uint4(res[4 * c] & keep, res[4 * c + 1] & keep, res[4 * c + 2] & keep, res[4 * c + 3] & keep);
+      dst.status(p, w[27]);
+    }
+    if (p == first) break;
+    p -= step;
+  }
+}
+
 // ---- kernels ----
-// WGB: the fixed-base window, 8 bits (128 odd multiples of G staged in LDS) or 9 (256; the resident
-// table only, a caller's converted table holds 128)
-template <class C, int WGB = 8>
+struct PlainItems {  // position p = item p
+  const uint4* sigs;
+  const uint4* digs;
+  uint4* outs;
+  u8* st;
+  DEV bool sig(u32 p, u32* w) const {
+    load_words(sigs + 4 * (u64)p, w, 4);
+    return true;
+  }
+  DEV bool digest(u32 p, u32* w) const {
+    load_words(digs + 2 * (u64)p, w, 2);
+    return true;
+  }
+  DEV uint4* out(u32 p) const { return outs + 4 * (u64)p; }
+  DEV void status(u32 p, u32 s) const { st[p] = (u8)s; }
+};
+
+template <class C, bool VERIFY>
+__global__ __launch_bounds__(256, SIGOPS_WAVES_PER_EU) void k_secp_scalars(const uint4* __restrict__ sigs,
+                                                                      const uint4* __restrict__ digs, u32 n,
+                                                                      ItemScratch sc) {
+  secp_scalars_lane<C, VERIFY>(blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x, n,
+                               PlainItems{sigs, digs, nullptr, nullptr}, sc);
+}
+
+template <class C>
+__global__ __launch_bounds__(256, SIGOPS_WAVES_PER_EU) void k_secp_finish(uint4* __restrict__ out,
+                                                                     u8* __restrict__ status, u32 n, ItemScratch sc) {
+  secp_finish_lane<C>(blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x, n,
+                      PlainItems{nullptr, nullptr, out, status}, sc);
+}
+
+template <class C>
+__global__ __launch_bounds__(256, SIGOPS_WAVES_PER_EU) void k_secp_points(const uint4* __restrict__ sigs, u32 n,
+                                                                     ItemScratch sc, const uint4* __restrict__ comb,
+                                                                     uint4* __restrict__ rtab, u32 slots,
+                                                                     u32* __restrict__ pend_list,
+                                                                     u32* __restrict__ pend_count) {
+  const u32 slot = blockIdx.x * blockDim.x + threadIdx.x;
+  STabDev tab;
+  tab.base = rtab;
+  tab.slots = slots;
+  tab.slot = slot;
+  const u32 stride = gridDim.x * blockDim.x;
+  for (u32 i = slot; i < n; i += stride) {
+    u32 sr[16];
+    load_words(sigs + 4 * (u64)i, sr, 4);
+    if (secp_recover_point<C>(sr, i, sc, tab, CombDev{comb}) == ST_PENDING) pend_list[atomicAdd(pend_count, 1u)] = i;
+  }
+}
+
+// ECDSA verification with a known key (fuel Signature::verify) after k_secp_scalars: the ladder with
+// the key in place of R and the projective x comparison in place of the affine output. Lanes that
+// meet an exceptional addition are finished by k_secp_verify_careful.
+template <class C>
+__global__ __launch_bounds__(256, SIGOPS_WAVES_PER_EU) void k_secp_verify(
+    const uint4* __restrict__ sigs, const uint4* __restrict__ pubs, u8* __restrict__ status, u32 n, ItemScratch sc,
+    const uint4* __restrict__ comb, uint4* __restrict__ rtab, u32 slots, u32* __restrict__ pend_list,
+    u32* __restrict__ pend_count) {
+  const u32 slot = blockIdx.x * blockDim.x + threadIdx.x;
+  STabDev tab;
+  tab.base = rtab;
+  tab.slots = slots;
+  tab.slot = slot;
+  const u32 stride = gridDim.x * blockDim.x;
+  for (u32 i = slot; i < n; i += stride) {
+    u32 sr[16], pr[16];
+    load_words(sigs + 4 * (u64)i, sr, 4);
+    load_words(pubs + 4 * (u64)i, pr, 4);
+    secp_sig g;
+    fe x, y;
+    u32 st = secp_decode_verify<C>(sr, pr, g, x, y);
+    if (st == ST_OK) {
+      bool exc = false;
+      const jac P = secp_point<C>(i, x, y, sc, tab, CombDev{comb}, exc);
+      if (exc) {
+        st = ST_PENDING;
+        pend_list[atomicAdd(pend_count, 1u)] = i;
+      } else {
+        load_words(sigs + 4 * (u64)i, sr, 4);
+        st = secp_verify_x<C>(P, sr);
+      }
+    }
+    status[i] = (u8)st;
+  }
+}
+
+// recovery with a caller's generator table (128 odd multiples, staged in LDS): one kernel, 8-bit
+// windows on the ladder's doubling chain. Converting a caller's point to the wide tables would take
+// longer than the call.
+template <class C>
 __global__ __launch_bounds__(256, SIGOPS_WAVES_PER_EU) void k_secp_recover(const uint4* __restrict__ sigs,
                                                       const uint4* __restrict__ digs, uint4* __restrict__ out,
                                                       u8* __restrict__ status, u32 n,
                                                       const uint4* __restrict__ gtab, uint4* __restrict__ rtab,
                                                       u32 slots, u32* __restrict__ pend_list,
                                                       u32* __restrict__ pend_count) {
-  constexpr u32 GN = WGB == 9 ? GTAB9_ENTRIES : GTAB_ENTRIES;
-  __shared__ uint4 sg[GN * gtab_chunks<C>()];
-  stage_gtab<C, GN>(sg, gtab);
+  __shared__ uint4 sg[GTAB_ENTRIES * gtab_chunks<C>()];
+  stage_gtab<C, GTAB_ENTRIES>(sg, gtab);
   __syncthreads();
   const GTabOf<C> gt{sg};
   const u32 slot = blockIdx.x * blockDim.x + threadIdx.x;
@@ -261,7 +544,7 @@ __global__ __launch_bounds__(256, SIGOPS_WAVES_PER_EU) void k_secp_recover(const
     u32 st = pro.status;
     if (st == ST_OK) {
       bool exc = false;
-      const jac Q = secp_ladder<C, WGB>(pro, tab, gt, exc);
+      const jac Q = secp_ladder<C, 8>(pro, tab, gt, exc);
       if (exc) {
         st = ST_PENDING;
         pend_list[atomicAdd(pend_count, 1u)] = i;
@@ -309,48 +592,6 @@ __global__ __launch_bounds__(64) void k_secp_careful(const uint4* __restrict__ s
   }
 }
 
-// ECDSA verification with a known key (fuel Signature::verify): the recovery kernel with the key
-// in place of R and the projective x comparison in place of the affine output. Lanes that meet an
-// exceptional addition are finished by k_secp_verify_careful. WGB as in k_secp_recover.
-template <class C, int WGB = 8>
-__global__ __launch_bounds__(256, SIGOPS_WAVES_PER_EU) void k_secp_verify(
-    const uint4* __restrict__ sigs, const uint4* __restrict__ digs, const uint4* __restrict__ pubs,
-    u8* __restrict__ status, u32 n, const uint4* __restrict__ gtab, uint4* __restrict__ rtab, u32 slots,
-    u32* __restrict__ pend_list, u32* __restrict__ pend_count) {
-  constexpr u32 GN = WGB == 9 ? GTAB9_ENTRIES : GTAB_ENTRIES;
-  __shared__ uint4 sg[GN * gtab_chunks<C>()];
-  stage_gtab<C, GN>(sg, gtab);
-  __syncthreads();
-  const GTabOf<C> gt{sg};
-  const u32 slot = blockIdx.x * blockDim.x + threadIdx.x;
-  STabDev tab;
-  tab.base = rtab;
-  tab.slots = slots;
-  tab.slot = slot;
-  const u32 stride = gridDim.x * blockDim.x;
-  for (u32 i = slot; i < n; i += stride) {
-    u32 sr[16], dr[8], pr[16];
-    load_words(sigs + 4 * (u64)i, sr, 4);
-    load_words(digs + 2 * (u64)i, dr, 2);
-    load_words(pubs + 4 * (u64)i, pr, 4);
-    secp_pro pro;
-    secp_prologue_verify<C>(sr, dr, pr, pro);
-    u32 st = pro.status;
-    if (st == ST_OK) {
-      bool exc = false;
-      const jac P = secp_ladder<C, WGB>(pro, tab, gt, exc);
-      if (exc) {
-        st = ST_PENDING;
-        pend_list[atomicAdd(pend_count, 1u)] = i;
-      } else {
-        load_words(sigs + 4 * (u64)i, sr, 4);
-        st = secp_verify_x<C>(P, sr);
-      }
-    }
-    status[i] = (u8)st;
-  }
-}
-
 template <class C>
 __global__ __launch_bounds__(64) void k_secp_verify_careful(const uint4* __restrict__ sigs,
                                                             const uint4* __restrict__ digs,
@@ -377,17 +618,18 @@ static __global__ void k_fill_u32(u32* p, u32 v, u32 n) {
   for (u32 i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = v;
 }
 
-// one recovery on the fast ladder: the status (ST_PENDING when the ladder met an exceptional
-// addition and the careful pass must redo the item) and the key X || Y (zeros unless ST_OK)
-// (WGB: the fixed-base window, 8 or 9 bits, which the table gt must match)
-template <class C, int WGB = 8, class GT>
-DEV u32 secp_item(const u32 sr[16], const u32 dr[8], STabDev& tab, const GT& gt, u32 o[16]) {
+// one recovery by itself (the streamed kernel's tiles): the status (ST_PENDING when the ladder met an
+// exceptional addition and the careful pass must redo the item) and the key X || Y (zeros unless
+// ST_OK)
+template <class C>
+DEV u32 secp_item(const u32 sr[16], const u32 dr[8], STabDev& tab, const CombDev& comb, u32 o[16]) {
   secp_pro pro;
-  secp_prologue<C>(sr, dr, pro);
+  secp_prologue<C, true>(sr, dr, pro);
   u32 st = pro.status;
   if (st == ST_OK) {
     bool exc = false;
-    const jac Q = secp_ladder<C, WGB>(pro, tab, gt, exc);
+    const jacs R = secp_ladder_s<C, 0>(pro, tab, comb, exc);
+    const jac Q = s_to_jac<C>(secp_comb<C>(R, pro, comb, exc));
     if (exc)
       st = ST_PENDING;
     else

@@ -377,87 +377,125 @@ struct secp_pro {
   u32 u1[8], u2[8];  // plain u1, u2 (for the careful path)
 };
 
-// Q = u1 G + u2 P ladder set-up shared by recovery (P = R) and verification (P = the key):
-// plain u1, u2 for the careful path, and the digit carriers of the fast ladder (GLV halves for
-// secp256k1, odd representatives otherwise). u1m, u2m in Montgomery form of n; P affine (x, y).
+// odd representative of a scalar k and its digit carrier: k, or n - k when k is even (neg: the digits
+// then spell -k), C = (k' >> 1) | 2^255
 template <class C>
-DEV void secp_scalars(secp_pro& o, const fe& u1m, const fe& u2m, const fe& x, const fe& y) {
+DEV bool odd_carrier(const u32 k[8], u32 c[8]) {
+  const bool neg = (k[0] & 1u) == 0;
+  u32 t[8];
+  words_sub(C::n32(), k, t);
+#pragma unroll
+  for (int i = 0; i < 8; i++) t[i] = neg ? t[i] : k[i];
+#pragma unroll
+  for (int i = 0; i < 8; i++) c[i] = (t[i] >> 1) | (i < 7 ? t[i + 1] << 31 : 0x80000000u);
+  return neg;
+}
+
+// Q = u1 G + u2 P ladder set-up shared by recovery (P = R) and verification (P = the key), from the
+// plain o.u1, o.u2: the digit carriers of the ladder (GLV halves for secp256k1, odd representatives
+// otherwise). WIDE: u1 for the wide fixed-base tables (secp_comb) instead of the ladder's G streams.
+// P affine (x, y).
+template <class C, bool WIDE = false>
+DEV void secp_carriers(secp_pro& o, const fe& x, const fe& y) {
   typedef typename C::Fp Fp;
-  typedef typename C::Fn Fn;
-  const u32(&n)[8] = C::n32();
-  fe_to_words(from_mont<Fn>(u1m), o.u1);
-  fe_to_words(from_mont<Fn>(u2m), o.u2);
   o.rx = x;
+  o.ry = y;
+  o.ry_neg = false;
+  o.g_neg = false;
+  if constexpr (WIDE || !C::GLV) o.g_neg = odd_carrier<C>(o.u1, o.c1);
   if constexpr (C::GLV) {
     u32 h1[5], h2[5];
-    glv_split(o.u1, h1, h2, o.sg1, o.sg2);
-    glv_carrier<GLV_BG>(h1, o.cg1);
-    glv_carrier<GLV_BG>(h2, o.cg2);
+    if constexpr (!WIDE) {
+      glv_split(o.u1, h1, h2, o.sg1, o.sg2);
+      glv_carrier<GLV_BG>(h1, o.cg1);
+      glv_carrier<GLV_BG>(h2, o.cg2);
+    }
     glv_split(o.u2, h1, h2, o.sr1, o.sr2);
     glv_carrier<GLV_BR>(h1, o.cr1);
     glv_carrier<GLV_BR>(h2, o.cr2);
-    o.ry = y;
-    o.ry_neg = false;
-    o.g_neg = false;
-    return;
+  } else {
+    o.ry_neg = odd_carrier<C>(o.u2, o.c2);
+    if (o.ry_neg) o.ry = fneg<Fp>(y);
   }
-  // odd representatives
-  o.g_neg = (o.u1[0] & 1u) == 0;
-  const bool r_neg = (o.u2[0] & 1u) == 0;
-  u32 k1[8], k2[8];
-  words_sub(n, o.u1, k1);
-  words_sub(n, o.u2, k2);
-#pragma unroll
-  for (int i = 0; i < 8; i++) {
-    k1[i] = o.g_neg ? k1[i] : o.u1[i];
-    k2[i] = r_neg ? k2[i] : o.u2[i];
-  }
-#pragma unroll
-  for (int i = 0; i < 8; i++) {
-    o.c1[i] = (k1[i] >> 1) | (i < 7 ? k1[i + 1] << 31 : 0x80000000u);
-    o.c2[i] = (k2[i] >> 1) | (i < 7 ? k2[i + 1] << 31 : 0x80000000u);
-  }
-  o.ry = r_neg ? fneg<Fp>(y) : y;
-  o.ry_neg = r_neg;
 }
 
-template <class C>
-DEV void secp_prologue(const u32 sig_raw[16], const u32 dig_raw[8], secp_pro& o) {
-  typedef typename C::Fp Fp;
+// the same from u1m, u2m in Montgomery form of n
+template <class C, bool WIDE = false>
+DEV void secp_scalars(secp_pro& o, const fe& u1m, const fe& u2m, const fe& x, const fe& y) {
   typedef typename C::Fn Fn;
+  fe_to_words(from_mont<Fn>(u1m), o.u1);
+  fe_to_words(from_mont<Fn>(u2m), o.u2);
+  secp_carriers<C, WIDE>(o, x, y);
+}
+
+// a signature's r, s, its recovery parity, and z = digest mod n; ST_OK, ST_BAD_R or ST_BAD_S
+struct secp_sig {
+  u32 r[8], s[8], z[8];
+  bool y_odd;
+};
+template <class C>
+DEV u32 secp_decode_sig(const u32 sig_raw[16], secp_sig& o) {
   const u32(&n)[8] = C::n32();
-  u32 r[8], s[8], z[8], sraw[8];
+  u32 sraw[8];
 #pragma unroll
   for (int i = 0; i < 8; i++) sraw[i] = sig_raw[8 + i];
-  const bool y_odd = (sraw[0] & 0x80u) != 0;  // first byte of s
+  o.y_odd = (sraw[0] & 0x80u) != 0;  // first byte of s
   sraw[0] &= ~0x80u;
-  words_from_be_bytes(sig_raw, r);
-  words_from_be_bytes(sraw, s);
-  words_from_be_bytes(dig_raw, z);
-  o.status = ST_OK;
-  if (words_is_zero(r) || !words_lt(r, n)) o.status = ST_BAD_R;
-  else if (words_is_zero(s) || !words_lt(s, n)) o.status = ST_BAD_S;
-  if (!words_lt(z, n)) {
+  words_from_be_bytes(sig_raw, o.r);
+  words_from_be_bytes(sraw, o.s);
+  if (words_is_zero(o.r) || !words_lt(o.r, n)) return ST_BAD_R;
+  if (words_is_zero(o.s) || !words_lt(o.s, n)) return ST_BAD_S;
+  return ST_OK;
+}
+template <class C>
+DEV void secp_decode_digest(const u32 dig_raw[8], secp_sig& o) {
+  const u32(&n)[8] = C::n32();
+  words_from_be_bytes(dig_raw, o.z);
+  if (!words_lt(o.z, n)) {
     u32 t[8];
-    words_sub(z, n, t);
+    words_sub(o.z, n, t);
 #pragma unroll
-    for (int i = 0; i < 8; i++) z[i] = t[i];
+    for (int i = 0; i < 8; i++) o.z[i] = t[i];
   }
-  // lift x = r
-  const fe x = to_mont<Fp>(fe_from_words(r));
+}
+
+// x^3 + a x + b
+template <class C>
+DEV fe secp_rhs(const fe& x) {
+  typedef typename C::Fp Fp;
   fe rhs = mont_mul<Fp>(mont_sqr<Fp>(x), x);
   if (C::A_IS_M3) rhs = fsub<Fp>(rhs, fadd<Fp>(fdbl<Fp>(x), x));
-  rhs = fadd<Fp>(rhs, C::b());
-  fe y = fpow_chain<Fp, typename C::SqrtChain>(rhs);
-  if (o.status == ST_OK && !feq<Fp>(mont_sqr<Fp>(y), rhs)) o.status = ST_NO_POINT;
+  return fadd<Fp>(rhs, C::b());
+}
+
+// the curve point with x-coordinate r and the given parity of y; false if there is none
+template <class C>
+DEV bool secp_lift(const u32 r[8], bool y_odd, fe& x, fe& y) {
+  typedef typename C::Fp Fp;
+  x = to_mont<Fp>(fe_from_words(r));
+  const fe rhs = secp_rhs<C>(x);
+  y = s_to_fe<Fp, 1>(s_pow_chain<Fp, typename C::SqrtChain>(s_from(rhs)));
+  const bool ok = feq<Fp>(mont_sqr<Fp>(y), rhs);
   const fe yc = from_mont<Fp>(y);
   if ((bool)(yc.v[0] & 1u) != y_odd) y = fneg<Fp>(y);
+  return ok;
+}
+
+template <class C, bool WIDE = false>
+DEV void secp_prologue(const u32 sig_raw[16], const u32 dig_raw[8], secp_pro& o) {
+  typedef typename C::Fn Fn;
+  secp_sig g;
+  o.status = secp_decode_sig<C>(sig_raw, g);
+  secp_decode_digest<C>(dig_raw, g);
+  fe x, y;
+  const bool ok = secp_lift<C>(g.r, g.y_odd, x, y);
+  if (o.status == ST_OK && !ok) o.status = ST_NO_POINT;
   // u1 = -z/r, u2 = s/r (mod n)
-  const fe rn = to_mont<Fn>(fe_from_words(r));
+  const fe rn = to_mont<Fn>(fe_from_words(g.r));
   const fe rinv = finv<Fn>(rn);
-  const fe u1m = fneg<Fn>(mont_mul<Fn>(to_mont<Fn>(fe_from_words(z)), rinv));
-  const fe u2m = mont_mul<Fn>(to_mont<Fn>(fe_from_words(s)), rinv);
-  secp_scalars<C>(o, u1m, u2m, x, y);
+  const fe u1m = fneg<Fn>(mont_mul<Fn>(to_mont<Fn>(fe_from_words(g.z)), rinv));
+  const fe u2m = mont_mul<Fn>(to_mont<Fn>(fe_from_words(g.s)), rinv);
+  secp_scalars<C, WIDE>(o, u1m, u2m, x, y);
 }
 
 // ---- verification with a known public key (fuel Signature::verify) ----
@@ -467,41 +505,33 @@ DEV void secp_prologue(const u32 sig_raw[16], const u32 dig_raw[8], secp_pro& o)
 // z = digest mod n, u1 = z/s, u2 = r/s, P = u1 G + u2 Q != infinity, accept iff x(P) mod n == r.
 // pub_raw: the 64 key bytes as 16 little-endian u32 loads. The same ladders then run with the key
 // in place of R.
+// the key as an affine point and the checks that do not need the scalars
 template <class C>
-DEV void secp_prologue_verify(const u32 sig_raw[16], const u32 dig_raw[8], const u32 pub_raw[16], secp_pro& o) {
+DEV u32 secp_decode_verify(const u32 sig_raw[16], const u32 pub_raw[16], secp_sig& g, fe& x, fe& y) {
   typedef typename C::Fp Fp;
-  typedef typename C::Fn Fn;
-  const u32(&n)[8] = C::n32();
-  u32 r[8], s[8], z[8], sraw[8], xw[8], yw[8];
-#pragma unroll
-  for (int i = 0; i < 8; i++) sraw[i] = sig_raw[8 + i];
-  sraw[0] &= ~0x80u;
-  words_from_be_bytes(sig_raw, r);
-  words_from_be_bytes(sraw, s);
-  words_from_be_bytes(dig_raw, z);
+  u32 xw[8], yw[8];
   words_from_be_bytes(pub_raw, xw);
   words_from_be_bytes(pub_raw + 8, yw);
-  o.status = ST_OK;
-  if (words_is_zero(r) || !words_lt(r, n)) o.status = ST_BAD_R;
-  else if (words_is_zero(s) || !words_lt(s, n)) o.status = ST_BAD_S;
-  else if (C::LOW_S && words_lt(C::nhalf32(), s)) o.status = ST_HIGH_S;
-  else if (!words_lt(xw, C::p32()) || !words_lt(yw, C::p32())) o.status = ST_BAD_KEY;
-  if (!words_lt(z, n)) {
-    u32 t[8];
-    words_sub(z, n, t);
-#pragma unroll
-    for (int i = 0; i < 8; i++) z[i] = t[i];
-  }
-  const fe x = to_mont<Fp>(fe_from_words(xw));
-  const fe y = to_mont<Fp>(fe_from_words(yw));
-  fe rhs = mont_mul<Fp>(mont_sqr<Fp>(x), x);
-  if (C::A_IS_M3) rhs = fsub<Fp>(rhs, fadd<Fp>(fdbl<Fp>(x), x));
-  rhs = fadd<Fp>(rhs, C::b());
-  if (o.status == ST_OK && !feq<Fp>(mont_sqr<Fp>(y), rhs)) o.status = ST_BAD_KEY;
+  u32 st = secp_decode_sig<C>(sig_raw, g);
+  if (st == ST_OK && C::LOW_S && words_lt(C::nhalf32(), g.s)) st = ST_HIGH_S;
+  if (st == ST_OK && (!words_lt(xw, C::p32()) || !words_lt(yw, C::p32()))) st = ST_BAD_KEY;
+  x = to_mont<Fp>(fe_from_words(xw));
+  y = to_mont<Fp>(fe_from_words(yw));
+  if (st == ST_OK && !feq<Fp>(mont_sqr<Fp>(y), secp_rhs<C>(x))) st = ST_BAD_KEY;
+  return st;
+}
+
+template <class C>
+DEV void secp_prologue_verify(const u32 sig_raw[16], const u32 dig_raw[8], const u32 pub_raw[16], secp_pro& o) {
+  typedef typename C::Fn Fn;
+  secp_sig g;
+  fe x, y;
+  o.status = secp_decode_verify<C>(sig_raw, pub_raw, g, x, y);
+  secp_decode_digest<C>(dig_raw, g);
   // u1 = z/s, u2 = r/s (mod n)
-  const fe sinv = finv<Fn>(to_mont<Fn>(fe_from_words(s)));
-  const fe u1m = mont_mul<Fn>(to_mont<Fn>(fe_from_words(z)), sinv);
-  const fe u2m = mont_mul<Fn>(to_mont<Fn>(fe_from_words(r)), sinv);
+  const fe sinv = finv<Fn>(to_mont<Fn>(fe_from_words(g.s)));
+  const fe u1m = mont_mul<Fn>(to_mont<Fn>(fe_from_words(g.z)), sinv);
+  const fe u2m = mont_mul<Fn>(to_mont<Fn>(fe_from_words(g.r)), sinv);
   secp_scalars<C>(o, u1m, u2m, x, y);
 }
 
@@ -771,6 +801,40 @@ DEV jacs secp_ladder_s(const secp_pro& o, Tab& tab, const GTab& gt, bool& exc) {
   return acc;
 }
 
+// ---- u1 G from wide fixed-base tables ----
+// For every 16-bit window i of a scalar the 32,768 odd multiples (2j + 1) 2^(16 i) G, affine as
+// (x, w = 2y), 64 bytes each: 33.5 MB per curve, built on the GPU once per device (kern_comb.hip).
+// u1 G then takes 16 mixed additions and no doubling, against 30 (secp256k1) or 29 (P-256) additions
+// from 9-bit windows on the ladder's chain.
+constexpr int COMB_BITS = 16;
+constexpr int COMB_WINDOWS = 256 / COMB_BITS;
+constexpr u32 COMB_ENTRIES = 1u << (COMB_BITS - 1);
+
+struct comb_entry {
+  u32 v[16];  // x, w as 8 little-endian words each, canonical Montgomery form
+};
+
+// acc + the 16 entries that u1's digits spell (o.c1, o.g_neg from secp_carriers<C, true>). Comb:
+// load(i, j, comb_entry&). The next entry's load is issued before an addition that does not need it.
+template <class C, class Comb>
+DEV jacs secp_comb(jacs acc, const secp_pro& o, const Comb& comb, bool& exc) {
+  auto digit = [&](int i) { return (o.c1[i >> 1] >> ((i & 1) * 16)) & 0xFFFFu; };
+  auto load = [&](int i, comb_entry& e) {
+    const u32 d = digit(i);
+    comb.load(i, ((d < COMB_ENTRIES) ? ~d : d) & (COMB_ENTRIES - 1u), e);
+  };
+  comb_entry e;
+  load(0, e);
+#pragma unroll 1
+  for (int i = 0; i < COMB_WINDOWS; i++) {
+    const sfe x = s_from(fe_from_words(e.v)), w = s_from(fe_from_words(e.v + 8));
+    const bool neg = (digit(i) < COMB_ENTRIES) != o.g_neg;
+    if (i + 1 < COMB_WINDOWS) load(i + 1, e);
+    acc = smadd<C>(acc, x, s_neg_if(neg, w), exc);
+  }
+  return acc;
+}
+
 // secp_ladder_s with its result in field.hpp's form. R-table stored per lane (secp_build_table).
 // GTab provides load(idx, fe& x, fe& y) for the odd multiples (2 idx + 1) G: 128 of them for
 // fixed-base windows of WGB = 8 bits, 256 for 9.
@@ -803,19 +867,24 @@ DEV jacf secp_ladder_careful(const secp_pro& o, const GTab& gt) {
   return acc;
 }
 
-// Jacobian -> affine big-endian X||Y (16 words as stored to memory)
+// affine x, y (Montgomery form) from X, Y, Z and 1 / Z, as big-endian X || Y (16 words as stored)
 template <class C>
-DEV void secp_output(const jac& Q, u32 out_raw[16]) {
+DEV void secp_store_affine(const fe& X, const fe& Y, const fe& zi, u32 out_raw[16]) {
   typedef typename C::Fp F;
-  const fe zi = finv<F>(Q.Z);
   const fe zi2 = mont_sqr<F>(zi);
-  const fe x = from_mont<F>(mont_mul<F>(Q.X, zi2));
-  const fe y = from_mont<F>(mont_mul<F>(Q.Y, mont_mul<F>(zi2, zi)));
+  const fe x = from_mont<F>(mont_mul<F>(X, zi2));
+  const fe y = from_mont<F>(mont_mul<F>(Y, mont_mul<F>(zi2, zi)));
   u32 w[8];
   fe_to_words(x, w);
   words_to_be_bytes(w, out_raw);
   fe_to_words(y, w);
   words_to_be_bytes(w, out_raw + 8);
+}
+
+// Jacobian -> affine
+template <class C>
+DEV void secp_output(const jac& Q, u32 out_raw[16]) {
+  secp_store_affine<C>(Q.X, Q.Y, finv<typename C::Fp>(Q.Z), out_raw);
 }
 
 }  // namespace sigops

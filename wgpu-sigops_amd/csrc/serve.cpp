@@ -740,7 +740,8 @@ void RingEngine::publish_counts() {
   L.seq = seq;
   L.lane_slots = res.lane_slots;
   L.grid = res.grid;
-  L.g_window = res.g_window;
+  L.comb_k1 = res.comb_k1;
+  L.comb_r1 = res.comb_r1;
   sigops::stream_poll_ticks(S->cfg.device, L);
   const bool ok = e.ev && sigops::launch_stream(L, res.stream) == hipSuccess &&
                   hipEventRecord(e.ev, res.stream) == hipSuccess;

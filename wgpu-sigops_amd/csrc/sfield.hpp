@@ -391,6 +391,26 @@ DEV_MUL sfe s_dot_sqr(const sfe& a, const sfe& b, const sfe& c) {
   return r;
 }
 
+// x to a fixed exponent along an addition chain (field.hpp, fpow_chain)
+template <class F, class CH, int S>
+DEV void s_chain_steps(sfe* t) {
+  if constexpr (S < CH::N) {
+    sfe v = t[CH::SRC[S]];
+#pragma unroll 1
+    for (int k = 0; k < CH::NSQ[S]; k++) v = s_sqr<F>(v);
+    if constexpr (CH::MUL[S] >= 0) v = s_mul<F>(v, t[CH::MUL[S]]);
+    t[CH::DST[S]] = v;
+    s_chain_steps<F, CH, S + 1>(t);
+  }
+}
+template <class F, class CH>
+DEV sfe s_pow_chain(const sfe& x) {
+  sfe t[CH::SLOTS];
+  t[0] = x;
+  s_chain_steps<F, CH, 0>(t);
+  return t[CH::RESULT];
+}
+
 // SCALE (a^2 - b^2) 2^-261 with one reduction
 template <class F, int SCALE = 1>
 DEV_MUL sfe s_sqr_diff(const sfe& a, const sfe& b) {

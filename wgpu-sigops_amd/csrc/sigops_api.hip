@@ -10,6 +10,7 @@
 #include <atomic>
 #include <chrono>
 #include <cstdio>
+#include <map>
 #include <memory>
 #include <mutex>
 #include <cstring>
@@ -39,6 +40,55 @@ constexpr int NOALLOC_MAX_DEVICES = 64;
 std::mutex g_scratch_mu;
 void* g_scratch[NOALLOC_MAX_DEVICES];  // device address of `scratch` per device, 0 until looked up
 
+// ---- wide fixed-base tables ----
+// 33.5 MB per secp curve and 50 MB for Ed25519, built on the GPU by the first context on a device and shared by all contexts
+// there (servers hold one per slot); freed with the last one. They are only read after the build.
+struct CombTables {
+  void* t[3] = {};  // secp256k1, secp256r1, Ed25519
+  unsigned refs = 0;
+};
+std::mutex g_comb_mu;
+std::map<int, CombTables> g_comb;
+
+// the device is current; gtab: the resident tables, in the order of CombTables; s: a stream of the
+// caller's. Returns when the tables are complete.
+hipError_t comb_acquire(int device, const void* const gtab[3], hipStream_t s, CombTables& out) {
+  std::lock_guard<std::mutex> lk(g_comb_mu);
+  CombTables& t = g_comb[device];
+  if (t.refs == 0) {
+    void* tmp = nullptr;
+    hipError_t e = hipMalloc(&tmp, sigops::comb_tmp_bytes());
+    for (int k = 0; k < 3; k++) {  // one after the other: they share tmp
+      if (e == hipSuccess) e = hipMalloc(&t.t[k], sigops::comb_bytes(k));
+      if (e == hipSuccess) e = sigops::launch_comb_build(k, gtab[k], t.t[k], tmp, s);
+    }
+    const hipError_t se = hipStreamSynchronize(s);
+    if (e == hipSuccess) e = se;
+    if (tmp) (void)hipFree(tmp);
+    if (e != hipSuccess) {
+      for (void* p : t.t)
+        if (p) (void)hipFree(p);
+      g_comb.erase(device);
+      return e;
+    }
+  }
+  t.refs++;
+  out = t;
+  return hipSuccess;
+}
+
+void comb_release(int device) {
+  std::lock_guard<std::mutex> lk(g_comb_mu);
+  auto it = g_comb.find(device);
+  if (it == g_comb.end() || --it->second.refs) return;
+  for (void* p : it->second.t) (void)hipFree(p);
+  g_comb.erase(it);
+}
+
+// Items the stages' scratch holds (470 MB); a larger device call runs in consecutive pieces of this
+// size on its stream.
+constexpr size_t STAGE_ITEMS = 1u << 22;
+
 constexpr uint8_t CANARY = 0xEE;
 // largest caller table: 16 entries x 3 coordinates x 24 limbs (l = 11)
 constexpr size_t TABLE_LIMBS_MAX = 16 * 3 * 24;
@@ -54,17 +104,20 @@ struct sigops_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   uint32_t grid = 0;
+  uint32_t blocks_per_cu = 0;
   uint32_t slots = 0;
   uint32_t max_batch = 1u << 22;
   void* d_gtab_k1 = nullptr;
   void* d_gtab_r1 = nullptr;
   void* d_btab = nullptr;
+  CombTables comb;            // wide fixed-base tables, shared by the contexts of this device
+  void* d_scratch = nullptr;  // ItemScratch of the secp stages: scratch_stride positions
+  uint32_t scratch_stride = 0;
   void* d_lane_tab = nullptr;
   uint32_t* d_pend = nullptr;  // [0] = count, [1 ..] = list
   // mixed batch
   uint32_t tile_rounds = 1;
   uint32_t waves = 2;  // waves per SIMD the mixed batch's persistent kernel is built for
-  uint32_t g_window = 8;  // the mixed batch's fixed-base window (secp streams), 8 or 9 bits
   bool use_graph = true;
   uint8_t* d_rank = nullptr;
   uint32_t* d_work = nullptr;
@@ -186,22 +239,36 @@ __global__ void k_fill_bytes(uint8_t* p, uint8_t v, size_t n) {
     p[i] = v;
 }
 
-// gtab: the fixed-base table to use (NULL: the resident table of G, with the context's window; a
-// caller's converted table holds 128 entries, so 8-bit windows)
+// a device address `bytes` further on
+const void* at(const void* p, size_t bytes) { return (const uint8_t*)p + bytes; }
+void* at(void* p, size_t bytes) { return (uint8_t*)p + bytes; }
+
+// gtab8: a caller's converted table (8-bit windows), or NULL for the resident ones
+sigops::SecpLaunch secp_launch(sigops_ctx* c, int curve, const void* gtab8 = nullptr) {
+  sigops::SecpLaunch L{};
+  L.gtab = curve == 0 ? c->d_gtab_k1 : c->d_gtab_r1;
+  L.gtab8 = gtab8;
+  L.comb = c->comb.t[curve];
+  L.scratch = c->d_scratch;
+  L.scratch_stride = c->scratch_stride;
+  L.lane_tab = c->d_lane_tab;
+  L.slots = c->slots;
+  L.grid = c->grid;
+  L.pend_list = c->d_pend + 1;
+  L.pend_count = c->d_pend;
+  return L;
+}
+
 int secp_recover_dev(sigops_ctx* c, int curve, const void* d_sigs, const void* d_digs, size_t n, void* d_out,
-                     void* d_status, hipStream_t s, const void* gtab = nullptr) {
+                     void* d_status, hipStream_t s, const void* gtab8 = nullptr) {
   if (n > c->max_batch) return fail(c, SIGOPS_E_ARG, "n exceeds max_batch");
   if (n == 0) return SIGOPS_OK;
   if (c->fault & SIGOPS_FAULT_SKIP_COMPUTE) return SIGOPS_OK;
-  const uint32_t w = gtab ? 8u : c->g_window;
-  if (curve == 0)
-    HIPCHK(c, sigops::launch_secp_recover_CurveK1(d_sigs, d_digs, d_out, d_status, (uint32_t)n,
-                                                 gtab ? gtab : c->d_gtab_k1, c->d_lane_tab, c->slots, c->d_pend + 1,
-                                                 c->d_pend, c->grid, w, s));
-  else
-    HIPCHK(c, sigops::launch_secp_recover_CurveR1(d_sigs, d_digs, d_out, d_status, (uint32_t)n,
-                                                 gtab ? gtab : c->d_gtab_r1, c->d_lane_tab, c->slots, c->d_pend + 1,
-                                                 c->d_pend, c->grid, w, s));
+  const sigops::SecpLaunch L = secp_launch(c, curve, gtab8);
+  const auto launch = curve == 0 ? sigops::launch_secp_recover_CurveK1 : sigops::launch_secp_recover_CurveR1;
+  for (size_t a = 0; a < n; a += STAGE_ITEMS)
+    HIPCHK(c, launch(L, at(d_sigs, 64 * a), at(d_digs, 32 * a), at(d_out, 64 * a), at(d_status, a),
+                     (uint32_t)std::min(n - a, STAGE_ITEMS), s));
   return SIGOPS_OK;
 }
 
@@ -275,14 +342,11 @@ int secp_verify_dev(sigops_ctx* c, int curve, const void* d_sigs, const void* d_
   if (n == 0) return SIGOPS_OK;
   if (!d_sigs || !d_digs || !d_pubs || !d_status) return fail(c, SIGOPS_E_ARG, "NULL buffer");
   if (c->fault & SIGOPS_FAULT_SKIP_COMPUTE) return SIGOPS_OK;
-  if (curve == 0)
-    HIPCHK(c, sigops::launch_secp_verify_CurveK1(d_sigs, d_digs, d_pubs, d_status, (uint32_t)n, c->d_gtab_k1,
-                                                c->d_lane_tab, c->slots, c->d_pend + 1, c->d_pend, c->grid,
-                                                c->g_window, s));
-  else
-    HIPCHK(c, sigops::launch_secp_verify_CurveR1(d_sigs, d_digs, d_pubs, d_status, (uint32_t)n, c->d_gtab_r1,
-                                                c->d_lane_tab, c->slots, c->d_pend + 1, c->d_pend, c->grid,
-                                                c->g_window, s));
+  const sigops::SecpLaunch L = secp_launch(c, curve);
+  const auto launch = curve == 0 ? sigops::launch_secp_verify_CurveK1 : sigops::launch_secp_verify_CurveR1;
+  for (size_t a = 0; a < n; a += STAGE_ITEMS)
+    HIPCHK(c, launch(L, at(d_sigs, 64 * a), at(d_digs, 32 * a), at(d_pubs, 64 * a), at(d_status, a),
+                     (uint32_t)std::min(n - a, STAGE_ITEMS), s));
   return SIGOPS_OK;
 }
 
@@ -354,10 +418,8 @@ sigops_ctx* sigops_create(const sigops_config* cfg) {
     return nullptr;
   }
   c->waves = cfg->waves_per_simd ? cfg->waves_per_simd : 2;
-  // 9-bit windows measured faster on the MI355X (and chosen by the autotuner); the one-wave kernel
-  // is built with 8-bit ones only
-  c->g_window = cfg->g_window ? cfg->g_window : (c->waves == 1 ? 8 : 9);
   const uint32_t bpc = cfg->blocks_per_cu ? cfg->blocks_per_cu : c->waves;
+  c->blocks_per_cu = bpc;
   c->grid = (uint32_t)cus * bpc;
   c->slots = c->grid * 256;
   if ((e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking)) != hipSuccess) return bad(e, "stream");
@@ -372,6 +434,14 @@ sigops_ctx* sigops_create(const sigops_config* cfg) {
     return bad(e, "upload");
   if ((e = hipMemcpy(c->d_btab, sigops::ED_BTABLE, sizeof(sigops::ED_BTABLE), hipMemcpyHostToDevice)) != hipSuccess)
     return bad(e, "upload");
+  const void* const gtabs[3] = {c->d_gtab_k1, c->d_gtab_r1, c->d_btab};
+  if ((e = comb_acquire(c->device, gtabs, c->stream, c->comb)) != hipSuccess)
+    return bad(e, "wide fixed-base tables");
+  const size_t positions = std::min<size_t>(c->max_batch, STAGE_ITEMS) +
+                           (size_t)sigops::NBUCKETS * 64 * sigops::MAX_TILE_ROUNDS;
+  c->scratch_stride = (uint32_t)positions;
+  if ((e = hipMalloc(&c->d_scratch, positions * sigops::ITEM_SCRATCH_BYTES)) != hipSuccess)
+    return bad(e, "hipMalloc item scratch");
   const size_t lane_bytes =
       (size_t)c->slots * std::max(sigops::SECP_LANE_TAB_BYTES, sigops::ED_LANE_TAB_BYTES);
   if ((e = hipMalloc(&c->d_lane_tab, lane_bytes)) != hipSuccess) return bad(e, "hipMalloc lane tables");
@@ -430,11 +500,12 @@ void sigops_destroy(sigops_ctx* c) {
   if (c->d_sctr) (void)hipFree(c->d_sctr);
   for (hipEvent_t e : c->stage_ev)
     if (e) (void)hipEventDestroy(e);
-  for (void* p : {c->d_gtab_k1, c->d_gtab_r1, c->d_btab, c->d_lane_tab, (void*)c->d_pend, c->in.p, c->aux.p,
+  for (void* p : {c->d_gtab_k1, c->d_gtab_r1, c->d_btab, c->d_scratch, c->d_lane_tab, (void*)c->d_pend, c->in.p, c->aux.p,
                   c->msg.p, c->off.p, c->out.p, c->st.p, c->sch.p, (void*)c->d_rank, (void*)c->d_work,
                   (void*)c->d_order, (void*)c->d_io, (void*)c->d_hq, (void*)c->d_horder, (void*)c->d_tlimbs,
                   c->d_ctab, (void*)c->d_tflags})
     if (p) (void)hipFree(p);
+  if (c->comb.refs) comb_release(c->device);
   c->pool.reset();
   sigops_host::pinned_free(c->h_up);
   sigops_host::pinned_free(c->h_down);
@@ -503,6 +574,14 @@ static int ed_verify_dev(sigops_ctx* c, const void* d_sigs, const void* d_pubkey
   if (!d_sigs || !d_pubkeys || !d_msgs || !d_msg_off || !d_status) return fail(c, SIGOPS_E_ARG, "NULL buffer");
   if (((uintptr_t)d_msgs & 3u) != 0) return fail(c, SIGOPS_E_ARG, "d_msgs must be 4-byte aligned");
   hipStream_t s = (hipStream_t)stream;
+  // (8 lanes of the lane tables per item, for challenges that need the full-length check)
+  if (!btab && n <= sigops::QUAD_MAX_ITEMS && c->slots >= sigops::QUAD_MAX_ITEMS * 8) {
+    if (c->fault & SIGOPS_FAULT_SKIP_COMPUTE) return SIGOPS_OK;
+    const sigops::EdQuadLaunch L{d_sigs, d_pubkeys, d_msgs, d_msg_off, d_status, c->comb.t[2], c->d_btab, c->d_lane_tab,
+                                 c->slots};
+    HIPCHK(c, sigops::launch_quad_ed(strict, L, (uint32_t)n, s));
+    return SIGOPS_OK;
+  }
   HIPCHK(c, sigops::launch_set_batch_io(c->d_io, {nullptr, d_sigs, d_pubkeys, d_msgs, d_msg_off, nullptr, d_status,
                                                   (uint32_t)n}, s));
   sigops::BatchLaunch L{};
@@ -648,6 +727,14 @@ int sigops_batch_dev(sigops_ctx* c, const void* d_schemes, const void* d_sigs, c
   if (!d_schemes || !d_sigs || !d_aux || !d_msgs || !d_msg_off || !d_out || !d_status)
     return fail(c, SIGOPS_E_ARG, "NULL buffer");
   if (((uintptr_t)d_msgs & 3u) != 0) return fail(c, SIGOPS_E_ARG, "d_msgs must be 4-byte aligned");
+  if (n > STAGE_ITEMS) {
+    for (size_t a = 0; a < n; a += STAGE_ITEMS) {
+      const int rc = sigops_batch_dev(c, at(d_schemes, a), at(d_sigs, 64 * a), at(d_aux, 32 * a), d_msgs, d_msg_off + a,
+                                      std::min(n - a, STAGE_ITEMS), at(d_out, 64 * a), at(d_status, a), stream);
+      if (rc) return rc;
+    }
+    return SIGOPS_OK;
+  }
   hipStream_t s = (hipStream_t)stream;
   // the call's buffers and n go to device memory first (stream-ordered, by value at enqueue time),
   // so one captured graph serves every call and back-to-back enqueues do not race
@@ -668,8 +755,12 @@ int sigops_batch_dev(sigops_ctx* c, const void* d_schemes, const void* d_sigs, c
   L.grid = c->grid;
   L.aux_grid = std::min<uint32_t>(c->grid, (uint32_t)((n + 255) / 256));
   L.tile_rounds = c->tile_rounds;
+  L.comb_k1 = c->comb.t[0];
+  L.comb_r1 = c->comb.t[1];
+  L.scratch = c->d_scratch;
+  L.scratch_stride = c->scratch_stride;
+  L.stage_grid = c->grid / c->blocks_per_cu;
   L.waves = c->waves;
-  L.g_window = c->g_window;
   L.stage_ev = nullptr;
   if (c->stage_timing) {
     L.stage_ev = c->stage_ev;
@@ -965,7 +1056,8 @@ int batch_streamed(sigops_ctx* c, const uint8_t* schemes, const uint8_t* sigs, c
   L.seq = seq;
   L.lane_slots = c->slots;
   L.grid = std::min<uint32_t>(c->grid, (uint32_t)((g.slots + 3) / 4));
-  L.g_window = c->g_window;
+  L.comb_k1 = c->comb.t[0];
+  L.comb_r1 = c->comb.t[1];
   sigops::stream_poll_ticks(c->device, L);
   HIPCHK(c, hipEventRecord(c->s_tev[0], s));
   if (!(c->fault & SIGOPS_FAULT_SKIP_COMPUTE)) HIPCHK(c, sigops::launch_stream(L, s));
@@ -1034,7 +1126,8 @@ int sigops_ring_resources(sigops_ctx* c, sigops::RingResources* r) {
   r->lane_tab = c->d_lane_tab;
   r->lane_slots = c->slots;
   r->grid = c->grid;
-  r->g_window = c->g_window;
+  r->comb_k1 = c->comb.t[0];
+  r->comb_r1 = c->comb.t[1];
   r->bucket_order = c->bucket_order;
   r->stream = c->stream;
   return SIGOPS_OK;
