@@ -88,3 +88,39 @@ def test_ed25519_sizes(ctx, strict):
         valid, st = ctx.ed25519_verify(sigs[at], keys[at], data, moff, strict=strict)
         assert np.array_equal(valid, good[at]), n
         assert np.array_equal(st == 0, good[at]), n
+
+
+def test_mixed_sizes(ctx):
+    """mixed batches around the sizes where they change from four lanes per item to one, and from
+    copying to streaming"""
+    rows = []  # scheme, signature, digest or key, message, key out, status
+    for curve in (0, 1):
+        cases = edge_cases.secp_cases(curve)
+        rows += [(curve, c[1], c[2], b"", e[1], e[0]) for c, e in zip(cases, edge_cases.secp_expected(curve, cases))]
+        s, d, _, _ = O.gen_secp(curve, 41, 200, corrupt_ppm=200000)
+        o, t = O.recover_batch(curve, s, d)
+        rows += [(curve, s[i].tobytes(), d[i].tobytes(), b"", o[i].tobytes(), int(t[i])) for i in range(200)]
+    cases = edge_cases.ed_cases()
+    rows += [(2, c[1], c[2], bytes(c[3]), bytes(64), None) for c in cases]
+    good = dict(zip(range(len(rows) - len(cases), len(rows)), edge_cases.ed_expected(cases)))
+    off = np.concatenate([[0], np.cumsum(np.arange(200) * 41 % 4200)]).astype(np.uint64)
+    s, k, m, _ = O.gen_ed25519(43, 200, off, corrupt_ppm=200000)
+    ok = O.verify_batch(s, k, m, off)
+    for i in range(200):
+        good[len(rows)] = bool(ok[i])
+        rows.append((2, s[i].tobytes(), k[i].tobytes(), m[int(off[i]):int(off[i + 1])].tobytes(), bytes(64), None))
+    schemes = np.array([r[0] for r in rows], np.uint8)
+    sigs, aux, out = (_bytes([r[j] for r in rows], w) for j, w in ((1, 64), (2, 32), (4, 64)))
+    lens = np.array([len(r[3]) for r in rows])
+    perm = np.random.default_rng(5).permutation(len(rows))
+    for n in (1, 15, 17, len(rows), 16384, 24576, 24577, 65535, 65536):
+        print(f"mixed n={n}", flush=True)
+        at = perm[_at(n, len(rows), n)]
+        moff = np.concatenate([[0], np.cumsum(lens[at])]).astype(np.uint64)
+        data = np.frombuffer(b"".join(rows[i][3] for i in at), np.uint8)
+        got, st = ctx.batch(schemes[at], sigs[at], aux[at], data, moff)
+        assert np.array_equal(got, out[at]), n
+        for j in range(len(rows)):
+            want = rows[j][5]
+            mine = st[at == j]
+            assert np.all((mine == 0) == good[j]) if want is None else np.all(mine == want), (n, j)

@@ -15,8 +15,9 @@
 // is no exceptional path. Scalar multiplication shares one doubling chain (Strauss-Shamir):
 //   [s]B: w = 8 signed odd digits over an LDS-staged table of (2j+1)B in affine Niels form;
 //   [k](-A): w = 4 signed odd digits over a per-lane table of odd multiples in cached form.
-// The kernels that verify only Ed25519 run the lattice-reduced form of the final check instead
-// (ed_check_lattice: a 136-bit chain, same results); the mixed-scheme kernels keep the full one.
+// The kernels run the lattice-reduced form of the final check (a 136-bit chain, same results) with
+// [v]B from wide tables (ed_check_lattice_wide), or from 8-bit ones for a caller's table; the
+// full-length form is left for challenges without a short pair.
 #pragma once
 #include "secp.hpp"  // nibble / byte8 helpers and status codes
 #include "sha512.hpp"
@@ -53,17 +54,6 @@ DEV cached to_cached(const ext& P) {
   c.z = P.Z;
   c.t2d = mont_mul<Fe>(P.T, fe_from_const(ED_D2));
   return c;
-}
-
-// -Q when neg: swap Y+X and Y-X and negate 2dT (lazily)
-DEV cached neg_cached_if(bool neg, const cached& c) {
-  const u32 m = lane_mask(neg);
-  cached r;
-  r.ypx = fsel_mask(m, c.ymx, c.ypx);
-  r.ymx = fsel_mask(m, c.ypx, c.ymx);
-  r.z = c.z;
-  r.t2d = fsel_mask(m, fsub_nr<Fe, 2, 1>(fe_zero(), c.t2d), c.t2d);
-  return r;
 }
 
 // completed point (E:G:H:Tc) with x = E/Tc, y = G/H -> extended; each pair product within bounds
@@ -114,11 +104,78 @@ DEV ext eadd_niels(const ext& P, const fe& ypx, const fe& ymx, const fe& t2d, bo
   return completed_to_ext(E, G, H, Tc, want_t);               // [1]x[1], [2]x[3], [3]x[1], [1]x[2]
 }
 
+// ---- the ladders' group law, on signed arithmetic (sfield.hpp): no folds and no biases; a doubling
+// takes 1,070 VALU instructions against edbl's 1,250 ----
+struct sext {
+  sfe X, Y, Z, T;  // normalised
+};
+struct scached {  // (Y+X, Y-X, Z, 2d*T); t2d may be negated
+  sfe ypx, ymx, z, t2d;
+};
+
+DEV sext sext_identity() {
+  const sfe zero = s_from(fe_zero()), one = s_from(fe_from_const(Fe::ONE));
+  return sext{zero, one, one, zero};
+}
+
+DEV sext s_completed(const sfe& E, const sfe& G, const sfe& H, const sfe& Tc, bool want_t) {
+  sext r;
+  r.X = s_mul<Fe>(E, Tc);
+  r.Y = s_mul<Fe>(G, H);
+  r.Z = s_mul<Fe>(H, Tc);
+  r.T = want_t ? s_mul<Fe>(E, G) : s_from(fe_zero());
+  return r;
+}
+
+// doubling; E = 2XY as a product
+DEV sext sedbl(const sext& P, bool want_t) {
+  const sfe XX = s_sqr<Fe>(P.X), YY = s_sqr<Fe>(P.Y), ZZ2 = s_sqr<Fe, 2>(P.Z);
+  const sfe H = s_sub(YY, XX);
+  return s_completed(s_mul<Fe, 2>(P.X, P.Y), s_add(YY, XX), H, s_sub(ZZ2, H), want_t);
+}
+
+DEV sext seadd(const sext& P, const scached& Q, bool want_t) {
+  const sfe PP = s_mul<Fe>(s_add(P.Y, P.X), Q.ypx), MM = s_mul<Fe>(s_sub(P.Y, P.X), Q.ymx);
+  const sfe TT = s_mul<Fe>(P.T, Q.t2d), ZZ2 = s_mul<Fe, 2>(P.Z, Q.z);
+  return s_completed(s_sub(PP, MM), s_add(PP, MM), s_add(ZZ2, TT), s_sub(ZZ2, TT), want_t);
+}
+
+// + an affine point given as (y + x)/2, (y - x)/2, d x y (the wide table's entries)
+DEV sext seadd_half(const sext& P, const sfe& ypx, const sfe& ymx, const sfe& td, bool want_t) {
+  const sfe PP = s_mul<Fe>(s_add(P.Y, P.X), ypx), MM = s_mul<Fe>(s_sub(P.Y, P.X), ymx);
+  const sfe TT = s_mul<Fe>(P.T, td);
+  return s_completed(s_sub(PP, MM), s_add(PP, MM), s_add(P.Z, TT), s_sub(P.Z, TT), want_t);
+}
+
+// + an affine point given as y + x, y - x, 2dxy
+DEV sext seadd_niels(const sext& P, const sfe& ypx, const sfe& ymx, const sfe& t2d, bool want_t) {
+  const sfe PP = s_mul<Fe>(s_add(P.Y, P.X), ypx), MM = s_mul<Fe>(s_sub(P.Y, P.X), ymx);
+  const sfe TT = s_mul<Fe>(P.T, t2d), ZZ2 = s_carry(s_dbl(P.Z));
+  return s_completed(s_sub(PP, MM), s_add(PP, MM), s_add(ZZ2, TT), s_sub(ZZ2, TT), want_t);
+}
+
+DEV scached s_to_cached(const sext& P) {
+  scached c;
+  c.ypx = s_carry(s_add(P.Y, P.X));
+  c.ymx = s_carry(s_sub(P.Y, P.X));
+  c.z = P.Z;
+  c.t2d = s_mul<Fe>(P.T, s_from(fe_from_const(ED_D2)));
+  return c;
+}
+DEV cached s_raw(const scached& c) { return cached{s_raw(c.ypx), s_raw(c.ymx), s_raw(c.z), s_raw(c.t2d)}; }
+
+// a table entry as stored, or its negative: Y+X and Y-X swapped, 2dT negated
+DEV scached s_entry(const cached& c, bool neg) {
+  const u32 m = lane_mask(neg);
+  const sfe a = s_unraw<Fe>(c.ypx), b = s_unraw<Fe>(c.ymx);
+  return scached{s_sel(m, b, a), s_sel(m, a, b), s_unraw<Fe>(c.z), s_neg_if(neg, s_unraw<Fe>(c.t2d))};
+}
+
 // dalek FieldElement::sqrt_ratio_i (field.rs): returns was_nonzero_square, r = nonnegative root
 DEV bool sqrt_ratio_i(const fe& u, const fe& v, fe& r_out) {
   const fe v3 = mont_mul<Fe>(mont_sqr<Fe>(v), v);
   const fe v7 = mont_mul<Fe>(mont_sqr<Fe>(v3), v);
-  fe r = mont_mul<Fe>(mont_mul<Fe>(u, v3), fpow_chain<Fe, CH_ED_P58>(mont_mul<Fe>(u, v7)));
+  fe r = mont_mul<Fe>(mont_mul<Fe>(u, v3), s_to_fe<Fe, 1>(s_pow_chain<Fe, CH_ED_P58>(s_from(mont_mul<Fe>(u, v7)))));
   const fe check = mont_mul<Fe>(v, mont_sqr<Fe>(r));
   const fe i = fe_from_const(ED_SQRTM1);
   const fe neg_u = fneg<Fe>(u);
@@ -372,80 +429,177 @@ DEV bool ed_lattice(const u32 k[8], u32 c0[5], u32 c1[5], bool& c0_neg) {
   return ok && hi0 == 0 && (c1[4] >> (ED_LAT_BITS - 128)) == 0;
 }
 
-// table of the odd multiples (2e+1) P, e = 0..7, of P = (x, y) in cached form at entries e0..e0+7
+// table of the odd multiples (2e+1) P, e = 0..7, of P = (x, y) in cached form (raw signed limbs) at
+// entries e0..e0+7
 template <class Tab>
 DEV void ed_table_odd(Tab& tab, int e0, const fe& x, const fe& y) {
-  ext P;
-  P.X = x;
-  P.Y = y;
-  P.Z = fe_from_const(Fe::ONE);
-  P.T = mont_mul<Fe>(x, y);
-  const cached P2 = to_cached(edbl(P, true));
-  ext T = P;
-  tab.store(e0, to_cached(P));
+  sext P;
+  P.X = s_from(x);
+  P.Y = s_from(y);
+  P.Z = s_from(fe_from_const(Fe::ONE));
+  P.T = s_mul<Fe>(P.X, P.Y);
+  const scached P2 = s_to_cached(sedbl(P, true));
+  sext T = P;
+  tab.store(e0, s_raw(s_to_cached(P)));
 #pragma unroll 1
   for (int e = 1; e < 8; e++) {
-    T = eadd_cached(T, P2, true);
-    tab.store(e0 + e, to_cached(T));
+    T = seadd(T, P2, true);
+    tab.store(e0 + e, s_raw(s_to_cached(T)));
   }
 }
 
 // acc + (digit's odd multiple of the table's point, negated per digit and stream sign); the table
 // holds (2j+1) B at entries base + j in affine Niels form
 template <class BTab>
-DEV ext ed_add_b(const ext& acc, const BTab& bt, u32 base, u32 digit, bool neg_stream, bool want_t) {
+DEV sext ed_add_b(const sext& acc, const BTab& bt, u32 base, u32 digit, bool neg_stream, bool want_t) {
   const bool neg = (digit < 128) != neg_stream;
   fe ypx, ymx, t2d;
   bt.load(base + (((digit < 128) ? ~digit : digit) & 127u), ypx, ymx, t2d);
   const u32 m = lane_mask(neg);
-  return eadd_niels(acc, fsel_mask(m, ymx, ypx), fsel_mask(m, ypx, ymx),
-                    fsel_mask(m, fsub_nr<Fe, 2, 1>(fe_zero(), t2d), t2d), want_t);
+  const sfe a = s_from(ypx), b = s_from(ymx);
+  return seadd_niels(acc, s_sel(m, b, a), s_sel(m, a, b), s_neg_if(neg, s_from(t2d)), want_t);
 }
 
 // the cached identity (Y+X, Y-X, Z, 2dT) = (1, 1, 1, 0), or entry e of the table when use
 template <class Tab>
-DEV cached ed_entry_or_identity(const Tab& tab, u32 e, bool neg, bool use) {
-  cached c = neg_cached_if(neg, tab.load(e));
-  if (!use) {
-    const fe one = fe_from_const(Fe::ONE);
-    c.ypx = one;
-    c.ymx = one;
-    c.z = one;
-    c.t2d = fe_zero();
-  }
-  return c;
+DEV scached ed_entry_or_identity(const Tab& tab, u32 e, bool neg, bool use) {
+  const scached c = s_entry(tab.load(e), neg);
+  const u32 m = lane_mask(use);
+  const sfe one = s_from(fe_from_const(Fe::ONE));
+  return scached{s_sel(m, c.ypx, one), s_sel(m, c.ymx, one), s_sel(m, c.z, one), s_sel(m, c.t2d, s_from(fe_zero()))};
 }
 
-// the 136-bit check: [v0](+-B) + [v1](+-[2^136]B) + [a](+-(-A)) + [c1](-R) (- the +-(-A) that made
-// an even |c0| odd) == identity. Carriers of 5 words; tab entries 0..7 hold -A's odd multiples,
-// 8..15 -R's. Per 4-bit window: four doublings and the A and R digits; per 8-bit window also the
-// two B digits.
-template <class Tab, class BTab>
-DEV bool ed_check_lattice(const u32 ca[5], bool a_neg, bool a_fix, const u32 cr[5], const u32 cb0[5], bool b0_neg,
-                          const u32 cb1[5], bool b1_neg, const Tab& tab, const BTab& bt) {
+// the wide table's entry (ed_comb): (y + x)/2, (y - x)/2, dxy as 8 little-endian words each,
+// canonical Montgomery form
+struct ed_comb_entry {
+  u32 v[24];
+};
+
+// acc + [v]B from the wide table: the 16 digits of the carrier c of an odd v (b_neg: negated). Comb:
+// load(i, j, entry&) for the odd multiple (2j + 1) 2^(16 i) B.
+template <class Comb>
+DEV sext ed_comb(sext acc, const u32 c[8], bool b_neg, const Comb& comb) {
+  auto digit = [&](int i) { return (c[i >> 1] >> ((i & 1) * 16)) & 0xFFFFu; };
+  auto load = [&](int i, ed_comb_entry& e) {
+    const u32 d = digit(i);
+    comb.load(i, ((d < COMB_ENTRIES) ? ~d : d) & (COMB_ENTRIES - 1u), e);
+  };
+  ed_comb_entry e;
+  load(0, e);
+#pragma unroll 1
+  for (int i = 0; i < COMB_WINDOWS; i++) {
+    const bool neg = (digit(i) < COMB_ENTRIES) != b_neg;
+    const u32 m = lane_mask(neg);
+    const sfe a = s_from(fe_from_words(e.v)), b = s_from(fe_from_words(e.v + 8)), t = s_from(fe_from_words(e.v + 16));
+    if (i + 1 < COMB_WINDOWS) load(i + 1, e);
+    acc = seadd_half(acc, s_sel(m, b, a), s_sel(m, a, b), s_neg_if(neg, t), i + 1 < COMB_WINDOWS);
+  }
+  return acc;
+}
+
+// the scalars of the lattice-reduced check, as digit carriers of odd values: c0 and c1 (136 bits), and
+// v = c1 s mod l
+struct ed_lat {
+  u32 ca[5], cr[5];
+  u32 v[8];              // v, or l - v when v is even
+  bool a_neg, a_fix;     // c0 is negative; |c0| was even and one was added
+  bool b_neg;            // v was even
+};
+
+// false when k has no short pair (the full-length check then decides)
+DEV bool ed_lat_scalars(const u32 k[8], const u32 s[8], ed_lat& o) {
+  u32 c0[5], c1[5];
+  o.a_neg = false;
+  const bool ok = ed_lattice(k, c0, c1, o.a_neg);
+  u32 cw[8], t[8];
+#pragma unroll
+  for (int i = 0; i < 8; i++) cw[i] = i < 5 ? c1[i] : 0u;
+  fe_to_words(fcanon<Fl>(to_mont<Fl>(mont_mul<Fl>(fe_from_words(cw), fe_from_words(s)))), o.v);
+  o.b_neg = (o.v[0] & 1u) == 0;
+  words_sub(ED_L32, o.v, t);
+#pragma unroll
+  for (int i = 0; i < 8; i++) o.v[i] = o.b_neg ? t[i] : o.v[i];
+  o.a_fix = (c0[0] & 1u) == 0;
+  c0[0] |= 1u;
+  glv_carrier<ED_LAT_BITS>(c0, o.ca);
+  glv_carrier<ED_LAT_BITS>(c1, o.cr);
+  return ok;
+}
+// carrier of the odd v < 2^253 over 256 bits, for ed_comb
+DEV void ed_v_carrier(const u32 v[8], u32 c[8]) {
+#pragma unroll
+  for (int i = 0; i < 8; i++) c[i] = (v[i] >> 1) | (i < 7 ? v[i + 1] << 31 : 0x80000000u);
+}
+
+// One 136-bit chain: [c0](-A) + [c1](-R), the A digits at tab's entries 0..7 and the R digits at 8..15,
+// four doublings and one addition of each per 4-bit window; add_b(acc, i) adds what belongs to an
+// even window i (the B digits of the 8-bit tables, or nothing).
+template <class Tab, class AddB>
+DEV sext ed_lat_ladder(const ed_lat& o, const Tab& tab, const AddB& add_b) {
   constexpr int W = ED_LAT_BITS / 4;
   // top windows: the digits are positive; the A stream's sign applies
-  ext acc = eadd_cached(ext_identity(), neg_cached_if(a_neg, tab.load(nibble(ca, W - 1) - 8)), true);
-  acc = eadd_cached(acc, tab.load(8 + nibble(cr, W - 1) - 8), false);
+  sext acc = seadd(sext_identity(), s_entry(tab.load(nibble(o.ca, W - 1) - 8), o.a_neg), true);
+  acc = seadd(acc, s_entry(tab.load(8 + nibble(o.cr, W - 1) - 8), false), false);
 #pragma unroll 1
   for (int i = W - 2; i >= 0; i--) {
-    const u32 da = nibble(ca, i), dr = nibble(cr, i);
-    cached ea = tab.load((da < 8 ? ~da : da) & 7u);
-    acc = edbl(acc, false);
-    acc = edbl(acc, false);
-    acc = edbl(acc, false);
-    acc = edbl(acc, true);
-    cached er = tab.load(8 + ((dr < 8 ? ~dr : dr) & 7u));
-    acc = eadd_cached(acc, neg_cached_if((da < 8) != a_neg, ea), true);
-    acc = eadd_cached(acc, neg_cached_if(dr < 8, er), (i & 1) == 0);
-    if ((i & 1) == 0) {
-      acc = ed_add_b(acc, bt, 0, byte8(cb0, i >> 1), b0_neg, true);
-      acc = ed_add_b(acc, bt, ED_BTAB_HI, byte8(cb1, i >> 1), b1_neg, i == 0);
-    }
+    const u32 da = nibble(o.ca, i), dr = nibble(o.cr, i);
+    const cached ea = tab.load((da < 8 ? ~da : da) & 7u);
+#pragma unroll 1
+    for (int d = 0; d < 4; d++) acc = sedbl(acc, d == 3);  // T is needed only by an addition that follows
+    const cached er = tab.load(8 + ((dr < 8 ? ~dr : dr) & 7u));
+    acc = seadd(acc, s_entry(ea, (da < 8) != o.a_neg), true);
+    acc = add_b(seadd(acc, s_entry(er, dr < 8), (i & 1) == 0), i);
   }
+  return acc;
+}
+
+// X == 0 and Y == Z
+DEV bool s_is_identity(const sext& P) {
+  return fis_zero<Fe>(s_to_fe<Fe, 8>(P.X)) && fis_zero<Fe>(s_to_fe<Fe, 8>(s_carry(s_sub(P.Y, P.Z))));
+}
+
+// the 136-bit check with 8-bit windows of B: [v0](+-B) + [v1](+-[2^136]B) + [a](+-(-A)) + [c1](-R) (-
+// the +-(-A) that made an even |c0| odd) == identity
+template <class Tab, class BTab>
+DEV bool ed_check_lattice(const ed_lat& o, const Tab& tab, const BTab& bt) {
+  // v split at bit 136; an even high half takes one more: v = (v_lo - 2^136) + 2^136 (v_hi + 1), the
+  // low stream then negated
+  const u32(&v)[8] = o.v;
+  u32 lo[5] = {v[0], v[1], v[2], v[3], v[4] & 0xffu};
+  u32 hi[5] = {(v[4] >> 8) | (v[5] << 24), (v[5] >> 8) | (v[6] << 24), (v[6] >> 8) | (v[7] << 24), v[7] >> 8, 0u};
+  const bool hi_even = (hi[0] & 1u) == 0;
+  hi[0] |= 1u;
+  const u32 top[5] = {0, 0, 0, 0, 1u << (ED_LAT_BITS - 128)};
+  u32 t[5], br = 0;
+#pragma unroll
+  for (int i = 0; i < 5; i++) {
+    const u64 d = (u64)top[i] - lo[i] - br;
+    t[i] = (u32)d;
+    br = (u32)(d >> 63);
+  }
+#pragma unroll
+  for (int i = 0; i < 5; i++) lo[i] = hi_even ? t[i] : lo[i];
+  u32 cb0[5], cb1[5];
+  glv_carrier<ED_LAT_BITS>(lo, cb0);
+  glv_carrier<ED_LAT_BITS>(hi, cb1);
+  const bool b0_neg = o.b_neg != hi_even, b1_neg = o.b_neg;
+  sext acc = ed_lat_ladder(o, tab, [&](const sext& a, int i) {
+    if (i & 1) return a;
+    const sext b = ed_add_b(a, bt, 0, byte8(cb0, i >> 1), b0_neg, true);
+    return ed_add_b(b, bt, ED_BTAB_HI, byte8(cb1, i >> 1), b1_neg, i == 0);
+  });
   // the A stream ran on |c0| + 1 when |c0| was even: take its point off once
-  acc = eadd_cached(acc, ed_entry_or_identity(tab, 0, !a_neg, a_fix), false);
-  return fis_zero<Fe>(acc.X) && feq<Fe>(acc.Y, acc.Z);
+  return s_is_identity(seadd(acc, ed_entry_or_identity(tab, 0, !o.a_neg, o.a_fix), false));
+}
+
+// the same with [v]B from the wide table
+template <class Tab, class Comb>
+DEV bool ed_check_lattice_wide(const ed_lat& o, const Tab& tab, const Comb& comb) {
+  u32 c[8];
+  ed_v_carrier(o.v, c);
+  sext acc = ed_lat_ladder(o, tab, [](const sext& a, int) { return a; });
+  acc = seadd(acc, ed_entry_or_identity(tab, 0, !o.a_neg, o.a_fix), true);
+  return s_is_identity(ed_comb(acc, c, o.b_neg, comb));
 }
 
 // the full-length check: compress([s]B + [k](-A)) == R bytes, tab entries 0..7 = -A's odd multiples
@@ -468,33 +622,24 @@ DEV bool ed_check_full(const u32 s[8], const u32 k[8], const u32 sig_raw[16], co
     }
   }
   u32 c1[8], c2[8];
-#pragma unroll
-  for (int i = 0; i < 8; i++) {
-    c1[i] = (s1[i] >> 1) | (i < 7 ? s1[i + 1] << 31 : 0x80000000u);
-    c2[i] = (k1[i] >> 1) | (i < 7 ? k1[i + 1] << 31 : 0x80000000u);
-  }
-  ext acc = eadd_cached(ext_identity(), tab.load(nibble(c2, 63) - 8), true);
+  ed_v_carrier(s1, c1);
+  ed_v_carrier(k1, c2);
+  sext acc = seadd(sext_identity(), s_entry(tab.load(nibble(c2, 63) - 8), false), true);
 #pragma unroll 1
   for (int i = 62; i >= 0; i--) {
-    // issue the HBM load of this window's table entry before the doublings, which hide its latency
     const u32 c = nibble(c2, i);
-    const bool neg = c < 8;
-    cached E = tab.load((neg ? ~c : c) & 7u);
-    acc = edbl(acc, false);
-    acc = edbl(acc, false);
-    acc = edbl(acc, false);
-    acc = edbl(acc, true);
-    E = neg_cached_if(neg, E);
-    // T is needed only by a following addition: doublings do not read it (uniform branches)
-    acc = eadd_cached(acc, E, (i & 1) == 0);
+    const cached E = tab.load((c < 8 ? ~c : c) & 7u);
+#pragma unroll 1
+    for (int d = 0; d < 4; d++) acc = sedbl(acc, d == 3);
+    acc = seadd(acc, s_entry(E, c < 8), (i & 1) == 0);
     if ((i & 1) == 0) acc = ed_add_b(acc, bt, 0, byte8(c1, i >> 1), b_neg, i == 0);
   }
   // + A when k was made odd by adding one, else + identity (complete formulas)
-  acc = eadd_cached(acc, ed_entry_or_identity(tab, 0, true, k_even), false);
+  acc = seadd(acc, ed_entry_or_identity(tab, 0, true, k_even), false);
   // compress and compare with R
-  const fe zi = finv<Fe>(acc.Z);
-  const fe xa = from_mont<Fe>(mont_mul<Fe>(acc.X, zi));
-  const fe ya = from_mont<Fe>(mont_mul<Fe>(acc.Y, zi));
+  const fe zi = finv<Fe>(s_to_fe<Fe, 8>(acc.Z));
+  const fe xa = from_mont<Fe>(mont_mul<Fe>(s_to_fe<Fe, 8>(acc.X), zi));
+  const fe ya = from_mont<Fe>(mont_mul<Fe>(s_to_fe<Fe, 8>(acc.Y), zi));
   u32 enc[8];
   fe_to_words(ya, enc);
   enc[7] ^= (xa.v[0] & 1u) << 31;
@@ -504,19 +649,13 @@ DEV bool ed_check_full(const u32 s[8], const u32 k[8], const u32 sig_raw[16], co
   return diff == 0;
 }
 
-// verification given the challenge k (from ed25519_challenge).
-// LATTICE: the lattice-reduced check (and the full-length one for challenges without a short
-// pair); otherwise the full-length check only. Measured on the MI355X: 3.5% faster in the kernels
-// that verify only Ed25519, 2.5% slower in the mixed-scheme kernel, whose secp paths share its
-// registers and code.
-// BTab: load(idx, ypx, ymx, t2d) for (2 idx + 1) B at idx < ED_BTAB_HI and, with LATTICE,
-// (2 j + 1) [2^136] B at idx = ED_BTAB_HI + j. Tab: per-lane store(e, cached) / load(e), 8 entries
-// (16 with LATTICE).
+// Verification given the challenge k (from ed25519_challenge). lattice(k, s, tab): the lattice-reduced
+// check on tab's entries 0..7 (-A) and 8..15 (-R), or false in `found` when k has no short pair.
 // STRICT: dalek VerifyingKey::verify_strict; the status of its rules on R arrives in the top bits
 // of k (ed25519_strict_r_checks) and A's small order is checked here.
-template <bool STRICT = false, bool LATTICE = false, class Tab, class BTab>
-DEV u32 ed25519_verify_core(const u32 sig_raw[16], const u32 pk_raw[8], const u32 k_in[8], Tab& tab,
-                            const BTab& bt) {
+template <bool STRICT, class Tab, class BTab, class Lattice>
+DEV u32 ed25519_verify_with(const u32 sig_raw[16], const u32 pk_raw[8], const u32 k_in[8], Tab& tab, const BTab& bt,
+                            const Lattice& lattice) {
   u32 k[8];
 #pragma unroll
   for (int i = 0; i < 8; i++) k[i] = k_in[i];
@@ -538,68 +677,69 @@ DEV u32 ed25519_verify_core(const u32 sig_raw[16], const u32 pk_raw[8], const u3
   // verify_strict: A of small order (checked after R's rules, as dalek checks R first)
   if (STRICT && status == ED_OK && ed_small_order(x, y)) status = ED_SMALL_ORDER;
   ed_table_odd(tab, 0, fneg<Fe>(x), y);
-  u32 c0[5], c1[5];
-  bool c0_neg = false;
-  bool equal;
-  if (LATTICE && ed_lattice(k, c0, c1, c0_neg)) {
-    fe rx, ry;
-    const bool r_ok = ed_decode_canonical(sig_raw, rx, ry);
-    ed_table_odd(tab, 8, fneg<Fe>(rx), ry);
-    // v = c1 s mod l, made odd (l - v with B negated), split at bit 136; an even high half takes
-    // one more: v = (v_lo - 2^136) + 2^136 (v_hi + 1), the low stream then negated
-    u32 v[8];
-    {
-      u32 cw[8];
-#pragma unroll
-      for (int i = 0; i < 8; i++) cw[i] = i < 5 ? c1[i] : 0u;
-      fe_to_words(fcanon<Fl>(to_mont<Fl>(mont_mul<Fl>(fe_from_words(cw), fe_from_words(s)))), v);
-    }
-    const bool b_neg = (v[0] & 1u) == 0;
-    {
-      u32 t[8];
-      words_sub(ED_L32, v, t);
-#pragma unroll
-      for (int i = 0; i < 8; i++) v[i] = b_neg ? t[i] : v[i];
-    }
-    u32 lo[5] = {v[0], v[1], v[2], v[3], v[4] & 0xffu};
-    u32 hi[5] = {(v[4] >> 8) | (v[5] << 24), (v[5] >> 8) | (v[6] << 24), (v[6] >> 8) | (v[7] << 24), v[7] >> 8, 0u};
-    const bool hi_even = (hi[0] & 1u) == 0;
-    hi[0] |= 1u;
-    {
-      const u32 top[5] = {0, 0, 0, 0, 1u << (ED_LAT_BITS - 128)};
-      u32 t[5];
-      u32 br = 0;
-#pragma unroll
-      for (int i = 0; i < 5; i++) {
-        const u64 d = (u64)top[i] - lo[i] - br;
-        t[i] = (u32)d;
-        br = (u32)(d >> 63);
-      }
-#pragma unroll
-      for (int i = 0; i < 5; i++) lo[i] = hi_even ? t[i] : lo[i];
-    }
-    const bool a_fix = (c0[0] & 1u) == 0;
-    c0[0] |= 1u;
-    u32 ca[5], cr[5], cb0[5], cb1[5];
-    glv_carrier<ED_LAT_BITS>(c0, ca);
-    glv_carrier<ED_LAT_BITS>(c1, cr);
-    glv_carrier<ED_LAT_BITS>(lo, cb0);
-    glv_carrier<ED_LAT_BITS>(hi, cb1);
-    equal = ed_check_lattice(ca, c0_neg, a_fix, cr, cb0, b_neg != hi_even, cb1, b_neg, tab, bt) && r_ok;
-  } else {
-    equal = ed_check_full(s, k, sig_raw, tab, bt);
-  }
+  bool found = false;
+  bool equal = lattice(k, s, found);
+  if (!found) equal = ed_check_full(s, k, sig_raw, tab, bt);
   if (status == ED_OK && !equal) status = ED_MISMATCH;
   return status;
+}
+
+// R decoded and its table built, then `check` on the scalars
+template <class Tab, class Check>
+DEV bool ed_with_lattice(const u32 sig_raw[16], const u32 k[8], const u32 s[8], Tab& tab, bool& found,
+                         const Check& check) {
+  ed_lat o;
+  found = ed_lat_scalars(k, s, o);
+  if (!found) return false;
+  fe rx, ry;
+  const bool r_ok = ed_decode_canonical(sig_raw, rx, ry);
+  ed_table_odd(tab, 8, fneg<Fe>(rx), ry);
+  return check(o) && r_ok;
+}
+
+// the same with the resident or a caller's 8-bit table of B.
+// LATTICE: the lattice-reduced check (and the full-length one for challenges without a short
+// pair); otherwise the full-length check only.
+// BTab: load(idx, ypx, ymx, t2d) for (2 idx + 1) B at idx < ED_BTAB_HI and, with LATTICE,
+// (2 j + 1) [2^136] B at idx = ED_BTAB_HI + j. Tab: per-lane store(e, cached) / load(e), 8 entries
+// (16 with LATTICE).
+template <bool STRICT = false, bool LATTICE = false, class Tab, class BTab>
+DEV u32 ed25519_verify_core(const u32 sig_raw[16], const u32 pk_raw[8], const u32 k_in[8], Tab& tab,
+                            const BTab& bt) {
+  return ed25519_verify_with<STRICT>(sig_raw, pk_raw, k_in, tab, bt, [&](const u32* k, const u32* s, bool& found) {
+    if constexpr (LATTICE)
+      return ed_with_lattice(sig_raw, k, s, tab, found, [&](const ed_lat& o) { return ed_check_lattice(o, tab, bt); });
+    else
+      return false;
+  });
+}
+
+// the challenge, with the status of verify_strict's rules on R in its top bits
+template <bool STRICT, class Mem>
+DEV void ed25519_challenge_strict(const u32 sig_raw[16], const u32 pk_raw[8], const Mem& mem, u64 msg_off, u32 len,
+                                  u32 k[8]) {
+  ed25519_challenge(sig_raw, pk_raw, mem, msg_off, len, k);
+  if constexpr (STRICT) k[7] |= ed25519_strict_r_checks(sig_raw) << ED_K_STRICT_SHIFT;
 }
 
 template <bool STRICT = false, bool LATTICE = false, class Tab, class BTab, class Mem>
 DEV u32 ed25519_verify_item(const u32 sig_raw[16], const u32 pk_raw[8], const Mem& mem, u64 msg_off, u32 len,
                             Tab& tab, const BTab& bt) {
   u32 k[8];
-  ed25519_challenge(sig_raw, pk_raw, mem, msg_off, len, k);
-  if constexpr (STRICT) k[7] |= ed25519_strict_r_checks(sig_raw) << ED_K_STRICT_SHIFT;
+  ed25519_challenge_strict<STRICT>(sig_raw, pk_raw, mem, msg_off, len, k);
   return ed25519_verify_core<STRICT, LATTICE>(sig_raw, pk_raw, k, tab, bt);
+}
+
+// the lattice-reduced check with the wide table of B; bt: the 8-bit table, for the full-length check
+template <bool STRICT, class Tab, class BTab, class Comb, class Mem>
+DEV u32 ed25519_verify_wide(const u32 sig_raw[16], const u32 pk_raw[8], const Mem& mem, u64 msg_off, u32 len,
+                            Tab& tab, const BTab& bt, const Comb& comb) {
+  u32 k8[8];
+  ed25519_challenge_strict<STRICT>(sig_raw, pk_raw, mem, msg_off, len, k8);
+  return ed25519_verify_with<STRICT>(sig_raw, pk_raw, k8, tab, bt, [&](const u32* k, const u32* s, bool& found) {
+    return ed_with_lattice(sig_raw, k, s, tab, found,
+                           [&](const ed_lat& o) { return ed_check_lattice_wide(o, tab, comb); });
+  });
 }
 
 }  // namespace sigops

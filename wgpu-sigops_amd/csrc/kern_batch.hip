@@ -14,9 +14,12 @@
 //   5. k_batch_careful finishes secp items whose fast ladder met an exceptional addition.
 // The batch's buffers and n are read from device memory (BatchIO), so the captured graph of these
 // launches replays for any buffers and any n up to the context capacity.
-#include "kernels_impl.hpp"
+#include "kern_quad.hpp"
 
 namespace sigops {
+
+static_assert(BATCH_QUAD_LANES == BATCH_QUAD_BLOCKS * 64 && BATCH_QUAD_TILE == QUAD_ITEMS,
+              "kernels.hpp's launch shape of a small batch");
 
 constexpr u32 DUMMY = 0xFFFFFFFFu;
 
@@ -33,6 +36,7 @@ struct BatchArgs {
   u32* counts;      // [NB]
   u32* cursor;      // [NB]
   u32* tile_start;  // [NB + 1] in processing order
+  u32* bucket_of;   // [NB] processing rank -> bucket
   u32* order;       // padded item lists, bucket-major in processing order
   u32* tile_counter;
   u32* pend_list;
@@ -86,31 +90,74 @@ __global__ __launch_bounds__(256) void k_bucket_hist(BatchArgs a) {
     if (h[t]) atomicAdd(&a.counts[t], h[t]);
 }
 
-// one block: tile offsets in processing order, cursors, and DUMMY padding of each bucket's tail
+// By one wavefront (the block's first): tile offsets in processing order from the buckets' counts c
+// (LDS), DUMMY padding of each bucket's last tile, and each bucket's first position (start, LDS).
+// One thread walking the ranks took 29 us, longer than the sort's other passes.
+DEV void bucket_scan(const BatchArgs& a, const u32* c, u32* start, u32* bucket_of) {
+  static_assert(NBUCKETS <= 64, "one lane per bucket");
+  const u32 lane = threadIdx.x;
+  if (lane < 64) {
+    if (lane < NBUCKETS) bucket_of[a.rank[lane]] = lane;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const u32 b = lane < NBUCKETS ? bucket_of[lane] : 0;
+    const u32 tiles = lane < NBUCKETS ? (c[b] + a.tile_items - 1) / a.tile_items : 0;
+    u32 end = tiles;  // inclusive prefix sum over the ranks
+#pragma unroll
+    for (u32 d = 1; d < 64; d <<= 1) {
+      const u32 v = __shfl_up(end, d);
+      if (lane >= d) end += v;
+    }
+    if (lane < NBUCKETS) {
+      a.tile_start[lane] = end - tiles;
+      if (lane == NBUCKETS - 1) a.tile_start[NBUCKETS] = end;
+      start[b] = (end - tiles) * a.tile_items;
+      a.bucket_of[lane] = b;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    for (u32 q = 0; q < NBUCKETS; q++) {
+      const u32 padded = (c[q] + a.tile_items - 1) / a.tile_items * a.tile_items;
+      for (u32 k = c[q] + lane; k < padded; k += 64) a.order[start[q] + k] = DUMMY;
+    }
+  }
+}
+
 __global__ __launch_bounds__(64) void k_bucket_scan(BatchArgs a) {
   bind_io(a);
-  __shared__ u32 start[NBUCKETS];
-  if (threadIdx.x == 0) {
-    u32 pos_tiles = 0;
-    for (u32 r = 0; r < NBUCKETS; r++) {
-      u32 b = 0;
-      for (u32 q = 0; q < NBUCKETS; q++)
-        if (a.rank[q] == r) b = q;
-      const u32 c = a.counts[b];
-      const u32 tiles = (c + a.tile_items - 1) / a.tile_items;
-      a.tile_start[r] = pos_tiles;
-      start[b] = pos_tiles * a.tile_items;
-      pos_tiles += tiles;
-    }
-    a.tile_start[NBUCKETS] = pos_tiles;
+  __shared__ u32 c[NBUCKETS], start[NBUCKETS], bucket_of[NBUCKETS];
+  if (threadIdx.x < NBUCKETS) c[threadIdx.x] = a.counts[threadIdx.x];
+  __syncthreads();
+  bucket_scan(a, c, start, bucket_of);
+  if (threadIdx.x < NBUCKETS) a.cursor[threadIdx.x] = start[threadIdx.x];
+}
+
+// the whole bucketing of a small batch in one workgroup (clear, histogram, scan, scatter: four
+// launches otherwise)
+__global__ __launch_bounds__(1024) void k_bucket_small(BatchArgs a) {
+  bind_io(a);
+  __shared__ u32 c[NBUCKETS], start[NBUCKETS], bucket_of[NBUCKETS];
+  if (threadIdx.x < NBUCKETS) c[threadIdx.x] = 0;
+  if (threadIdx.x == 0) *a.pend_count = 0;
+  __syncthreads();
+  const u32 n = a.n;
+  for (u32 i = threadIdx.x; i < n; i += blockDim.x) {
+    if (item_scheme(a, i) > 2)
+      a.status[i] = 0xFD;  // unknown scheme: reported as a canary failure by the host
+    else
+      atomicAdd(&c[item_bucket(a, i)], 1u);
   }
   __syncthreads();
-  for (u32 b = 0; b < NBUCKETS; b++) {
-    const u32 c = a.counts[b];
-    const u32 padded = (c + a.tile_items - 1) / a.tile_items * a.tile_items;
-    for (u32 q = c + threadIdx.x; q < padded; q += blockDim.x) a.order[start[b] + q] = DUMMY;
-    if (threadIdx.x == 0) a.cursor[b] = start[b];
-  }
+  bucket_scan(a, c, start, bucket_of);
+  __syncthreads();
+  for (u32 i = threadIdx.x; i < n; i += blockDim.x)
+    if (item_scheme(a, i) <= 2) a.order[atomicAdd(&start[item_bucket(a, i)], 1u)] = i;
+}
+
+// the bucket of tile t, the same on every lane of the wavefront
+DEV u32 tile_bucket(const BatchArgs& a, u32 t) {
+  const u32 lane = threadIdx.x & 63u;
+  const bool here = lane < NBUCKETS && a.tile_start[lane] <= t && t < a.tile_start[lane + 1];
+  const u64 m = __ballot(here);
+  return __builtin_amdgcn_readfirstlane(a.bucket_of[__ffsll((unsigned long long)m) - 1]);
 }
 
 // Each workgroup ranks its chunk of 1024 items (4 per thread) per bucket with LDS atomics,
@@ -210,9 +257,10 @@ __global__ __launch_bounds__(256, SIGOPS_WAVES_PER_EU) void k_batch_finish(Batch
 }
 
 // The schemes a persistent launch serves (template mask): the mixed batch serves all three; the
-// plain Ed25519 entry points serve only Ed25519 (dalek `verify`, or `verify_strict` rules), so
-// they run the same tile loop, with the challenge hashed inside it, and stage only B's table.
-constexpr u32 RUN_K1 = 1, RUN_R1 = 2, RUN_ED = 4, RUN_ED_STRICT = 8;
+// plain Ed25519 entry points serve only Ed25519 (dalek `verify`, or `verify_strict` rules, or `verify`
+// with a caller's table of B staged in LDS), so they run the same tile loop, with the challenge
+// hashed inside it.
+constexpr u32 RUN_K1 = 1, RUN_R1 = 2, RUN_ED = 4, RUN_ED_STRICT = 8, RUN_ED_TABLE = 16;
 constexpr u32 RUN_MIXED = RUN_K1 | RUN_R1 | RUN_ED;
 
 // WAVES: waves per SIMD the kernel is built for, which sets its register budget per lane (512 /
@@ -221,18 +269,17 @@ constexpr u32 RUN_MIXED = RUN_K1 | RUN_R1 | RUN_ED;
 // latencies. The autotuner measures them.
 template <u32 MASK, int WAVES = SIGOPS_WAVES_PER_EU>
 __global__ __launch_bounds__(256, WAVES) void k_batch_run(BatchArgs a, const uint4* __restrict__ comb_k1,
-                                                   const uint4* __restrict__ comb_r1, const uint4* __restrict__ gb,
+                                                   const uint4* __restrict__ comb_r1,
+                                                   const uint4* __restrict__ comb_ed, const uint4* __restrict__ gb,
                                                    uint4* __restrict__ lane_tab, u32 slots) {
-  static_assert(!((MASK & RUN_ED) && (MASK & RUN_ED_STRICT)), "one Ed25519 rule set per launch");
-  constexpr bool K1 = MASK & RUN_K1, R1 = MASK & RUN_R1, ED = MASK & (RUN_ED | RUN_ED_STRICT);
-  // the kernels that serve only Ed25519 run the lattice-reduced check (both fixed-base tables)
-  constexpr bool LAT = ED && !K1 && !R1;
-  constexpr u32 BN = LAT ? BTAB_UINT4 : BTAB_ENTRIES * 7;
+  constexpr bool K1 = MASK & RUN_K1, R1 = MASK & RUN_R1, TABLE = MASK & RUN_ED_TABLE;
+  constexpr bool ED = MASK & (RUN_ED | RUN_ED_STRICT | RUN_ED_TABLE);
   bind_io(a);
-  __shared__ uint4 s_b[ED ? BN : 1];
-  if constexpr (ED)
-    for (int t = threadIdx.x; t < BN; t += blockDim.x) s_b[t] = gb[t];
-  __syncthreads();
+  __shared__ uint4 s_b[TABLE ? BTAB_UINT4 : 1];
+  if constexpr (TABLE) {
+    for (int t = threadIdx.x; t < BTAB_UINT4; t += blockDim.x) s_b[t] = gb[t];
+    __syncthreads();
+  }
   const u32 slot = blockIdx.x * blockDim.x + threadIdx.x;
   const u32 lane = threadIdx.x & 63u;
   STabDev jt;
@@ -249,12 +296,7 @@ __global__ __launch_bounds__(256, WAVES) void k_batch_run(BatchArgs a, const uin
     if (lane == 0) t = atomicAdd(a.tile_counter, 1u);
     t = __shfl(t, 0);
     if (t >= ntiles) break;
-    u32 r = 0;
-    while (r + 1 < NBUCKETS && a.tile_start[r + 1] <= t) r++;
-    u32 b = 0;
-    for (u32 q = 0; q < NBUCKETS; q++)
-      if (a.rank[q] == r) b = q;
-    b = __builtin_amdgcn_readfirstlane(b);
+    const u32 b = tile_bucket(a, t);
     for (u32 k = 0; k < a.tile_items; k += 64) {
       const u32 pos = t * a.tile_items + k + lane;
       const u32 i = a.order[pos];
@@ -271,8 +313,12 @@ __global__ __launch_bounds__(256, WAVES) void k_batch_run(BatchArgs a, const uin
         load_words(a.sigs + 4 * (u64)i, sr, 4);
         load_words(a.aux + 2 * (u64)i, pr, 2);
         const u64 off = a.msg_off[i];
-        a.status[i] = (u8)ed25519_verify_item<(MASK & RUN_ED_STRICT) != 0, LAT>(
-            sr, pr, MemDev{a.msgs}, off, (u32)(a.msg_off[i + 1] - off), ct, BTabLds{s_b});
+        const u32 len = (u32)(a.msg_off[i + 1] - off);
+        if constexpr (TABLE)
+          a.status[i] = (u8)ed25519_verify_item<false, true>(sr, pr, MemDev{a.msgs}, off, len, ct, BTabLds{s_b});
+        else
+          a.status[i] = (u8)ed25519_verify_wide<(MASK & RUN_ED_STRICT) != 0>(sr, pr, MemDev{a.msgs}, off, len, ct,
+                                                                            BTabGlobal{gb}, EdCombDev{comb_ed});
         if (a.out) {
           const u32 zero[16] = {0};
           store16(a.out + 4 * (u64)i, zero);
@@ -280,6 +326,41 @@ __global__ __launch_bounds__(256, WAVES) void k_batch_run(BatchArgs a, const uin
       }
     }
   }
+}
+
+// A small mixed batch: one workgroup per tile of 16 items, four lanes per item (kern_quad.hpp). The
+// grid is that of the largest such batch; workgroups beyond the tiles end at once.
+__global__ __launch_bounds__(QUAD_THREADS, 2) void k_batch_quad(BatchArgs a, const uint4* __restrict__ comb_k1,
+                                                            const uint4* __restrict__ comb_r1,
+                                                            const uint4* __restrict__ comb_ed,
+                                                            const uint4* __restrict__ gb,
+                                                            uint4* __restrict__ lane_tab, u32 slots,
+                                                            u32* __restrict__ load) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  bind_io(a);
+  __shared__ QuadShared sh;
+  const u32 t = blockIdx.x;
+  if (t >= a.tile_start[NBUCKETS]) return;
+  const QuadRole role(load, sh.role);
+  const u32 b = tile_bucket(a, t);
+  const u32 i = a.order[t * QUAD_ITEMS + quad_item()];
+  const bool valid = i != DUMMY;
+  const auto pend = [&](u32 p) { a.pend_list[atomicAdd(a.pend_count, 1u)] = p; };
+  if (b == BUCKET_K1) {
+    quad_secp_tile<CurveK1, false>(sh, role.points, valid, i, a.sigs, a.aux, nullptr, a.out, a.status, comb_k1, pend);
+  } else if (b == BUCKET_R1) {
+    quad_secp_tile<CurveR1, false>(sh, role.points, valid, i, a.sigs, a.aux, nullptr, a.out, a.status, comb_r1, pend);
+  } else {
+    if (valid && role.points) a.out[4 * (u64)i + q_lane()] = make_uint4(0, 0, 0, 0);
+    CTabDev ct;
+    ct.base = lane_tab;
+    ct.slots = slots;
+    ct.slot = blockIdx.x * 64 + (threadIdx.x & 63u);  // the point wave's lanes
+    quad_ed_tile<false>(sh, role.points, valid, i, a.sigs, a.aux, a.msgs, a.msg_off, a.status, comb_ed, ct,
+                        BTabGlobal{gb});
+  }
+  role.done();
+#endif
 }
 
 __global__ __launch_bounds__(64) void k_batch_careful(BatchArgs a, const uint4* __restrict__ gk1,
@@ -330,6 +411,7 @@ static BatchArgs batch_args(const BatchLaunch& L) {
   a.tile_start = L.work + 2 * NBUCKETS;  // NBUCKETS + 1
   a.tile_counter = L.work + 3 * NBUCKETS + 1;
   a.pend_count = L.work + 3 * NBUCKETS + 2;
+  a.bucket_of = L.work + 3 * NBUCKETS + 3;
   a.pend_list = L.pend_list;
   a.order = L.order;
   a.rank = L.rank;
@@ -347,11 +429,28 @@ hipError_t launch_ed_verify(const BatchLaunch& L, bool strict, hipStream_t s) {
   k_bucket_hist<<<L.aux_grid, 256, 0, s>>>(a);
   k_bucket_scan<<<1, 64, 0, s>>>(a);
   k_bucket_scatter<<<L.aux_grid, 256, 0, s>>>(a);
-  if (strict)
-    k_batch_run<RUN_ED_STRICT><<<L.grid, 256, 0, s>>>(a, nullptr, nullptr, (const uint4*)L.gb, (uint4*)L.lane_tab,
-                                                      L.slots);
-  else
-    k_batch_run<RUN_ED><<<L.grid, 256, 0, s>>>(a, nullptr, nullptr, (const uint4*)L.gb, (uint4*)L.lane_tab, L.slots);
+  const auto run = L.caller_gb ? k_batch_run<RUN_ED_TABLE> : (strict ? k_batch_run<RUN_ED_STRICT> : k_batch_run<RUN_ED>);
+  run<<<L.grid, 256, 0, s>>>(a, nullptr, nullptr, (const uint4*)L.comb_ed,
+                             (const uint4*)(L.caller_gb ? L.caller_gb : L.gb), (uint4*)L.lane_tab, L.slots);
+  return hipGetLastError();
+}
+
+// a batch of at most BATCH_QUAD_MAX_ITEMS items; L.lane_tab holds at least
+// BATCH_QUAD_LANES lanes
+hipError_t launch_batch_small(const BatchLaunch& L, hipStream_t s) {
+  BatchArgs a = batch_args(L);
+  a.tile_items = QUAD_ITEMS;
+  auto mark = [&](int i) -> hipError_t { return L.stage_ev ? hipEventRecord(L.stage_ev[i], s) : hipSuccess; };
+  hipError_t e;
+  if ((e = mark(0)) != hipSuccess) return e;
+  k_bucket_small<<<1, 1024, 0, s>>>(a);
+  if ((e = mark(1)) != hipSuccess || (e = mark(2)) != hipSuccess) return e;
+  k_batch_quad<<<BATCH_QUAD_BLOCKS, QUAD_THREADS, 0, s>>>(a, (const uint4*)L.comb_k1, (const uint4*)L.comb_r1,
+                                                          (const uint4*)L.comb_ed, (const uint4*)L.gb,
+                                                          (uint4*)L.lane_tab, L.slots, L.quad_load);
+  if ((e = mark(3)) != hipSuccess) return e;
+  k_batch_careful<<<64, 64, 0, s>>>(a, (const uint4*)L.gk1, (const uint4*)L.gr1);
+  if ((e = mark(4)) != hipSuccess) return e;
   return hipGetLastError();
 }
 
@@ -371,12 +470,9 @@ hipError_t launch_batch(const BatchLaunch& L, hipStream_t s) {
   // stage indices of earlier measurements keep their meaning)
   if ((e = mark(2)) != hipSuccess) return e;
   k_batch_scalars<<<L.stage_grid, 256, 0, s>>>(a);
-  if (L.waves == 1)
-    k_batch_run<RUN_MIXED, 1><<<L.grid, 256, 0, s>>>(a, (const uint4*)L.comb_k1, (const uint4*)L.comb_r1,
-                                                    (const uint4*)L.gb, (uint4*)L.lane_tab, L.slots);
-  else
-    k_batch_run<RUN_MIXED><<<L.grid, 256, 0, s>>>(a, (const uint4*)L.comb_k1, (const uint4*)L.comb_r1,
-                                                 (const uint4*)L.gb, (uint4*)L.lane_tab, L.slots);
+  const auto run = L.waves == 1 ? k_batch_run<RUN_MIXED, 1> : k_batch_run<RUN_MIXED>;
+  run<<<L.grid, 256, 0, s>>>(a, (const uint4*)L.comb_k1, (const uint4*)L.comb_r1, (const uint4*)L.comb_ed,
+                             (const uint4*)L.gb, (uint4*)L.lane_tab, L.slots);
   k_batch_finish<<<L.stage_grid, 256, 0, s>>>(a);
   if ((e = mark(3)) != hipSuccess) return e;
   k_batch_careful<<<64, 64, 0, s>>>(a, (const uint4*)L.gk1, (const uint4*)L.gr1);

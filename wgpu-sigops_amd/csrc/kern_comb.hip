@@ -88,7 +88,7 @@ __global__ __launch_bounds__(256, SIGOPS_WAVES_PER_EU) void k_comb_build(const u
   }
 }
 
-// the same for Ed25519's B, entries (Y + X, Y - X, 2dXY): every formula is complete
+// the same for Ed25519's B, entries ((y + x)/2, (y - x)/2, dxy): every formula is complete
 __global__ __launch_bounds__(256, SIGOPS_WAVES_PER_EU) void k_comb_build_ed(const uint4* __restrict__ btab,
                                                                        uint4* __restrict__ comb,
                                                                        uint4* __restrict__ tmp_base) {
@@ -137,9 +137,11 @@ __global__ __launch_bounds__(256, SIGOPS_WAVES_PER_EU) void k_comb_build_ed(cons
     inv = mont_mul<Fe>(inv, Z);
     const fe x = mont_mul<Fe>(X, zi), y = mont_mul<Fe>(Y, zi);
     u32 o[24];
-    fe_to_words(fcanon<Fe>(fadd<Fe>(y, x)), o);
-    fe_to_words(fcanon<Fe>(fsub<Fe>(y, x)), o + 8);
-    fe_to_words(fcanon<Fe>(mont_mul<Fe>(mont_mul<Fe>(x, y), fe_from_const(ED_D2))), o + 16);
+    fe half = fe_zero();  // 1/2 in Montgomery form: 2^260 = 32 * 2^255 = 608 (mod p)
+    half.v[0] = 608;
+    fe_to_words(fcanon<Fe>(mont_mul<Fe>(fadd<Fe>(y, x), half)), o);
+    fe_to_words(fcanon<Fe>(mont_mul<Fe>(fsub<Fe>(y, x), half)), o + 8);
+    fe_to_words(fcanon<Fe>(mont_mul<Fe>(mont_mul<Fe>(x, y), fe_from_const(ED_D))), o + 16);
     uint4* p = comb + 6 * ((u64)win * COMB_ENTRIES + RUN * r + e);
 #pragma unroll
     for (int c = 0; c < 6; c++) p[c] = make_uint4(o[4 * c], o[4 * c + 1], o[4 * c + 2], o[4 * c + 3]);

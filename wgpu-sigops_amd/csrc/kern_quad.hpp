@@ -1,15 +1,12 @@
 // kern_quad.hpp -- signature items spread over the four lanes of a quad (quad.hpp), 16 items per
 // workgroup of two wavefronts, for calls that would otherwise leave SIMDs idle.
 //
-// The first wavefront (the point wave) lifts the points, builds their tables in LDS and runs the
-// ladder; the second (the scalar wave) meanwhile hashes, inverts, splits and recodes the scalars, and
-// hands the digits over through LDS. The point wave runs several times as long, so no two of them
-// should share a SIMD: a compute unit deals the wavefronts of its workgroups to its SIMDs in the
-// order 0, 2, 1, 3 and starts each workgroup one further on, which puts the first wavefronts of the
-// four workgroups it gets at QUAD_MAX_ITEMS on four different SIMDs (read back from the hardware
-// register; with the roles swapped in every other pair of workgroups, or with four wavefronts per
-// workgroup, two point waves met and 16,384 recoveries took 864 us). Everything an item needs stays in the one kernel: a call of a few
-// thousand items is bound by the length of one item's chain of instructions and by its launches.
+// One wavefront (the point wave) lifts the points, builds their tables in LDS and runs the ladder;
+// the other (the scalar wave) meanwhile hashes, inverts, splits and recodes the scalars, and hands
+// the digits over through LDS. The point wave runs several times as long, so two of them should not
+// share a SIMD while another has none: the workgroup makes its point wave the one on the SIMD with
+// fewer of them (QuadRole). Fixed roles met on SIMDs from some 500 workgroups on, which ones
+// depending on the launch (16,384 recoveries took 864 us instead of 551).
 #pragma once
 #include "kernels_impl.hpp"
 #include "quad.hpp"
@@ -19,14 +16,41 @@ namespace sigops {
 constexpr u32 QUAD_ITEMS = 16;    // items per workgroup
 constexpr u32 QUAD_THREADS = 128;
 
-// the wide Ed25519 table in HBM: entry j of window i, 96 bytes (Y + X, Y - X, 2dXY as 8 words each)
-constexpr u32 ED_COMB_UINT4 = 6;
-
 #if defined(__HIP_DEVICE_COMPILE__)
 
-DEV bool quad_point_wave() { return threadIdx.x < 64; }
 // this lane's item of the workgroup's, the same for the point and the scalar wave
 DEV u32 quad_item() { return (threadIdx.x & 63u) >> 2; }
+
+// The point waves running on every SIMD of the device, counted by the workgroups themselves (load: 4
+// words per compute unit, by the hardware's ids; zero when nothing runs).
+struct QuadRole {
+  u32* mine;    // the counter of this workgroup's point wave
+  bool points;  // whether this wavefront is the point wave
+  DEV static u32 hw_id() { return __builtin_amdgcn_s_getreg(4 | (31 << 11)); }          // HW_ID
+  DEV static u32 xcc_id() { return __builtin_amdgcn_s_getreg(20 | (3 << 11)); }         // XCC_ID, 4 bits
+  DEV QuadRole(u32* load, u32* sh) {  // sh: 3 words of LDS; every thread of the workgroup calls
+    const u32 w = threadIdx.x >> 6, hw = hw_id();
+    if ((threadIdx.x & 63u) == 0) sh[w] = (hw >> 4) & 3u;
+    __syncthreads();
+    u32* cu = load + 4 * ((xcc_id() & 15u) * 256 + ((hw >> 8) & 255u));
+    if (threadIdx.x == 0) {
+      const u32 c0 = atomicAdd(cu + sh[0], 1u);
+      u32 pick = 0;
+      if (c0) {
+        const u32 c1 = atomicAdd(cu + sh[1], 1u);
+        pick = c1 < c0 ? 1u : 0u;
+        atomicSub(cu + sh[1 - pick], 1u);
+      }
+      sh[2] = pick;
+    }
+    __syncthreads();
+    points = w == sh[2];
+    mine = cu + sh[sh[2]];
+  }
+  DEV void done() const {  // after the workgroup's last work
+    if (points && (threadIdx.x & 63u) == 0) atomicSub(mine, 1u);
+  }
+};
 
 // a table in LDS, WORDS words per entry, as the per-lane tables' interface; lane 0 of the quad writes
 struct QuadSecpTab {
@@ -67,6 +91,7 @@ struct QuadSecpTab {
 
 constexpr u32 QUAD_SCALAR_WORDS = 27;  // per item, from the scalar wave; odd, for the banks
 struct QuadShared {
+  u32 role[4];
   u32 sc[QUAD_ITEMS * QUAD_SCALAR_WORDS];
   u32 tab[QUAD_ITEMS * (16 * 36 + 1)];  // secp: QuadSecpTab; Ed25519: 16 cached entries of 36 words
 };
@@ -216,14 +241,13 @@ DEV u32 quad_verify_out(u32 st, const qfe& acc, bool exc, const u32 r[8]) {
   return (eq1 || (eq2 && words_lt(r, C::pmn32()))) ? ST_OK : ST_MISMATCH;
 }
 
-// QUAD_ITEMS items of one curve by one workgroup. valid, i: this quad's item; VERIFY: pubs, status only.
+// 16 items of one curve by one workgroup. points: the wavefront's role; valid, i: this quad's item; VERIFY: pubs, status only.
 // pend: called with the item that needs the careful pass.
 template <class C, bool VERIFY, class Pend>
-DEV void quad_secp_tile(QuadShared& sh, bool valid, u32 i, const uint4* sigs, const uint4* digs, const uint4* pubs,
+DEV void quad_secp_tile(QuadShared& sh, bool points, bool valid, u32 i, const uint4* sigs, const uint4* digs, const uint4* pubs,
                         uint4* out, u8* status, const uint4* comb, const Pend& pend) {
   const u32 item = quad_item();
   u32* sc = sh.sc + item * QUAD_SCALAR_WORDS;
-  const bool points = quad_point_wave();
   QuadSecpTab tab{sh.tab + item * QuadSecpTab::ITEM};
   u32 sr[16];
   u32 st = ST_OK;
@@ -301,31 +325,13 @@ struct QuadEdTab {  // cached odd multiples in LDS: -A at entries 0..7 (written 
 // was found), 19..26 the challenge
 template <class Mem>
 DEV void quad_ed_scalars(const u32 sr[16], const u32 pr[8], const Mem& mem, u64 off, u32 len, u32* sc) {
-  u32 k[8], s[8], c0[5], c1[5];
+  u32 k[8], s[8], cv[8];
   ed25519_challenge(sr, pr, mem, off, len, k);
 #pragma unroll
   for (int i = 0; i < 8; i++) s[i] = sr[8 + i];
-  bool c0_neg = false;
-  const bool ok = ed_lattice(k, c0, c1, c0_neg);
-  u32 v[8], cv[8];
-  {
-    u32 cw[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) cw[i] = i < 5 ? c1[i] : 0u;
-    fe_to_words(fcanon<Fl>(to_mont<Fl>(mont_mul<Fl>(fe_from_words(cw), fe_from_words(s)))), v);
-  }
-  const bool b_neg = (v[0] & 1u) == 0;
-  u32 t[8];
-  words_sub(ED_L32, v, t);
-#pragma unroll
-  for (int i = 0; i < 8; i++) v[i] = b_neg ? t[i] : v[i];
-#pragma unroll
-  for (int i = 0; i < 8; i++) cv[i] = (v[i] >> 1) | (i < 7 ? v[i + 1] << 31 : 0x80000000u);
-  const bool a_fix = (c0[0] & 1u) == 0;
-  c0[0] |= 1u;
-  u32 ca[5], cr[5];
-  glv_carrier<ED_LAT_BITS>(c0, ca);
-  glv_carrier<ED_LAT_BITS>(c1, cr);
+  ed_lat o;
+  const bool ok = ed_lat_scalars(k, s, o);
+  ed_v_carrier(o.v, cv);
   if (q_lane() == 0) {
 #pragma unroll
     for (int i = 0; i < 8; i++) {
@@ -334,20 +340,22 @@ DEV void quad_ed_scalars(const u32 sr[16], const u32 pr[8], const Mem& mem, u64 
     }
 #pragma unroll
     for (int i = 0; i < 5; i++) {
-      sc[8 + i] = ca[i];
-      sc[13 + i] = cr[i];
+      sc[8 + i] = o.ca[i];
+      sc[13 + i] = o.cr[i];
     }
-    sc[18] = (u32)b_neg | ((u32)c0_neg << 1) | ((u32)a_fix << 2) | ((u32)ok << 3);
+    sc[18] = (u32)o.b_neg | ((u32)o.a_neg << 1) | ((u32)o.a_fix << 2) | ((u32)ok << 3);
   }
 }
 
-// [v]B - [c0]A - [c1]R == identity (ed_check_lattice), on every lane
+// [v]B - [c0]A - [c1]R == identity (ed_check_lattice_wide), on every lane
 DEV bool quad_ed_check(const QuadEdTab& tab, const u32* sc, const uint4* comb) {
   constexpr int W = ED_LAT_BITS / 4;
   const u32 sg = sc[18], q = q_lane();
   const bool b_neg = sg & 1u, a_neg = (sg >> 1) & 1u, a_fix = (sg >> 2) & 1u;
   const qfe one = s_from(fe_from_const(Fe::ONE));
   const qfe identity = q_keep<Q1 | Q2>(one);
+  qfe half = s_from(fe_zero());  // 2^260 mod p
+  half.v[0] = 608;
   auto entry = [&](int base, const u32* c, int i, bool neg) {
     const u32 d = quad_digit4(c, i);
     return tab.load(base + (((d < 8) ? ~d : d) & 7u), (d < 8) != neg);
@@ -370,7 +378,8 @@ DEV bool quad_ed_check(const QuadEdTab& tab, const u32* sc, const uint4* comb) {
     const u32 d = quad_digit16(sc, i);
     const u32 j = ((d < COMB_ENTRIES) ? ~d : d) & (COMB_ENTRIES - 1u);
     const bool neg = (d < COMB_ENTRIES) != b_neg;
-    // lanes Y - X, Y + X, (1), 2dXY of entries stored as Y + X, Y - X, 2dXY
+    // lanes (y - x)/2, (y + x)/2, -, dxy of entries stored as (y + x)/2, (y - x)/2, dxy; lane 2 takes
+    // 1/2, so that q_eadd's doubled Z product is Z
     const u32 f = q < 2 ? ((1u - q) ^ (u32)neg) : 2u;
     const uint4* p = comb + ED_COMB_UINT4 * ((u64)i * COMB_ENTRIES + j) + 2 * f;
     const uint4 a = p[0], b = p[1];
@@ -383,7 +392,7 @@ DEV bool quad_ed_check(const QuadEdTab& tab, const u32* sc, const uint4* comb) {
     const sfe x = s_from(fe_from_words(w));
     const bool neg = (quad_digit16(sc, i) < COMB_ENTRIES) != b_neg;
     if (i + 1 < COMB_WINDOWS) load(i + 1, w);
-    acc = q_eadd(acc, q_sel<Q2>(one, s_neg_if(neg && q == 3, x)));
+    acc = q_eadd(acc, q_sel<Q2>(half, s_neg_if(neg && q == 3, x)));
   }
   // X == 0 (lane 0) and Y == Z (lane 1)
   const qfe z = s_carry(s_sub(acc, q_keep<Q1>(q_bcast<2>(acc))));
@@ -391,20 +400,14 @@ DEV bool quad_ed_check(const QuadEdTab& tab, const u32* sc, const uint4* comb) {
   return quad_flags(zero, 0) && quad_flags(zero, 1);
 }
 
-struct BTabGlobal {  // the resident fixed-base table read from HBM
-  const uint4* t;
-  DEV void load(u32 idx, fe& ypx, fe& ymx, fe& t2d) const { BTabLds{t}.load(idx, ypx, ymx, t2d); }
-};
-
 // QUAD_ITEMS Ed25519 items by one workgroup; ct, bt: the full-length check's tables (challenges without a
 // short pair, about 3 in 10^6)
 template <bool STRICT>
-DEV void quad_ed_tile(QuadShared& sh, bool valid, u32 i, const uint4* sigs, const uint4* aux, const u32* msgs,
+DEV void quad_ed_tile(QuadShared& sh, bool points, bool valid, u32 i, const uint4* sigs, const uint4* aux, const u32* msgs,
                       const u64* msg_off, u8* status, const uint4* comb, CTabDev& ct, const BTabGlobal& bt) {
   const u32 item = quad_item();
   u32* sc = sh.sc + item * QUAD_SCALAR_WORDS;
   QuadEdTab tab{sh.tab + item * QuadEdTab::ITEM};
-  const bool points = quad_point_wave();
   u32 sr[16], pr[8];
   u32 flags = 0;  // of this lane's point: bit 0 decodes, 1 as compress would have encoded it, 2 small order
   if (valid) {

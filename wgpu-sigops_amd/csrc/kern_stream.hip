@@ -187,11 +187,9 @@ DEV void stream_store_out(const StreamArgs& a, u32 t, u32 l, const u32 o[16]) {
 // its tiles run out: the batch's last slot, or the count the host closed.
 __global__ __launch_bounds__(256, SIGOPS_WAVES_PER_EU) void k_stream_run(StreamArgs a, const uint4* __restrict__ comb_k1,
                                                                     const uint4* __restrict__ comb_r1,
+                                                                    const uint4* __restrict__ comb_ed,
                                                                     const uint4* __restrict__ gb,
                                                                     uint4* __restrict__ lane_tab, u32 lane_slots) {
-  __shared__ uint4 s_b[BTAB_ENTRIES * 7];
-  for (int t = threadIdx.x; t < BTAB_ENTRIES * 7; t += blockDim.x) s_b[t] = gb[t];
-  __syncthreads();
   const u32 lane = threadIdx.x & 63u;
   const u32 slot = blockIdx.x * blockDim.x + threadIdx.x;
   STabDev jt;
@@ -251,8 +249,8 @@ __global__ __launch_bounds__(256, SIGOPS_WAVES_PER_EU) void k_stream_run(StreamA
         if ((u64)rel + len <= d.y) {
           u32 sr[16], ar[8];
           stream_load(a, p, lane, sr, ar);
-          const u32 st = ed25519_verify_item<false>(sr, ar, MemDev{(const u32*)a.dmsgs}, m0 + rel, len, ct,
-                                                    BTabLds{s_b});
+          const u32 st = ed25519_verify_wide<false>(sr, ar, MemDev{(const u32*)a.dmsgs}, m0 + rel, len, ct,
+                                                    BTabGlobal{gb}, EdCombDev{comb_ed});
           a.st[(u64)p * 64 + lane] = (u8)st;
         }
       }
@@ -335,8 +333,8 @@ hipError_t launch_stream(const StreamLaunch& L, hipStream_t s) {
   a.limit_ticks = L.limit_ticks;
   a.msg_cap = L.msg_cap;
   k_zero_words<<<1, 256, 0, s>>>(L.ctr, STREAM_CTR_BYTES / 4);
-  k_stream_run<<<L.grid, 256, 0, s>>>(a, (const uint4*)L.comb_k1, (const uint4*)L.comb_r1, (const uint4*)L.gb,
-                                      (uint4*)L.lane_tab, L.lane_slots);
+  k_stream_run<<<L.grid, 256, 0, s>>>(a, (const uint4*)L.comb_k1, (const uint4*)L.comb_r1, (const uint4*)L.comb_ed,
+                                      (const uint4*)L.gb, (uint4*)L.lane_tab, L.lane_slots);
   k_stream_careful<<<64, 64, 0, s>>>(a, (const uint4*)L.gk1, (const uint4*)L.gr1);
   return hipGetLastError();
 }

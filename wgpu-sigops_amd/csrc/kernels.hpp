@@ -29,6 +29,7 @@ struct SecpLaunch {
   uint32_t slots, grid;
   uint32_t* pend_list;
   uint32_t* pend_count;
+  uint32_t* quad_load;  // QUAD_LOAD_WORDS, shared by every launch on the device
 };
 hipError_t launch_secp_recover_CurveK1(const SecpLaunch& L, const void* sigs, const void* digs, void* out,
                                       void* status, uint32_t n, hipStream_t s);
@@ -47,6 +48,8 @@ hipError_t launch_secp_verify_CurveR1(const SecpLaunch& L, const void* sigs, con
 // / 812 at 20,011; secp256r1 verification 563 / 1,140, 656 / 1,148, 1,255 / 1,148; Ed25519 with
 // messages up to 200 bytes 320 / 990, 543 / 1,000 (one lane per item with its bucketing).
 constexpr uint32_t QUAD_MAX_ITEMS = 16384;
+// the counters that keep point waves apart (kern_quad.hpp, QuadRole), zero at first
+constexpr uint32_t QUAD_LOAD_WORDS = 16 * 256 * 4;
 // pend_count is cleared; the careful pass is the caller's (launch_secp_*_careful)
 hipError_t launch_quad_secp(int curve, bool verify, const SecpLaunch& L, const void* sigs, const void* digs,
                             const void* pubs, void* out, void* status, uint32_t n, hipStream_t s);
@@ -59,7 +62,8 @@ struct EdQuadLaunch {
   const void* comb;
   const void* gb;     // resident table, for the full-length check
   void* lane_tab;
-  uint32_t slots;     // at least QUAD_MAX_ITEMS / 16 * 128
+  uint32_t slots;     // at least QUAD_MAX_ITEMS / 16 * 64
+  uint32_t* quad_load;
 };
 hipError_t launch_quad_ed(bool strict, const EdQuadLaunch& L, uint32_t n, hipStream_t s);
 
@@ -73,7 +77,7 @@ hipError_t launch_comb_build(int curve, const void* gtab, void* comb, void* tmp,
 constexpr uint32_t BUCKET_K1 = 0, BUCKET_R1 = 1, BUCKET_ED0 = 2;
 constexpr uint32_t ED_BINS = 40;  // Ed25519 buckets by SHA-512 block count 1..40 (40 = "40 or more")
 constexpr uint32_t NBUCKETS = 2 + ED_BINS;
-constexpr uint32_t BATCH_WORK_WORDS = 3 * NBUCKETS + 3;  // counts, cursors, tile starts, tile ctr, pending ctr
+constexpr uint32_t BATCH_WORK_WORDS = 4 * NBUCKETS + 3;  // counts, cursors, tile starts, tile ctr, pending ctr, buckets
 constexpr uint32_t MAX_TILE_ROUNDS = 4;
 
 // The buffers of one batch call and its size. The host writes them into device memory
@@ -102,6 +106,9 @@ struct BatchLaunch {
   const void* gb;
   const void* comb_k1;
   const void* comb_r1;
+  const void* comb_ed;
+  const void* caller_gb;    // plain Ed25519 only: a caller's converted table of B, or null
+  uint32_t* quad_load;
   void* scratch;            // ItemScratch of the secp items, by position in `order`
   uint32_t scratch_stride;  // its positions: the capacity of `order`
   void* lane_tab;
@@ -112,9 +119,17 @@ struct BatchLaunch {
 };
 
 hipError_t launch_batch(const BatchLaunch& L, hipStream_t s);
+// A small mixed batch: four lanes per item, one workgroup per tile of 16 items of one bucket. Measured
+// (us per device call, four lanes against one lane per item, messages up to 4 KB): 684 / 1,650 at 1,000
+// items, 711 / 1,650 at 8,000, 1,181 / 1,650 at 16,384, 1,466 / 1,482 at 24,576.
+constexpr uint32_t BATCH_QUAD_MAX_ITEMS = 24576;
+constexpr uint32_t BATCH_QUAD_TILE = 16;
+constexpr uint32_t BATCH_QUAD_BLOCKS = BATCH_QUAD_MAX_ITEMS / BATCH_QUAD_TILE + NBUCKETS;
+constexpr uint32_t BATCH_QUAD_LANES = BATCH_QUAD_BLOCKS * 64;  // point lanes
+hipError_t launch_batch_small(const BatchLaunch& L, hipStream_t s);
 // plain Ed25519 verification of an all-Ed25519 batch (io->scheme == NULL, io->out == NULL): the
 // bucketing, then the persistent kernel on Ed25519 tiles with the challenges hashed inside it;
-// strict: ed25519-dalek verify_strict rules; L.gb is the fixed-base table
+// strict: ed25519-dalek verify_strict rules (resident table only)
 hipError_t launch_ed_verify(const BatchLaunch& L, bool strict, hipStream_t s);
 
 // ---- streamed tiles: the host packs tiles into pinned, device-mapped memory while one persistent
@@ -157,6 +172,7 @@ struct StreamLaunch {
   const void* gb;
   const void* comb_k1;   // wide tables
   const void* comb_r1;
+  const void* comb_ed;
   void* lane_tab;
   uint32_t slots;        // tiles a wavefront may take at most
   uint32_t base, mask;   // see qpos (a batch: 0 and ~0)
@@ -182,6 +198,7 @@ struct RingResources {
   const void* gb;
   const void* comb_k1;
   const void* comb_r1;
+  const void* comb_ed;
   void* lane_tab;
   uint32_t lane_slots, grid;
   const uint32_t* bucket_order;  // processing rank -> bucket, NBUCKETS entries

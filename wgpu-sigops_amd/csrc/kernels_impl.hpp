@@ -220,6 +220,25 @@ struct CombDev {
   }
 };
 
+// the wide Ed25519 table
+constexpr u32 ED_COMB_UINT4 = 6;  // per entry
+struct EdCombDev {
+  const uint4* t;
+  DEV void load(int i, u32 j, ed_comb_entry& e) const {
+    const uint4* p = t + ED_COMB_UINT4 * ((u64)i * COMB_ENTRIES + j);
+#pragma unroll
+    for (int c = 0; c < (int)ED_COMB_UINT4; c++) {
+      const uint4 q = p[c];
+      e.v[4 * c] = q.x; e.v[4 * c + 1] = q.y; e.v[4 * c + 2] = q.z; e.v[4 * c + 3] = q.w;
+    }
+  }
+};
+
+struct BTabGlobal {  // the resident 8-bit table of B read from HBM
+  const uint4* t;
+  DEV void load(u32 idx, fe& ypx, fe& ymx, fe& t2d) const { BTabLds{t}.load(idx, ypx, ymx, t2d); }
+};
+
 // Per-item scratch between the stages of a secp call, chunk c of position p at base[c * stride + p]:
 // first u1 and u2 (4 chunks), then the Jacobian result and its status (7 chunks)
 struct ItemScratch {

@@ -742,6 +742,7 @@ void RingEngine::publish_counts() {
   L.grid = res.grid;
   L.comb_k1 = res.comb_k1;
   L.comb_r1 = res.comb_r1;
+  L.comb_ed = res.comb_ed;
   sigops::stream_poll_ticks(S->cfg.device, L);
   const bool ok = e.ev && sigops::launch_stream(L, res.stream) == hipSuccess &&
                   hipEventRecord(e.ev, res.stream) == hipSuccess;

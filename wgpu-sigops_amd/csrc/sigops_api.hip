@@ -45,6 +45,7 @@ void* g_scratch[NOALLOC_MAX_DEVICES];  // device address of `scratch` per device
 // there (servers hold one per slot); freed with the last one. They are only read after the build.
 struct CombTables {
   void* t[3] = {};  // secp256k1, secp256r1, Ed25519
+  uint32_t* quad_load = nullptr;  // counters of the running point waves per SIMD (kern_quad.hpp)
   unsigned refs = 0;
 };
 std::mutex g_comb_mu;
@@ -62,12 +63,15 @@ hipError_t comb_acquire(int device, const void* const gtab[3], hipStream_t s, Co
       if (e == hipSuccess) e = hipMalloc(&t.t[k], sigops::comb_bytes(k));
       if (e == hipSuccess) e = sigops::launch_comb_build(k, gtab[k], t.t[k], tmp, s);
     }
+    if (e == hipSuccess) e = hipMalloc((void**)&t.quad_load, sigops::QUAD_LOAD_WORDS * sizeof(uint32_t));
+    if (e == hipSuccess) e = hipMemsetAsync(t.quad_load, 0, sigops::QUAD_LOAD_WORDS * sizeof(uint32_t), s);
     const hipError_t se = hipStreamSynchronize(s);
     if (e == hipSuccess) e = se;
     if (tmp) (void)hipFree(tmp);
     if (e != hipSuccess) {
       for (void* p : t.t)
         if (p) (void)hipFree(p);
+      if (t.quad_load) (void)hipFree(t.quad_load);
       g_comb.erase(device);
       return e;
     }
@@ -82,12 +86,19 @@ void comb_release(int device) {
   auto it = g_comb.find(device);
   if (it == g_comb.end() || --it->second.refs) return;
   for (void* p : it->second.t) (void)hipFree(p);
+  (void)hipFree(it->second.quad_load);
   g_comb.erase(it);
 }
 
 // Items the stages' scratch holds (470 MB); a larger device call runs in consecutive pieces of this
 // size on its stream.
 constexpr size_t STAGE_ITEMS = 1u << 22;
+
+// Host batches from this size on are streamed unless the caller has chosen (sigops_set_streaming).
+// Streamed against copied, ms per call: 2.20 / 1.29 at 5,000 items, 2.96 / 2.16 at 50,000, 3.87 / 4.16 at
+// 100,003, 5.37 / 5.18 at 200,000, 9.37 / 9.96 at 400,000, 20.95 / 22.79 at 2^20: below some 65,536 the
+// persistent launch's start and its polling cost more than the overlap gives.
+constexpr size_t STREAM_FROM = 65536;
 
 constexpr uint8_t CANARY = 0xEE;
 // largest caller table: 16 entries x 3 coordinates x 24 limbs (l = 11)
@@ -132,11 +143,12 @@ struct sigops_ctx {
   // the captured mixed-batch launches; they read the call's buffers from d_io, so one graph serves
   // every call on this context
   hipGraphExec_t graph = nullptr;
+  hipGraphExec_t graph_small = nullptr;  // batches of at most BATCH_QUAD_MAX_ITEMS
   DevBuf in, aux, msg, off, out, st, sch;
   uint32_t fault = 0;  // SIGOPS_FAULT_* test switch
   // streamed host batches (stream_host.hpp): one pinned, device-mapped block carved into the
   // layout's regions, a pinned control block, the device counters, the batch tag
-  bool streaming = true;
+  enum { STREAM_OFF, STREAM_ON, STREAM_AUTO } streaming = STREAM_AUTO;
   uint32_t bucket_order[sigops::NBUCKETS];  // processing rank -> bucket (the rank table inverted)
   uint8_t* s_pin = nullptr;
   size_t s_cap = 0;
@@ -256,6 +268,7 @@ sigops::SecpLaunch secp_launch(sigops_ctx* c, int curve, const void* gtab8 = nul
   L.grid = c->grid;
   L.pend_list = c->d_pend + 1;
   L.pend_count = c->d_pend;
+  L.quad_load = c->comb.quad_load;
   return L;
 }
 
@@ -492,6 +505,7 @@ void sigops_destroy(sigops_ctx* c) {
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   if (c->graph) (void)hipGraphExecDestroy(c->graph);
+  if (c->graph_small) (void)hipGraphExecDestroy(c->graph_small);
   if (c->s_ev) (void)hipEventDestroy(c->s_ev);
   for (hipEvent_t e : c->s_tev)
     if (e) (void)hipEventDestroy(e);
@@ -574,11 +588,11 @@ static int ed_verify_dev(sigops_ctx* c, const void* d_sigs, const void* d_pubkey
   if (!d_sigs || !d_pubkeys || !d_msgs || !d_msg_off || !d_status) return fail(c, SIGOPS_E_ARG, "NULL buffer");
   if (((uintptr_t)d_msgs & 3u) != 0) return fail(c, SIGOPS_E_ARG, "d_msgs must be 4-byte aligned");
   hipStream_t s = (hipStream_t)stream;
-  // (8 lanes of the lane tables per item, for challenges that need the full-length check)
-  if (!btab && n <= sigops::QUAD_MAX_ITEMS && c->slots >= sigops::QUAD_MAX_ITEMS * 8) {
+  // (4 lanes of the lane tables per item, for challenges that need the full-length check)
+  if (!btab && n <= sigops::QUAD_MAX_ITEMS && c->slots >= sigops::QUAD_MAX_ITEMS * 4) {
     if (c->fault & SIGOPS_FAULT_SKIP_COMPUTE) return SIGOPS_OK;
     const sigops::EdQuadLaunch L{d_sigs, d_pubkeys, d_msgs, d_msg_off, d_status, c->comb.t[2], c->d_btab, c->d_lane_tab,
-                                 c->slots};
+                                 c->slots, c->comb.quad_load};
     HIPCHK(c, sigops::launch_quad_ed(strict, L, (uint32_t)n, s));
     return SIGOPS_OK;
   }
@@ -590,7 +604,9 @@ static int ed_verify_dev(sigops_ctx* c, const void* d_sigs, const void* d_pubkey
   L.order = c->d_order;
   L.pend_list = c->d_pend + 1;
   L.rank = c->d_rank;
-  L.gb = btab ? btab : c->d_btab;
+  L.gb = c->d_btab;
+  L.caller_gb = btab;
+  L.comb_ed = c->comb.t[2];
   L.lane_tab = c->d_lane_tab;
   L.slots = c->slots;
   // every bucket may end in a partial tile: at most NBUCKETS tiles beyond n / 64, 4 tiles per block
@@ -757,37 +773,44 @@ int sigops_batch_dev(sigops_ctx* c, const void* d_schemes, const void* d_sigs, c
   L.tile_rounds = c->tile_rounds;
   L.comb_k1 = c->comb.t[0];
   L.comb_r1 = c->comb.t[1];
+  L.comb_ed = c->comb.t[2];
+  L.quad_load = c->comb.quad_load;
   L.scratch = c->d_scratch;
   L.scratch_stride = c->scratch_stride;
   L.stage_grid = c->grid / c->blocks_per_cu;
   L.waves = c->waves;
   L.stage_ev = nullptr;
+  // a small batch needs lane tables for every lane of its launch (a context of one block per CU on a
+  // device with fewer CUs may not have them)
+  const bool small = n <= sigops::BATCH_QUAD_MAX_ITEMS && c->slots >= sigops::BATCH_QUAD_LANES;
+  const auto launch = small ? sigops::launch_batch_small : sigops::launch_batch;
   if (c->stage_timing) {
     L.stage_ev = c->stage_ev;
-    HIPCHK(c, sigops::launch_batch(L, s));
+    HIPCHK(c, launch(L, s));
     c->stage_recorded = true;
     return SIGOPS_OK;
   }
   if (!c->use_graph) {
-    HIPCHK(c, sigops::launch_batch(L, s));
+    HIPCHK(c, launch(L, s));
     return SIGOPS_OK;
   }
-  if (!c->graph) {
+  hipGraphExec_t& graph = small ? c->graph_small : c->graph;
+  if (!graph) {
     L.aux_grid = c->grid;  // the graph does not depend on n
     hipGraph_t g;
     HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    hipError_t le = sigops::launch_batch(L, c->stream);
+    hipError_t le = launch(L, c->stream);
     hipError_t ce = hipStreamEndCapture(c->stream, &g);
     if (le != hipSuccess) return hip_fail(c, le, "launch_batch under capture");
     if (ce != hipSuccess) return hip_fail(c, ce, "hipStreamEndCapture");
-    hipError_t ie = hipGraphInstantiate(&c->graph, g, nullptr, nullptr, 0);
+    hipError_t ie = hipGraphInstantiate(&graph, g, nullptr, nullptr, 0);
     (void)hipGraphDestroy(g);
     if (ie != hipSuccess) {
-      c->graph = nullptr;
+      graph = nullptr;
       return hip_fail(c, ie, "hipGraphInstantiate");
     }
   }
-  HIPCHK(c, hipGraphLaunch(c->graph, s));
+  HIPCHK(c, hipGraphLaunch(graph, s));
   return SIGOPS_OK;
 }
 
@@ -1058,6 +1081,7 @@ int batch_streamed(sigops_ctx* c, const uint8_t* schemes, const uint8_t* sigs, c
   L.grid = std::min<uint32_t>(c->grid, (uint32_t)((g.slots + 3) / 4));
   L.comb_k1 = c->comb.t[0];
   L.comb_r1 = c->comb.t[1];
+  L.comb_ed = c->comb.t[2];
   sigops::stream_poll_ticks(c->device, L);
   HIPCHK(c, hipEventRecord(c->s_tev[0], s));
   if (!(c->fault & SIGOPS_FAULT_SKIP_COMPUTE)) HIPCHK(c, sigops::launch_stream(L, s));
@@ -1128,6 +1152,7 @@ int sigops_ring_resources(sigops_ctx* c, sigops::RingResources* r) {
   r->grid = c->grid;
   r->comb_k1 = c->comb.t[0];
   r->comb_r1 = c->comb.t[1];
+  r->comb_ed = c->comb.t[2];
   r->bucket_order = c->bucket_order;
   r->stream = c->stream;
   return SIGOPS_OK;
@@ -1143,7 +1168,7 @@ int sigops_batch_host_ms(sigops_ctx* c, float* ms) {
 
 int sigops_set_streaming(sigops_ctx* c, int on) {
   if (!c) return SIGOPS_E_ARG;
-  c->streaming = on != 0;
+  c->streaming = on ? sigops_ctx::STREAM_ON : sigops_ctx::STREAM_OFF;
   return SIGOPS_OK;
 }
 
@@ -1167,7 +1192,7 @@ int sigops_batch(sigops_ctx* c, const uint8_t* schemes, const uint8_t* sigs, con
     st = c->host_status.data();
   }
   int rc;
-  if (c->streaming && n >= 4096) {
+  if (n >= (c->streaming == sigops_ctx::STREAM_ON ? 4096 : STREAM_FROM) && c->streaming != sigops_ctx::STREAM_OFF) {
     rc = batch_streamed(c, schemes, sigs, aux, msgs, msg_off, n, out, st);
     if (rc < 0) return rc;
     if (rc == SIGOPS_OK) {
