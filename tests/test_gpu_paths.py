@@ -1,7 +1,10 @@
 """Every path a plain call can take by its size: four lanes per item up to 16,384 items, one lane per
 item with shared inversions above, around the sizes where the path, the workgroups or the stages'
-lanes change. Each call holds the edge cases and corrupted generated items, repeated to the size, and
-every result is compared with the oracle's."""
+lanes change; for message digests the order in one or three launches and one or two wavefronts to a
+message. Each call holds the edge cases and corrupted generated items, repeated to the size, and every
+result is compared with the oracle's."""
+import hashlib
+
 import numpy as np
 import pytest
 
@@ -124,3 +127,26 @@ def test_mixed_sizes(ctx):
             want = rows[j][5]
             mine = st[at == j]
             assert np.all((mine == 0) == good[j]) if want is None else np.all(mine == want), (n, j)
+
+
+# one length (two wavefronts to a message while all lanes are not filled, one wavefront above), lengths
+# around the blocks' edges, and long ones among short ones
+@pytest.mark.parametrize("lens", [[40], [0, 1, 55, 56, 63, 64, 119, 120, 3, 200], [5] * 40 + [4096, 4300, 700]])
+@pytest.mark.parametrize("skew", [0, 4])
+def test_message_new_sizes(ctx, lens, skew):
+    import torch
+    for n in [1, 64, 65, 8192, 8193, 40001, 300001]:
+        if n * np.mean(lens) > 4e7:
+            continue
+        print(f"message_new lens={lens[-1]} skew={skew} n={n}", flush=True)
+        rng = np.random.default_rng(n)
+        ln = np.array(lens)[_at(n, len(lens), n)]
+        rng.shuffle(ln)
+        off = np.concatenate([[0], np.cumsum(ln)]).astype(np.int64)
+        buf = rng.integers(0, 256, skew + int(off[-1]) + 16, dtype=np.uint8)
+        want = [hashlib.sha256(buf[skew + off[i]:skew + off[i + 1]]).digest() for i in range(n)]
+        d_buf, d_off = torch.from_numpy(buf).cuda(), torch.from_numpy(off).cuda()
+        d_out = torch.zeros(n, 32, dtype=torch.uint8, device="cuda")
+        ctx.message_new_dev(d_buf.data_ptr() + skew, d_off.data_ptr(), n, d_out.data_ptr())
+        torch.cuda.synchronize()
+        assert np.array_equal(d_out.cpu().numpy(), _bytes(want, 32)), n

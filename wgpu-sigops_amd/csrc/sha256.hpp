@@ -74,6 +74,37 @@ DEV void sha256_compress(u32 h[8], u32 w[16]) {
   for (int i = 0; i < 8; i++) h[i] += s[i];
 }
 
+// sha256_compress for two wavefronts. K[t] + W[t] of half a block, four words at a time in put(q, ...),
+// q = 0..7: HALF 0 from the block's words, HALF 1 after it from what it left in w.
+template <int HALF, class Put>
+DEV void sha256_expand(u32 w[16], const Put& put) {
+#pragma unroll
+  for (int j = 0; j < 32; j++) {
+    const int t = 32 * HALF + j;
+    if (t >= 16) {
+      const u32 w15 = w[(t + 1) & 15], w2 = w[(t + 14) & 15];
+      const u32 s0 = xor3_32(rotr32(w15, 7), rotr32(w15, 18), w15 >> 3);
+      const u32 s1 = xor3_32(rotr32(w2, 17), rotr32(w2, 19), w2 >> 10);
+      w[t & 15] += s0 + w[(t + 9) & 15] + s1;
+    }
+    if ((t & 3) == 3)
+      put(j >> 2, w[(t - 3) & 15] + SHA256_K[t - 3], w[(t - 2) & 15] + SHA256_K[t - 2],
+          w[(t - 1) & 15] + SHA256_K[t - 1], w[t & 15] + SHA256_K[t]);
+  }
+}
+// and 4 Q rounds on the working state, get(q) being four words .x .y .z .w
+template <int Q, class Get>
+DEV void sha256_rounds(u32 (&s)[8], const Get& get) {
+#pragma unroll
+  for (int q = 0; q < Q; q++) {
+    const auto k = get(q);
+    sha256_round(s, (4 * q) & 7, k.x);
+    sha256_round(s, (4 * q + 1) & 7, k.y);
+    sha256_round(s, (4 * q + 2) & 7, k.z);
+    sha256_round(s, (4 * q + 3) & 7, k.w);
+  }
+}
+
 // a block whose schedule is a constant, given as K[t] + W[t] (the padding block of a message
 // whose length is a multiple of 64 bytes): rounds only
 DEV void sha256_compress_kw(u32 h[8], const u32 (&kw)[64]) {
@@ -118,14 +149,17 @@ DEV void sha256_block_assemble(const u32 raw[17], u32 sh, u32 len, u32 b, u32 nb
 // (the word at off for an empty message), so they never reach more than 3 bytes past the message
 // and need no branch.
 template <class Mem>
-DEV void sha256_block_words(const Mem& mem, u64 off, u32 len, u32 b, u32 nblk, u32 w[16]) {
-  const u64 base = off + (u64)b * 64;
-  const u64 wa = base >> 2;
+DEV void sha256_block_load(const Mem& mem, u64 off, u32 len, u32 b, u32 raw[17]) {
+  const u64 wa = (off + (u64)b * 64) >> 2;
   const u64 lim = (off + len - (len != 0)) >> 2;
-  u32 raw[17];
 #pragma unroll
   for (int k = 0; k < 17; k++) raw[k] = mem.word(wa + k < lim ? wa + k : lim);
-  sha256_block_assemble(raw, (u32)(base & 3u) * 8u, len, b, nblk, w);
+}
+template <class Mem>
+DEV void sha256_block_words(const Mem& mem, u64 off, u32 len, u32 b, u32 nblk, u32 w[16]) {
+  u32 raw[17];
+  sha256_block_load(mem, off, len, b, raw);
+  sha256_block_assemble(raw, (u32)(off & 3u) * 8u, len, b, nblk, w);
 }
 
 // The same from a 16-byte-aligned buffer with five 16-byte loads per lane instead of 17 word loads
@@ -135,15 +169,15 @@ DEV void sha256_block_words(const Mem& mem, u64 off, u32 len, u32 b, u32 nblk, u
 // The block's words are placed with lane masks; a version with conditional selects measured
 // twice as slow on messages of mixed lengths.
 template <class Mem>
-DEV void sha256_block_words_x4(const Mem& mem, u64 off, u32 len, u32 b, u32 nblk, u32 w[16]) {
-  const u64 base = off + (u64)b * 64;
-  const u64 c0 = base >> 4;
+DEV void sha256_block_load_x4(const Mem& mem, u64 off, u32 len, u32 b, u32 r[20]) {
+  const u64 c0 = (off + (u64)b * 64) >> 4;
   const u64 cl = (off + len - (len != 0)) >> 4;
-  u32 r[20];
 #pragma unroll
   for (int k = 0; k < 5; k++) mem.quad(c0 + k < cl ? c0 + k : cl, r + 4 * k);
+}
+DEV void sha256_block_place_x4(const u32 r[20], u64 off, u32 len, u32 b, u32 nblk, u32 w[16]) {
   // the block starts at word q0 = 0..3 of the first chunk: raw[j] = r[q0 + j], by lane masks
-  const u32 q0 = (u32)(base >> 2) & 3u;
+  const u32 q0 = (u32)(off >> 2) & 3u;
   const u32 m1 = 0u - (q0 & 1u), m2 = 0u - ((q0 >> 1) & 1u);
   u32 raw[17];
 #pragma unroll
@@ -152,7 +186,13 @@ DEV void sha256_block_words_x4(const Mem& mem, u64 off, u32 len, u32 b, u32 nblk
     const u32 odd = (r[j + 3] & m2) | (r[j + 1] & ~m2);
     raw[j] = (odd & m1) | (even & ~m1);
   }
-  sha256_block_assemble(raw, (u32)(base & 3u) * 8u, len, b, nblk, w);
+  sha256_block_assemble(raw, (u32)(off & 3u) * 8u, len, b, nblk, w);
+}
+template <class Mem>
+DEV void sha256_block_words_x4(const Mem& mem, u64 off, u32 len, u32 b, u32 nblk, u32 w[16]) {
+  u32 r[20];
+  sha256_block_load_x4(mem, off, len, b, r);
+  sha256_block_place_x4(r, off, len, b, nblk, w);
 }
 
 // SHA-256(msg[0..len)), msg at byte offset off; out: the 32 digest bytes as 8 little-endian words

@@ -834,7 +834,7 @@ int sigops_message_new_dev(sigops_ctx* c, const void* d_data, const uint64_t* d_
   if (!d_data || !d_off || !d_digests) return fail(c, SIGOPS_E_ARG, "NULL buffer");
   if (((uintptr_t)d_data & 3u) != 0) return fail(c, SIGOPS_E_ARG, "d_data must be 4-byte aligned");
   HIPCHK(c, sigops::launch_message_new(d_data, d_off, (uint32_t)n, d_digests, c->d_hq, c->d_horder, 2 * c->grid,
-                                       (hipStream_t)stream));
+                                       c->grid / c->blocks_per_cu, (hipStream_t)stream));
   return SIGOPS_OK;
 }
 
@@ -853,7 +853,7 @@ int sigops_message_new_noalloc(sigops_ctx* c, const void* d_data, const uint64_t
   // the launch clears the work words with a kernel and writes the order before reading it, so
   // what an earlier call left in the array does not matter
   HIPCHK(c, sigops::launch_message_new(d_data, d_off, (uint32_t)n, d_digests, work, order, 2 * c->grid,
-                                       (hipStream_t)stream));
+                                       c->grid / c->blocks_per_cu, (hipStream_t)stream));
   return SIGOPS_OK;
 }
 
@@ -875,7 +875,7 @@ int sigops_message_new(sigops_ctx* c, const uint8_t* data, const uint64_t* off, 
   k_fill_bytes<<<1, 64, 0, s>>>((uint8_t*)c->msg.p + total, 0, 16);
   HIPCHK(c, hipGetLastError());
   HIPCHK(c, sigops::launch_message_new(c->msg.p, (const uint64_t*)c->off.p, (uint32_t)n, c->aux.p, c->d_hq, c->d_horder,
-                                       2 * c->grid, s));
+                                       2 * c->grid, c->grid / c->blocks_per_cu, s));
   return get(c, {{digests, c->aux.p, n * 32}});
 }
 
