@@ -4,11 +4,11 @@
 // of any length. The reference has one kernel chain per scheme and fixed 32-byte messages; here:
 //   1. k_bucket_hist / k_bucket_scan / k_bucket_scatter sort item indices into buckets (k1, r1, and
 //      Ed25519 by SHA-512 block count, so the lanes of a wavefront hash equally long messages), each
-//      bucket padded to whole tiles; the buckets are processed in the context's order (its rank
+//      scheme padded to whole tiles; the buckets are processed in the context's order (its rank
 //      table: secp256r1, secp256k1, then Ed25519 by decreasing block count);
 //   2. k_batch_scalars computes u1 and u2 of the secp items, several per lane with one inversion;
 //   3. k_batch_run is persistent: every wavefront pulls the next tile (64 x tile_rounds items of
-//      one bucket) from an atomic counter, so the scheme is uniform across the wavefront and load
+//      one scheme) from an atomic counter, so the scheme is uniform across the wavefront and load
 //      balances dynamically; it runs the same per-item code as the plain kernels;
 //   4. k_batch_finish makes the recovered keys affine, again several per lane with one inversion;
 //   5. k_batch_careful finishes secp items whose fast ladder met an exceptional addition.
@@ -91,33 +91,44 @@ __global__ __launch_bounds__(256) void k_bucket_hist(BatchArgs a) {
 }
 
 // By one wavefront (the block's first): tile offsets in processing order from the buckets' counts c
-// (LDS), DUMMY padding of each bucket's last tile, and each bucket's first position (start, LDS).
+// (LDS), each bucket's first position (start, LDS) and DUMMY padding. Ed25519 buckets that follow each
+// other share tiles: a tile belongs to the bucket of its first position, and one that spans two hashes
+// a block more on some lanes (5,000 VALU instructions of 340,000). With every bucket padded to whole
+// tiles instead, 65,536 items in 9 buckets were 1,029 tiles for 1,024 SIMDs, so that a few took two
+// (a host call 2,774 us; 2,157 us with shared tiles).
 // One thread walking the ranks took 29 us, longer than the sort's other passes.
 DEV void bucket_scan(const BatchArgs& a, const u32* c, u32* start, u32* bucket_of) {
-  static_assert(NBUCKETS <= 64, "one lane per bucket");
+  static_assert(NBUCKETS < 64, "one lane per bucket");
   const u32 lane = threadIdx.x;
   if (lane < 64) {
     if (lane < NBUCKETS) bucket_of[a.rank[lane]] = lane;
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     const u32 b = lane < NBUCKETS ? bucket_of[lane] : 0;
-    const u32 tiles = lane < NBUCKETS ? (c[b] + a.tile_items - 1) / a.tile_items : 0;
-    u32 end = tiles;  // inclusive prefix sum over the ranks
+    const u32 cnt = lane < NBUCKETS ? c[b] : 0;
+    auto prefix = [&](u32 v) {  // inclusive, over the ranks
 #pragma unroll
-    for (u32 d = 1; d < 64; d <<= 1) {
-      const u32 v = __shfl_up(end, d);
-      if (lane >= d) end += v;
-    }
+      for (u32 d = 1; d < 64; d <<= 1) {
+        const u32 u = __shfl_up(v, d);
+        if (lane >= d) v += u;
+      }
+      return v;
+    };
+    // runs of buckets that share tiles: heads, and the items from the run's head up to this bucket's end
+    const u64 ed = __ballot(lane < NBUCKETS && b >= BUCKET_ED0), heads = ~(ed & (ed << 1));
+    const u32 items = prefix(cnt), head = 63u - (u32)__builtin_clzll(heads & (~0ull >> (63u - lane)));
+    const u32 head_items = __shfl(items - cnt, head), run = items - head_items;
+    const bool tail = lane + 1 == NBUCKETS || ((heads >> 1 >> lane) & 1u);
+    const u32 tiles = tail && lane < NBUCKETS ? (run + a.tile_items - 1) / a.tile_items : 0;
+    const u32 end = prefix(tiles), first = (end - tiles) * a.tile_items + run - cnt;
     if (lane < NBUCKETS) {
-      a.tile_start[lane] = end - tiles;
+      a.tile_start[lane] = (first + a.tile_items - 1) / a.tile_items;
       if (lane == NBUCKETS - 1) a.tile_start[NBUCKETS] = end;
-      start[b] = (end - tiles) * a.tile_items;
+      start[b] = first;
       a.bucket_of[lane] = b;
     }
+    if (tiles)
+      for (u32 k = first + cnt; k < end * a.tile_items; k++) a.order[k] = DUMMY;
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    for (u32 q = 0; q < NBUCKETS; q++) {
-      const u32 padded = (c[q] + a.tile_items - 1) / a.tile_items * a.tile_items;
-      for (u32 k = c[q] + lane; k < padded; k += 64) a.order[start[q] + k] = DUMMY;
-    }
   }
 }
 

@@ -609,8 +609,7 @@ static int ed_verify_dev(sigops_ctx* c, const void* d_sigs, const void* d_pubkey
   L.comb_ed = c->comb.t[2];
   L.lane_tab = c->d_lane_tab;
   L.slots = c->slots;
-  // every bucket may end in a partial tile: at most NBUCKETS tiles beyond n / 64, 4 tiles per block
-  L.grid = std::min<uint32_t>(c->grid, (uint32_t)((n + 255) / 256 + (sigops::NBUCKETS + 3) / 4));
+  L.grid = std::min<uint32_t>(c->grid, (uint32_t)((n + 255) / 256));  // 4 tiles per block
   L.aux_grid = std::min<uint32_t>(c->grid, (uint32_t)((n + 255) / 256));
   L.tile_rounds = 1;
   if (c->fault & SIGOPS_FAULT_SKIP_COMPUTE) return SIGOPS_OK;
