@@ -150,3 +150,30 @@ def test_message_new_sizes(ctx, lens, skew):
         ctx.message_new_dev(d_buf.data_ptr() + skew, d_off.data_ptr(), n, d_out.data_ptr())
         torch.cuda.synchronize()
         assert np.array_equal(d_out.cpu().numpy(), _bytes(want, 32)), n
+
+
+@pytest.mark.parametrize("order", [0, 1, 2])
+def test_mixed_bucket_orders(order):
+    """tiles shared by neighbouring Ed25519 buckets and first tiles by place, in every bucket order, with
+    one and two workgroups per compute unit: keys and statuses as in the items' own order"""
+    for blocks in (1, 2):
+        c = sigops.Context(bucket_order=order, blocks_per_cu=blocks)
+        n = 30011
+        s0, d0, p0, _ = O.gen_secp(0, 51, 100, corrupt_ppm=0)
+        s1, d1, p1, _ = O.gen_secp(1, 52, 100, corrupt_ppm=0)
+        off = np.concatenate([[0], np.cumsum(np.arange(300) * 29 % 5000)]).astype(np.uint64)
+        s2, k2, m2, _ = O.gen_ed25519(53, 300, off, corrupt_ppm=300000)
+        ok = np.concatenate([np.ones(200, bool), O.verify_batch(s2, k2, m2, off).astype(bool)])
+        sigs, aux = np.concatenate([s0, s1, s2]), np.concatenate([d0, d1, k2])
+        keys = np.concatenate([p0, p1, np.zeros((300, 64), np.uint8)])
+        lens = np.concatenate([np.zeros(200, np.int64), np.diff(off.astype(np.int64))])
+        begin = np.concatenate([np.zeros(200, np.int64), off[:-1].astype(np.int64)])
+        at = np.random.default_rng(order).integers(0, 500, n)
+        moff = np.concatenate([[0], np.cumsum(lens[at])]).astype(np.uint64)
+        data = np.concatenate([m2[begin[i]:begin[i] + lens[i]] for i in at])
+        schemes = np.where(at < 100, 0, np.where(at < 200, 1, 2)).astype(np.uint8)
+        print(f"mixed order={order} blocks={blocks}", flush=True)
+        c.set_streaming(False)
+        got, st = c.batch(schemes, sigs[at], aux[at], data, moff)
+        c.close()
+        assert np.array_equal(st == 0, ok[at]) and np.array_equal(got, keys[at])

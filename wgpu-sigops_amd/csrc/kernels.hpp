@@ -77,7 +77,9 @@ hipError_t launch_comb_build(int curve, const void* gtab, void* comb, void* tmp,
 constexpr uint32_t BUCKET_K1 = 0, BUCKET_R1 = 1, BUCKET_ED0 = 2;
 constexpr uint32_t ED_BINS = 40;  // Ed25519 buckets by SHA-512 block count 1..40 (40 = "40 or more")
 constexpr uint32_t NBUCKETS = 2 + ED_BINS;
-constexpr uint32_t BATCH_WORK_WORDS = 4 * NBUCKETS + 3;  // counts, cursors, tile starts, tile ctr, pending ctr, buckets
+constexpr uint32_t BATCH_FIRST_TILES = 4096;  // bits of the first tiles' claims: 1,024 workgroups
+// counts, cursors, tile starts, tile ctrs, pending ctr, buckets, claims
+constexpr uint32_t BATCH_WORK_WORDS = 4 * NBUCKETS + 4 + BATCH_FIRST_TILES / 32;
 constexpr uint32_t MAX_TILE_ROUNDS = 4;
 
 // The buffers of one batch call and its size. The host writes them into device memory
@@ -113,7 +115,7 @@ struct BatchLaunch {
   uint32_t scratch_stride;  // its positions: the capacity of `order`
   void* lane_tab;
   uint32_t slots, grid, aux_grid, tile_rounds;
-  uint32_t stage_grid;   // blocks of the stages that share an inversion between items
+  uint32_t stage_grid;   // compute units: blocks of the stages that share an inversion between items
   uint32_t waves;        // mixed batch: waves per SIMD the persistent kernel is built for (1 or 2)
   hipEvent_t* stage_ev;  // null, or 5 events recorded before, between and after the 4 stages
 };
