@@ -116,7 +116,7 @@ def test_mixed_sizes(ctx):
     sigs, aux, out = (_bytes([r[j] for r in rows], w) for j, w in ((1, 64), (2, 32), (4, 64)))
     lens = np.array([len(r[3]) for r in rows])
     perm = np.random.default_rng(5).permutation(len(rows))
-    for n in (1, 15, 17, len(rows), 16384, 24576, 24577, 65535, 65536):
+    for n in (1, 15, 17, len(rows), 16384, 24576, 24577, 65536, 262143, 262144):
         print(f"mixed n={n}", flush=True)
         at = perm[_at(n, len(rows), n)]
         moff = np.concatenate([[0], np.cumsum(lens[at])]).astype(np.uint64)

@@ -95,10 +95,11 @@ void comb_release(int device) {
 constexpr size_t STAGE_ITEMS = 1u << 22;
 
 // Host batches from this size on are streamed unless the caller has chosen (sigops_set_streaming).
-// Streamed against copied, ms per call: 2.20 / 1.29 at 5,000 items, 2.96 / 2.16 at 50,000, 3.87 / 4.16 at
-// 100,003, 5.37 / 5.18 at 200,000, 9.37 / 9.96 at 400,000, 20.95 / 22.79 at 2^20: below some 65,536 the
-// persistent launch's start and its polling cost more than the overlap gives.
-constexpr size_t STREAM_FROM = 65536;
+// Streamed against copied, ms per call (messages up to 4 KB): 3.42 / 2.58 at 65,536 items, 3.62 / 3.27 at
+// 100,003, 5.36 / 5.08 at 200,000, 6.61 / 6.74 at 262,144, 9.36 / 9.76 at 400,000, 20.9 / 22.6 at 2^20: the
+// copied batch's tiles are placed (TileClaims) and its inversions shared, which below some four tiles
+// per wavefront saves more than the overlap with the copies.
+constexpr size_t STREAM_FROM = 1u << 18;
 
 constexpr uint8_t CANARY = 0xEE;
 // largest caller table: 16 entries x 3 coordinates x 24 limbs (l = 11)
