@@ -8,9 +8,8 @@ Candidates (each a Context setting; the library holds every variant's code):
                   atomics but a coarser tail at the end of the batch);
   * bucket_order: the processing order of the buckets (0: secp256r1, secp256k1, Ed25519 by
                   decreasing block count; 1: secp256r1, Ed25519, secp256k1; 2: secp256k1 first).
-  * g_window:     the fixed-base window of the secp streams, 8 bits (128 odd multiples of G in LDS)
-                  or 9 (256, 1.75x the LDS; 4 fewer G additions per secp256k1 item and 3 per P-256
-                  item, on a ladder that takes one doubling per loop iteration).
+  * g_window:     accepted and recorded, without effect: every kernel on the resident tables reads the
+                  16-bit windows, and a caller's table of G keeps 8 bits.
 blocks_per_cu follows waves (one 256-thread workgroup per SIMD wave): more workgroups than fit
 only queue behind the resident ones.
 

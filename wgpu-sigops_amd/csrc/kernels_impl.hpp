@@ -2,8 +2,8 @@
 //
 // One lane per signature, persistent grid-stride kernels (the grid is sized to the resident
 // capacity of the GPU, so a lane's slot index also names its private table in HBM). Per kernel:
-//   * the fixed-base table (odd multiples of G or B, uploaded to HBM once per context) is staged
-//     into LDS by each workgroup and read with ds_read_b128;
+//   * the fixed-base scalars read wide tables in HBM (16-bit windows, 33.5 MB per curve, built once
+//     per device); a caller's own table is staged into LDS and read with ds_read_b128;
 //   * the per-signature variable-base table lives in HBM scratch, laid out [entry][chunk][slot]
 //     so that lanes that pick the same entry read contiguous 16-byte chunks;
 //   * secp lanes whose fast ladder meets an exceptional addition are appended to a pending list

@@ -11,9 +11,10 @@
 //   * both scalars in the signed all-odd digit form k = sum (2c_i - (2^w-1)) 2^(wi) with
 //     C = (k >> 1) | 2^255 for odd k (even k: use n - k and negate the base), so every window
 //     performs exactly one addition and no lane ever branches on a zero digit;
-//   * u2*R: w = 4, table of odd multiples R..15R in per-lane memory, made affine with one
-//     simultaneous inversion so that every addition of the R stream is a mixed addition;
-//   * u1*G: w = 8, table of odd multiples G..255G (affine) staged in LDS by the kernel;
+//   * u2*R: w = 4, table of odd multiples R..15R in per-lane memory, made affine (secp256k1: up to an
+//     isomorphism) so that every addition of the R stream is a mixed addition;
+//   * u1*G: 16 additions from wide tables of G after the chain (secp_comb); with a caller's table of
+//     G, w = 8 on the chain, odd multiples G..255G staged in LDS by the kernel;
 //   * Jacobian formulas dbl-2009-l (a = 0) / dbl-2001-b (a = -3), add-2007-bl, madd-2007-bl.
 //     These are incomplete: an addition of P and +-P is detected (H == 0) and the lane is marked
 //     for the careful path, which redoes the item with complete, branching formulas.
@@ -561,8 +562,8 @@ DEV u32 digit9(const u32* c, int j) {
   return v & 511u;
 }
 
-// fixed-base windows of 9 bits: 256 odd multiples of G (LDS 1.75x larger, 4 fewer G additions per
-// secp256k1 item and 3 per P-256 item). The carriers come from the 8-bit ones: a carrier is
+// fixed-base windows of 9 bits (the host check's second form): 256 odd multiples of G, 4 fewer G
+// additions per secp256k1 item and 3 per P-256 item than 8 bits. The carriers come from the 8-bit ones: a carrier is
 // (h >> 1) | 2^(B-1) for the odd h it spells, so moving the marker bit re-spells h over B' bits.
 constexpr int GLV_BG9 = 135;  // G streams of secp256k1: 15 windows of 9 bits
 constexpr int R1_BG9 = 261;   // the G stream of P-256: 29 windows of 9 bits
