@@ -52,10 +52,16 @@ struct QuadRole {
   }
 };
 
-// a table in LDS, WORDS words per entry, as the per-lane tables' interface; lane 0 of the quad writes
+// a table in LDS, as the per-lane tables' interface; lane 0 of the quad writes, all four read
 struct QuadSecpTab {
   u32* t;  // this item's 8 entries: x, w, then (building) the factor of Z or (secp256k1) beta x
   static constexpr u32 ENTRY = 27, ITEM = 8 * ENTRY + 1;  // + 1: the items' entries on different banks
+  // The quad is within one wavefront, whose LDS accesses execute in their order in the code: what is
+  // needed is that the compiler keeps that order across lanes. No instruction comes of it.
+  DEV void sync() const {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
   DEV void put(u32 e, int f, const fe& x) {
     if (q_lane() == 0) {
 #pragma unroll

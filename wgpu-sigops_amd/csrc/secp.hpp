@@ -622,7 +622,16 @@ DEV jacs g_add(const jacs& acc, const GTab& gt, u32 d, bool neg_stream, const sf
 //   * a = -3 (P-256): the doubling needs a, so the entries are made affine on the curve itself by
 //     one inversion of Z2 Z_7 (Montgomery's trick, with the same factors).
 // Tab: store_full(e, (X, W, zr), unused) / load_full and store_affine(e, x, w) / load_affine (and
-// the _phi forms with beta x). Returns zeta (1 for P-256).
+// the _phi forms with beta x); sync() if other lanes read what one lane stores: it orders the stores
+// before it with the other lanes' loads after it, and loads with stores likewise. Returns zeta (1 for
+// P-256).
+template <class Tab>
+DEV auto tab_sync(Tab& tab, int) -> decltype(tab.sync()) {
+  tab.sync();
+}
+template <class Tab>
+DEV void tab_sync(Tab&, long) {}
+
 template <class C, class Tab>
 DEV sfe secp_build_table(const secp_pro& o, Tab& tab, bool& exc) {
   typedef typename C::Fp F;
@@ -655,6 +664,7 @@ DEV sfe secp_build_table(const secp_pro& o, Tab& tab, bool& exc) {
     T.Z = s_mul<F>(T.Z, zr);
     tab.store_full(e, jac{s_raw(T.X), s_raw(T.W), s_raw(zr)}, fe_zero());
   }
+  tab_sync(tab, 0);
   sfe zeta = s_mul<F>(T.Z, P2.Z);  // Z2 Z_7
   sfe rho;
   if constexpr (C::GLV)
@@ -666,6 +676,7 @@ DEV sfe secp_build_table(const secp_pro& o, Tab& tab, bool& exc) {
     jac E;  // (X, W, zr)
     fe unused;
     tab.load_full(e, E, unused);
+    tab_sync(tab, 0);
     const sfe r2 = s_sqr<F>(rho);
     const sfe ax = s_mul<F>(s_unraw<F>(E.X), r2);
     const sfe aw = s_mul<F>(s_unraw<F>(E.Y), s_mul<F>(r2, rho));
