@@ -1,0 +1,97 @@
+"""Mixed batches above the sizes that run on four lanes per item (24,576 items): the bucketed launches with
+placed tiles and shared inversions. Items are drawn, with repetition, from a set of edge cases and corrupted
+generated ones, so every result is compared with the oracle's."""
+import numpy as np
+import pytest
+import torch
+
+import edge_cases
+import oracle_lib as O
+from sigops_pkg import sigops
+
+pytestmark = pytest.mark.gpu
+
+
+class Rows:
+    """distinct items: scheme, signature, digest or key, message, and the oracle's key and verdict (the status
+    of a secp item; for Ed25519 only whether it is 0)"""
+
+    def __init__(self):
+        rows = []
+        for curve in (0, 1):
+            cases = edge_cases.secp_cases(curve)
+            rows += [(curve, c[1], c[2], b"", e[1], e[0]) for c, e in
+                     zip(cases, edge_cases.secp_expected(curve, cases))]
+            s, d, _, _ = O.gen_secp(curve, 61, 200, corrupt_ppm=200000)
+            o, t = O.recover_batch(curve, s, d)
+            rows += [(curve, s[i].tobytes(), d[i].tobytes(), b"", o[i].tobytes(), int(t[i])) for i in range(200)]
+        cases = edge_cases.ed_cases()
+        rows += [(2, c[1], c[2], bytes(c[3]), bytes(64), 0 if e else 1) for c, e in
+                 zip(cases, edge_cases.ed_expected(cases))]
+        off = np.concatenate([[0], np.cumsum(np.arange(200) * 37 % 5200)]).astype(np.uint64)
+        s, k, m, _ = O.gen_ed25519(63, 200, off, corrupt_ppm=200000)
+        ok = O.verify_batch(s, k, m, off)
+        rows += [(2, s[i].tobytes(), k[i].tobytes(), m[int(off[i]):int(off[i + 1])].tobytes(), bytes(64),
+                  0 if ok[i] else 1) for i in range(200)]
+        col = [list(c) for c in zip(*rows)]
+        self.scheme = np.array(col[0], np.uint8)
+        self.sig, self.aux, self.out = (np.frombuffer(b"".join(col[j]), np.uint8).reshape(-1, w)
+                                        for j, w in ((1, 64), (2, 32), (4, 64)))
+        self.lens = np.array([len(x) for x in col[3]], np.int64)
+        self.begin = np.concatenate([[0], np.cumsum(self.lens)[:-1]])
+        self.msgs = np.frombuffer(b"".join(col[3]) + bytes(16), np.uint8)
+        self.verdict = np.array(col[5], np.uint8)
+
+    def draw(self, n, seed, longest=1 << 30):
+        """a batch of n items (messages of at most `longest` bytes): its arrays, and the rows they are"""
+        rng = np.random.default_rng(seed)
+        at = rng.choice(np.flatnonzero(self.lens <= longest), n)
+        lens = self.lens[at]
+        off = np.concatenate([[0], np.cumsum(lens)])
+        data = self.msgs[np.repeat(self.begin[at] - off[:-1], lens) + np.arange(off[-1])]
+        return (self.scheme[at], self.sig[at], self.aux[at], data, off.astype(np.uint64)), at
+
+    def check(self, at, out, st, what):
+        assert np.array_equal(out, self.out[at]), what
+        verdict = np.where(self.scheme[at] == 2, st != 0, st)
+        assert np.array_equal(verdict, self.verdict[at]), what
+
+
+@pytest.fixture(scope="module")
+def rows():
+    return Rows()
+
+
+def _on_device(batch):
+    sch, sig, aux, data, off = batch
+    data = np.concatenate([data, np.zeros(32 - len(data) % 16, np.uint8)])
+    n = len(sch)
+    return ([torch.from_numpy(np.ascontiguousarray(x)).cuda() for x in (sch, sig, aux, data, off.astype(np.int64))], n,
+            torch.zeros(n, 64, dtype=torch.uint8, device="cuda"), torch.full((n,), 0xEE, dtype=torch.uint8, device="cuda"))
+
+
+def _enqueue(ctx, dev, stream):
+    ins, n, out, st = dev
+    ctx.batch_dev(*[t.data_ptr() for t in ins], n, out.data_ptr(), st.data_ptr(), stream)
+
+
+def test_two_contexts_at_once(rows):
+    """batches of two contexts on two streams, together more than the GPU holds at a time: the workgroups of one
+    wait for the other's, and their first tiles go to the wavefronts that run"""
+    ctxs = [sigops.Context(), sigops.Context()]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    sizes = [(60000, 60011), (130000, 24576), (24577, 100003)]
+    drawn = [[rows.draw(n, 10 * k + j) for j, n in enumerate(pair)] for k, pair in enumerate(sizes)]
+    dev = [[_on_device(b) for b, _ in pair] for pair in drawn]
+    torch.cuda.synchronize()
+    print("two contexts", sizes, flush=True)
+    for _ in range(2):
+        for pair in dev:
+            for j in range(2):
+                _enqueue(ctxs[j], pair[j], streams[j].cuda_stream)
+    torch.cuda.synchronize()
+    for pair, d in zip(drawn, dev):
+        for (_, at), (_, n, out, st) in zip(pair, d):
+            rows.check(at, out.cpu().numpy(), st.cpu().numpy(), n)
+    for c in ctxs:
+        c.close()

@@ -14,12 +14,14 @@
 //   5. k_batch_careful finishes secp items whose fast ladder met an exceptional addition.
 // The batch's buffers and n are read from device memory (BatchIO), so the captured graph of these
 // launches replays for any buffers and any n up to the context capacity.
+#include "claims.hpp"
 #include "kern_quad.hpp"
 
 namespace sigops {
 
 static_assert(BATCH_QUAD_LANES == BATCH_QUAD_BLOCKS * 64 && BATCH_QUAD_TILE == QUAD_ITEMS,
               "kernels.hpp's launch shape of a small batch");
+static_assert(BATCH_FIRST_TILES == FIRST_TILES_MAX && (4 * NBUCKETS + 4) % 2 == 0, "claims as 64-bit words");
 
 constexpr u32 DUMMY = 0xFFFFFFFFu;
 
@@ -38,8 +40,8 @@ struct BatchArgs {
   u32* tile_start;  // [NB + 1] in processing order
   u32* bucket_of;   // [NB] processing rank -> bucket
   u32* order;       // padded item lists, bucket-major in processing order
-  u32* tile_counter;  // [2]: tiles beyond the launch's first, and chunks of 64 of the first looked over
-  u32* tile_taken;    // bit per first tile
+  u32* tile_counter;  // tiles taken beyond the launch's first
+  u32* tile_taken;    // bit per first tile (ClaimWave)
   u32* pend_list;
   u32* pend_count;
   const u8* rank;   // bucket -> processing rank
@@ -269,59 +271,35 @@ __global__ __launch_bounds__(256, SIGOPS_WAVES_PER_EU) void k_batch_finish(Batch
                             OrderItems{a}, a.sc);
 }
 
-// The tiles of a persistent launch, wavefront by wavefront. Workgroups of 4 wavefronts go round the
-// compute units, one wavefront to a SIMD, so wavefront w of each round of workgroups shares its SIMD
-// with wavefront w of the others. A wavefront's first tile is given by its place, odd rounds in reverse:
-// neighbours run the same code (they share the instruction cache), and as the tiles come longest first
-// (secp256r1), a launch of less than two rounds doubles up the SIMDs with the shortest tiles. A first
-// tile is claimed by its bit, so that those of workgroups which another kernel keeps from starting go to
-// the wavefronts that end (chunks of 64 tiles are looked over once); the tiles beyond come from a counter.
-// us, all tiles from one counter / so (mixed, messages up to 1 KB): 50,000 items 1,510 / 1,430, 80,000
-// 2,070 / 1,850, 100,003 2,180 / 1,820, 131,072 2,360 / 2,260, 300,000 5,000 / 4,630, 400,000 6,790 /
-// 6,720, 2^20 13,980 / 14,170: above four tiles per wavefront all come from the counter.
-struct TileClaims {
-  u32 ntiles, first_tiles, mine;
-  u64 found;  // first tiles of others this wavefront claimed: bits of chunk
-  u32 chunk;
-  bool look;
-  DEV explicit TileClaims(const BatchArgs& a) : ntiles(a.tile_start[NBUCKETS]), mine(DUMMY), found(0), chunk(0), look(true) {
-    first_tiles = a.cus && ntiles <= 16 * gridDim.x ? gridDim.x * 4 : 0;
-    if (first_tiles) {
-      const u32 round = 4 * a.cus, at = blockIdx.x * 4 + (threadIdx.x >> 6), r = at / round, w = at % round;
-      mine = r * round + ((r & 1) ? round - 1 - w : w);
-    }
-    first_tiles = first_tiles < ntiles ? first_tiles : ntiles;
+// a wavefront's view of the launch's tile claims (claims.hpp)
+struct ClaimWave {
+  u64* taken;    // bit per first tile
+  u32* counter;  // tiles taken beyond the first
+  u64 free;      // this lane's 64 first tiles as last seen: bits of those not taken
+  DEV explicit ClaimWave(const BatchArgs& a) : taken((u64*)a.tile_taken), counter(a.tile_counter), free(0) {}
+  DEV static u32 lane() { return threadIdx.x & 63u; }
+  DEV u64 take(u32 l, u32 b) { return atomicOr((unsigned long long*)taken + l, 1ull << b); }
+  DEV bool own(u32 t) { return __ballot(lane() == 0 && !((take(t >> 6, t & 63) >> (t & 63)) & 1u)) != 0; }
+  DEV void look(u32 n) {
+    const u32 l0 = 64 * lane();
+    const u64 in = n >= l0 + 64 ? ~0ull : (n > l0 ? ~0ull >> (64 - (n - l0)) : 0);
+    free = in ? ~__hip_atomic_load(taken + lane(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & in : 0;
   }
-  DEV static bool claim(const BatchArgs& a, u32 t) {
-    const u32 bit = 1u << (t & 31);
-    return !(a.tile_taken[t >> 5] & bit) && !(atomicOr(&a.tile_taken[t >> 5], bit) & bit);
+  DEV u64 words() const { return __ballot(free != 0); }
+  DEV u32 first(u32 l) const { return (u32)__builtin_amdgcn_readlane((int)__builtin_ctzll(free | (1ull << 63)), (int)l); }
+  DEV bool claim(u32 l, u32 b) {
+    bool won = false;
+    if (lane() == l) {
+      const u64 old = take(l, b);
+      won = !((old >> b) & 1u);
+      free &= ~(old | (1ull << b));
+    }
+    return __ballot(won) != 0;
   }
-  // the same on every lane; DUMMY when none is left
-  DEV u32 next(const BatchArgs& a) {
-    const u32 lane = threadIdx.x & 63u;
-    if (mine != DUMMY) {
-      const u32 t = __builtin_amdgcn_readfirstlane(mine);
-      mine = DUMMY;
-      if (t >= ntiles) return DUMMY;  // the rest is others' first tiles
-      if (__ballot(lane == 0 && claim(a, t))) return t;
-    }
-    while (look && found == 0) {
-      u32 c = 0;
-      if (lane == 0) c = atomicAdd(a.tile_counter + 1, 1u);
-      chunk = __shfl(c, 0);
-      look = chunk * 64 < first_tiles;
-      const u32 t = chunk * 64 + lane;
-      found = __ballot(look && t < first_tiles && claim(a, t));
-    }
-    if (found) {
-      const u32 t = chunk * 64 + (u32)__builtin_ctzll(found);
-      found &= found - 1;
-      return t;
-    }
+  DEV u32 beyond() {
     u32 t = 0;
-    if (lane == 0) t = first_tiles + atomicAdd(a.tile_counter, 1u);
-    t = __shfl(t, 0);
-    return t < ntiles ? t : DUMMY;
+    if (lane() == 0) t = atomicAdd(counter, 1u);
+    return __builtin_amdgcn_readfirstlane(t);
   }
 };
 
@@ -359,8 +337,10 @@ __global__ __launch_bounds__(256, WAVES) void k_batch_run(BatchArgs a, const uin
   ct.base = lane_tab;
   ct.slots = slots;
   ct.slot = slot;
-  TileClaims claims(a);
-  for (u32 t; (t = claims.next(a)) != DUMMY;) {
+  TileClaims claims(a.tile_start[NBUCKETS], a.cus, gridDim.x,
+                    __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6)));
+  ClaimWave wave(a);
+  for (u32 t; (t = claims.next(wave)) != NO_TILE;) {
     const u32 b = tile_bucket(a, t);
     for (u32 k = 0; k < a.tile_items; k += 64) {
       const u32 pos = t * a.tile_items + k + lane;
@@ -475,7 +455,7 @@ static BatchArgs batch_args(const BatchLaunch& L) {
   a.cursor = L.work + NBUCKETS;         // NBUCKETS
   a.tile_start = L.work + 2 * NBUCKETS;  // NBUCKETS + 1
   a.tile_counter = L.work + 3 * NBUCKETS + 1;
-  a.pend_count = L.work + 3 * NBUCKETS + 3;
+  a.pend_count = L.work + 3 * NBUCKETS + 2;
   a.bucket_of = L.work + 3 * NBUCKETS + 4;
   a.tile_taken = L.work + 4 * NBUCKETS + 4;
   a.pend_list = L.pend_list;

@@ -78,7 +78,7 @@ constexpr uint32_t BUCKET_K1 = 0, BUCKET_R1 = 1, BUCKET_ED0 = 2;
 constexpr uint32_t ED_BINS = 40;  // Ed25519 buckets by SHA-512 block count 1..40 (40 = "40 or more")
 constexpr uint32_t NBUCKETS = 2 + ED_BINS;
 constexpr uint32_t BATCH_FIRST_TILES = 4096;  // bits of the first tiles' claims: 1,024 workgroups
-// counts, cursors, tile starts, tile ctrs, pending ctr, buckets, claims
+// counts, cursors, tile starts, tile ctr, pending ctr, (one unused, to align the claims), buckets, claims
 constexpr uint32_t BATCH_WORK_WORDS = 4 * NBUCKETS + 4 + BATCH_FIRST_TILES / 32;
 constexpr uint32_t MAX_TILE_ROUNDS = 4;
 
