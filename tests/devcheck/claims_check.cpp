@@ -44,9 +44,11 @@ struct Wave {
 };
 }  // namespace
 
-// room: workgroups that may run at a time until `until`, all of them afterwards. A tile takes 100 time
-// units and a little that depends on it. done: how often each tile was run. Returns the time of the last.
-extern "C" long tc_run(u32 ntiles, u32 cus, u32 workgroups, u32 room, long until, unsigned* done) {
+// room: workgroups that may run at a time until `until`, all of them afterwards; the first `slow` ones run at
+// a tenth of the others' speed (their SIMDs are in use) and reach their first tile 5 time units later. A tile
+// takes 100 time units and a little that depends on it. done: how often each tile was run. Returns the time
+// of the last.
+extern "C" long tc_run(u32 ntiles, u32 cus, u32 workgroups, u32 room, long until, u32 slow, unsigned* done) {
   Launch m;
   std::vector<TileClaims> claims;
   std::vector<u32> running(workgroups, 4);
@@ -57,7 +59,7 @@ extern "C" long tc_run(u32 ntiles, u32 cus, u32 workgroups, u32 room, long until
   long end = 0;
   auto start = [&](long t) {
     while (started < workgroups && (resident < room || t >= until)) {
-      for (u32 k = 0; k < 4; k++) q.push(ev(t, 4 * started + k));
+      for (u32 k = 0; k < 4; k++) q.push(ev(started < slow ? t + 5 : t, 4 * started + k));
       started++;
       resident++;
     }
@@ -82,7 +84,7 @@ extern "C" long tc_run(u32 ntiles, u32 cus, u32 workgroups, u32 room, long until
     }
     if (tile >= ntiles) return -1;
     done[tile]++;
-    const long e = t + 100 + (tile * 7919u) % 13;
+    const long e = t + (100 + (tile * 7919u) % 13) * (w / 4 < slow ? 10 : 1);
     end = e > end ? e : end;
     q.push(ev(e, w));
   }

@@ -95,3 +95,22 @@ def test_two_contexts_at_once(rows):
             rows.check(at, out.cpu().numpy(), st.cpu().numpy(), n)
     for c in ctxs:
         c.close()
+
+
+def test_sizes_where_the_launch_changes(rows):
+    """around the sizes where a batch goes from four lanes per item to one, from tiles by counter to tiles by
+    place, and to shared inversions; host calls copied, and the largest two on the device"""
+    ctx = sigops.Context()
+    ctx.set_streaming(False)
+    for n in (20480, 20481, 32768, 33011, 65536, 65537, 131072):
+        print(f"mixed n={n}", flush=True)
+        batch, at = rows.draw(n, n)
+        rows.check(at, *ctx.batch(*batch), n)
+    for n in (786431, 786432):
+        print(f"mixed n={n}", flush=True)
+        batch, at = rows.draw(n, n, longest=300)
+        dev = _on_device(batch)
+        _enqueue(ctx, dev, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        rows.check(at, dev[2].cpu().numpy(), dev[3].cpu().numpy(), n)
+    ctx.close()

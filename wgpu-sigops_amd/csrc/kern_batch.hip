@@ -6,12 +6,13 @@
 //      Ed25519 by SHA-512 block count, so the lanes of a wavefront hash equally long messages), each
 //      scheme padded to whole tiles; the buckets are processed in the context's order (its rank
 //      table: secp256r1, secp256k1, then Ed25519 by decreasing block count);
-//   2. k_batch_scalars computes u1 and u2 of the secp items, several per lane with one inversion;
-//   3. k_batch_run is persistent: every wavefront pulls the next tile (64 x tile_rounds items of
-//      one scheme) from an atomic counter, so the scheme is uniform across the wavefront and load
-//      balances dynamically; it runs the same per-item code as the plain kernels;
-//   4. k_batch_finish makes the recovered keys affine, again several per lane with one inversion;
-//   5. k_batch_careful finishes secp items whose fast ladder met an exceptional addition.
+//   2. k_batch_run is persistent: every wavefront takes tiles (64 x tile_rounds items of one scheme,
+//      claims.hpp), so the scheme is uniform across the wavefront and load balances dynamically; it
+//      runs the same per-item code as the plain kernels;
+//   3. k_batch_careful finishes secp items whose fast ladder met an exceptional addition.
+// A large batch (BATCH_SHARED_FROM) shares its inversions between items: k_batch_scalars computes u1 and
+// u2 of the secp items before k_batch_run, several per lane with one inversion, and k_batch_finish makes
+// the recovered keys affine after it in the same way. A small one runs on four lanes per item.
 // The batch's buffers and n are read from device memory (BatchIO), so the captured graph of these
 // launches replays for any buffers and any n up to the context capacity.
 #include "claims.hpp"
@@ -219,12 +220,21 @@ DEV void store16(uint4* p, const u32 o[16]) {
   for (int c = 0; c < 4; c++) p[c] = make_uint4(o[4 * c], o[4 * c + 1], o[4 * c + 2], o[4 * c + 3]);
 }
 
-// a secp item up to its Jacobian result in the scratch (k_batch_finish makes it affine)
-template <class C>
+// a secp item; SHARED: up to its Jacobian result in the scratch (k_batch_finish makes it affine)
+template <class C, bool SHARED>
 DEV void batch_secp_item(const BatchArgs& a, u32 i, u32 pos, STabDev& tab, const CombDev& comb) {
-  u32 sr[16];
+  u32 sr[16], st;
   load_words(a.sigs + 4 * (u64)i, sr, 4);
-  if (secp_recover_point<C>(sr, pos, a.sc, tab, comb) == ST_PENDING) a.pend_list[atomicAdd(a.pend_count, 1u)] = i;
+  if constexpr (SHARED) {
+    st = secp_recover_point<C>(sr, pos, a.sc, tab, comb);
+  } else {
+    u32 dr[8], o[16];
+    load_words(a.aux + 2 * (u64)i, dr, 2);
+    st = secp_item<C>(sr, dr, tab, comb, o);
+    store16(a.out + 4 * (u64)i, o);
+    a.status[i] = (u8)st;
+  }
+  if (st == ST_PENDING) a.pend_list[atomicAdd(a.pend_count, 1u)] = i;
 }
 
 // the positions of one curve's tiles as items of the stages around the persistent kernel
@@ -313,8 +323,8 @@ constexpr u32 RUN_MIXED = RUN_K1 | RUN_R1 | RUN_ED;
 // WAVES: waves per SIMD the kernel is built for, which sets its register budget per lane (512 /
 // WAVES): 2 by default (256 registers, some values spilled to scratch memory); 1 lets the
 // compiler keep them in registers (accumulation registers included) with half the waves to hide
-// latencies. The autotuner measures them.
-template <u32 MASK, int WAVES = SIGOPS_WAVES_PER_EU>
+// latencies. The autotuner measures them. SHARED: between k_batch_scalars and k_batch_finish.
+template <u32 MASK, int WAVES = SIGOPS_WAVES_PER_EU, bool SHARED = false>
 __global__ __launch_bounds__(256, WAVES) void k_batch_run(BatchArgs a, const uint4* __restrict__ comb_k1,
                                                    const uint4* __restrict__ comb_r1,
                                                    const uint4* __restrict__ comb_ed, const uint4* __restrict__ gb,
@@ -347,9 +357,9 @@ __global__ __launch_bounds__(256, WAVES) void k_batch_run(BatchArgs a, const uin
       const u32 i = a.order[pos];
       if (i == DUMMY) continue;
       if (K1 && b == BUCKET_K1) {
-        if constexpr (K1) batch_secp_item<CurveK1>(a, i, pos, jt, CombDev{comb_k1});
+        if constexpr (K1) batch_secp_item<CurveK1, SHARED>(a, i, pos, jt, CombDev{comb_k1});
       } else if (R1 && b == BUCKET_R1) {
-        if constexpr (R1) batch_secp_item<CurveR1>(a, i, pos, jt, CombDev{comb_r1});
+        if constexpr (R1) batch_secp_item<CurveR1, SHARED>(a, i, pos, jt, CombDev{comb_r1});
       } else if constexpr (ED) {
         // the challenge is hashed here, inside the persistent kernel: the tile's items have equal
         // SHA-512 block counts (bucketed), and the hash's memory latency hides behind the other
@@ -502,7 +512,7 @@ hipError_t launch_batch_small(const BatchLaunch& L, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_batch(const BatchLaunch& L, hipStream_t s) {
+hipError_t launch_batch(const BatchLaunch& L, bool shared, hipStream_t s) {
   const BatchArgs a = batch_args(L);
   // stage events exist only on the eager (timed) path, never under graph capture
   auto mark = [&](int i) -> hipError_t { return L.stage_ev ? hipEventRecord(L.stage_ev[i], s) : hipSuccess; };
@@ -517,11 +527,13 @@ hipError_t launch_batch(const BatchLaunch& L, hipStream_t s) {
   // (the Ed25519 challenges are hashed inside k_batch_run; the stage stays empty, so that the
   // stage indices of earlier measurements keep their meaning)
   if ((e = mark(2)) != hipSuccess) return e;
-  k_batch_scalars<<<L.stage_grid, 256, 0, s>>>(a);
-  const auto run = L.waves == 1 ? k_batch_run<RUN_MIXED, 1> : k_batch_run<RUN_MIXED>;
+  if (shared) k_batch_scalars<<<L.stage_grid, 256, 0, s>>>(a);
+  const auto run = !shared        ? k_batch_run<RUN_MIXED>
+                   : L.waves == 1 ? k_batch_run<RUN_MIXED, 1, true>
+                                  : k_batch_run<RUN_MIXED, SIGOPS_WAVES_PER_EU, true>;
   run<<<L.grid, 256, 0, s>>>(a, (const uint4*)L.comb_k1, (const uint4*)L.comb_r1, (const uint4*)L.comb_ed,
                              (const uint4*)L.gb, (uint4*)L.lane_tab, L.slots);
-  k_batch_finish<<<L.stage_grid, 256, 0, s>>>(a);
+  if (shared) k_batch_finish<<<L.stage_grid, 256, 0, s>>>(a);
   if ((e = mark(3)) != hipSuccess) return e;
   k_batch_careful<<<64, 64, 0, s>>>(a, (const uint4*)L.gk1, (const uint4*)L.gr1);
   if ((e = mark(4)) != hipSuccess) return e;

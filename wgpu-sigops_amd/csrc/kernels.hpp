@@ -116,15 +116,27 @@ struct BatchLaunch {
   void* lane_tab;
   uint32_t slots, grid, aux_grid, tile_rounds;
   uint32_t stage_grid;   // compute units: blocks of the stages that share an inversion between items
-  uint32_t waves;        // mixed batch: waves per SIMD the persistent kernel is built for (1 or 2)
+  uint32_t waves;        // mixed batch: waves per SIMD the persistent kernel is built for (1 or 2); 1: shared only
   hipEvent_t* stage_ev;  // null, or 5 events recorded before, between and after the 4 stages
 };
 
-hipError_t launch_batch(const BatchLaunch& L, hipStream_t s);
+// shared: the secp items' inversions are shared between items, in a stage before and one after the
+// persistent kernel
+hipError_t launch_batch(const BatchLaunch& L, bool shared, hipStream_t s);
+// Batches from this size on share their inversions. A lane of the stages takes n / 65,536 items, and what
+// that saves has to pay for two launches: each waits for the GPU to drain, and beside other batches for
+// wavefronts to end. us per batch (messages up to 4 KB), shared / not: alone 1,371 / 1,294 at 20,000 items,
+// 1,744 / 1,572 at 65,536, 2,502 / 2,323 at 131,072, 4,174 / 4,138 at 262,144, 7,915 / 7,533 at 524,288,
+// 11,464 / 11,195 at 800,000, 13,801 / 14,451 at 2^20; on three streams at once 786 / 499, 1,029 / 890,
+// 1,862 / 1,722, 3,717 / 3,386, 6,949 / 6,718, 10,383 / 10,272, 13,362 / 13,507.
+constexpr uint32_t BATCH_SHARED_FROM = 13u << 16;
 // A small mixed batch: four lanes per item, one workgroup per tile of 16 items of one bucket. Measured
-// (us per device call, four lanes against one lane per item, messages up to 4 KB): 684 / 1,650 at 1,000
-// items, 711 / 1,650 at 8,000, 1,181 / 1,650 at 16,384, 1,466 / 1,482 at 24,576.
-constexpr uint32_t BATCH_QUAD_MAX_ITEMS = 24576;
+// (us per device call, four lanes against one lane per item, messages up to 4 KB): 690 / 1,303 at 2,000
+// items, 705 / 1,325 at 8,000, 1,182 / 1,326 at 16,000, 1,200 / 1,337 at 20,000, 1,451 / 1,364 at 24,000.
+constexpr uint32_t BATCH_QUAD_MAX_ITEMS = 20480;
+// The same beside other batches, which four lanes per item take more of the GPU from: per batch on three
+// streams 363 / 453 at 6,000, 409 / 469 at 10,000, 463 / 475 at 12,000, 534 / 477 at 14,000, 751 / 493 at 20,000.
+constexpr uint32_t BATCH_QUAD_MAX_BESIDE = 12288;
 constexpr uint32_t BATCH_QUAD_TILE = 16;
 constexpr uint32_t BATCH_QUAD_BLOCKS = BATCH_QUAD_MAX_ITEMS / BATCH_QUAD_TILE + NBUCKETS;
 constexpr uint32_t BATCH_QUAD_LANES = BATCH_QUAD_BLOCKS * 64;  // point lanes
@@ -235,4 +247,6 @@ hipError_t launch_gen_ed25519(uint64_t seed, uint32_t n, uint32_t ppm, const voi
 // error code
 struct sigops_ctx;
 int sigops_ring_resources(sigops_ctx* c, sigops::RingResources* r);
+// whether the next mixed batches on this context run beside others (a server's other slots)
+void sigops_set_beside(sigops_ctx* c, bool beside);
 

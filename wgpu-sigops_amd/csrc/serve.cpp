@@ -151,10 +151,11 @@ struct sigops_server {
 
   void dispatch_loop();
   void complete_loop();
-  int launch(Slot* s);
+  int launch(Slot* s, bool beside);
 };
 
-int sigops_server::launch(Slot* s) {
+// beside: batches of other slots are in flight
+int sigops_server::launch(Slot* s, bool beside) {
   // pack the slot's requests into pinned staging, then enqueue H2D, the batch and D2H on its stream
   size_t n = 0, msg = 0;
   for (auto& r : s->reqs) {
@@ -208,6 +209,7 @@ int sigops_server::launch(Slot* s) {
       hipMemcpyAsync(s->d_msg.p, s->h_msg.p, m0 + 16, hipMemcpyHostToDevice, st) != hipSuccess ||
       hipMemcpyAsync(s->d_off.p, s->h_off.p, (n + 1) * 8, hipMemcpyHostToDevice, st) != hipSuccess)
     return SIGOPS_E_DEVICE;
+  sigops_set_beside(s->ctx, beside);
   int rc = sigops_batch_dev(s->ctx, s->d_sch.p, s->d_sig.p, s->d_aux.p, s->d_msg.p, s->d_off.p, n, s->d_out.p,
                             s->d_st.p, st);
   if (rc) return rc;
@@ -247,8 +249,9 @@ void sigops_server::dispatch_loop() {
       s->reqs.push_back(r);
       queue.pop_front();
     }
+    const bool beside = !inflight.empty();
     lk.unlock();
-    const int rc = launch(s);
+    const int rc = launch(s, beside);
     lk.lock();
     if (rc) {
       // the requests fail with the error; the slot returns to the pool

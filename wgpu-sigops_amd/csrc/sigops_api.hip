@@ -144,7 +144,9 @@ struct sigops_ctx {
   // the captured mixed-batch launches; they read the call's buffers from d_io, so one graph serves
   // every call on this context
   hipGraphExec_t graph = nullptr;
-  hipGraphExec_t graph_small = nullptr;  // batches of at most BATCH_QUAD_MAX_ITEMS
+  hipGraphExec_t graph_small = nullptr;   // launch_batch_small
+  hipGraphExec_t graph_shared = nullptr;  // launch_batch with shared inversions
+  bool beside = false;                    // sigops_set_beside
   DevBuf in, aux, msg, off, out, st, sch;
   uint32_t fault = 0;  // SIGOPS_FAULT_* test switch
   // streamed host batches (stream_host.hpp): one pinned, device-mapped block carved into the
@@ -507,6 +509,7 @@ void sigops_destroy(sigops_ctx* c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   if (c->graph) (void)hipGraphExecDestroy(c->graph);
   if (c->graph_small) (void)hipGraphExecDestroy(c->graph_small);
+  if (c->graph_shared) (void)hipGraphExecDestroy(c->graph_shared);
   if (c->s_ev) (void)hipEventDestroy(c->s_ev);
   for (hipEvent_t e : c->s_tev)
     if (e) (void)hipEventDestroy(e);
@@ -782,24 +785,28 @@ int sigops_batch_dev(sigops_ctx* c, const void* d_schemes, const void* d_sigs, c
   L.stage_ev = nullptr;
   // a small batch needs lane tables for every lane of its launch (a context of one block per CU on a
   // device with fewer CUs may not have them)
-  const bool small = n <= sigops::BATCH_QUAD_MAX_ITEMS && c->slots >= sigops::BATCH_QUAD_LANES;
-  const auto launch = small ? sigops::launch_batch_small : sigops::launch_batch;
+  const bool small = n <= (c->beside ? sigops::BATCH_QUAD_MAX_BESIDE : sigops::BATCH_QUAD_MAX_ITEMS) &&
+                     c->slots >= sigops::BATCH_QUAD_LANES;
+  const bool shared = !small && (n >= sigops::BATCH_SHARED_FROM || c->waves == 1);
+  auto launch = [&](hipStream_t on) {
+    return small ? sigops::launch_batch_small(L, on) : sigops::launch_batch(L, shared, on);
+  };
   if (c->stage_timing) {
     L.stage_ev = c->stage_ev;
-    HIPCHK(c, launch(L, s));
+    HIPCHK(c, launch(s));
     c->stage_recorded = true;
     return SIGOPS_OK;
   }
   if (!c->use_graph) {
-    HIPCHK(c, launch(L, s));
+    HIPCHK(c, launch(s));
     return SIGOPS_OK;
   }
-  hipGraphExec_t& graph = small ? c->graph_small : c->graph;
+  hipGraphExec_t& graph = small ? c->graph_small : (shared ? c->graph_shared : c->graph);
   if (!graph) {
     L.aux_grid = c->grid;  // the graph does not depend on n
     hipGraph_t g;
     HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    hipError_t le = launch(L, c->stream);
+    hipError_t le = launch(c->stream);
     hipError_t ce = hipStreamEndCapture(c->stream, &g);
     if (le != hipSuccess) return hip_fail(c, le, "launch_batch under capture");
     if (ce != hipSuccess) return hip_fail(c, ce, "hipStreamEndCapture");
@@ -1141,6 +1148,8 @@ int batch_streamed(sigops_ctx* c, const uint8_t* schemes, const uint8_t* sigs, c
 }
 
 }  // namespace
+
+void sigops_set_beside(sigops_ctx* c, bool beside) { c->beside = beside; }
 
 int sigops_ring_resources(sigops_ctx* c, sigops::RingResources* r) {
   if (!c || !r) return SIGOPS_E_ARG;
