@@ -62,6 +62,36 @@ def rows():
     return Rows()
 
 
+def test_plain_calls_where_inversions_are_shared():
+    """plain recoveries and verifications around the size from which they share inversions between items
+    (three and four items to a lane), edge cases and corrupted items among the shared ones"""
+    ctx = sigops.Context()
+    for curve in (0, 1):
+        cases = edge_cases.secp_cases(curve)
+        exp = edge_cases.secp_expected(curve, cases)
+        s, d, p, _ = O.gen_secp(curve, 71, 300, corrupt_ppm=200000)
+        o, t = O.recover_batch(curve, s, d)
+        sigs = np.concatenate([np.frombuffer(b"".join(c[1] for c in cases), np.uint8).reshape(-1, 64), s])
+        digs = np.concatenate([np.frombuffer(b"".join(c[2] for c in cases), np.uint8).reshape(-1, 32), d])
+        out = np.concatenate([np.frombuffer(b"".join(e[1] for e in exp), np.uint8).reshape(-1, 64), o])
+        st = np.concatenate([np.array([e[0] for e in exp], np.uint8), t])
+        vcases = edge_cases.secp_verify_cases(curve)
+        vst = np.concatenate([np.array(edge_cases.secp_verify_expected(curve, vcases), np.uint8),
+                              O.secp_verify_batch(curve, s, d, p)])
+        vsigs = np.concatenate([np.frombuffer(b"".join(c[1] for c in vcases), np.uint8).reshape(-1, 64), s])
+        vdigs = np.concatenate([np.frombuffer(b"".join(c[2] for c in vcases), np.uint8).reshape(-1, 32), d])
+        vpubs = np.concatenate([np.frombuffer(b"".join(c[3] for c in vcases), np.uint8).reshape(-1, 64), p])
+        for n in (131072, 196607, 196608, 200003):
+            print(f"shared inversions curve={curve} n={n}", flush=True)
+            at = np.random.default_rng(n).integers(0, len(st), n)
+            got, gst = (ctx.secp256k1_recover if curve == 0 else ctx.secp256r1_recover)(sigs[at], digs[at])
+            assert np.array_equal(gst, st[at]) and np.array_equal(got, out[at]), n
+            at = np.random.default_rng(n).integers(0, len(vst), n)
+            _, gst = (ctx.secp256k1_verify if curve == 0 else ctx.secp256r1_verify)(vsigs[at], vdigs[at], vpubs[at])
+            assert np.array_equal(gst, vst[at]), n
+    ctx.close()
+
+
 def _on_device(batch):
     sch, sig, aux, data, off = batch
     data = np.concatenate([data, np.zeros(32 - len(data) % 16, np.uint8)])

@@ -12,7 +12,6 @@ namespace sigops {
 
 static constexpr int CURVE_ID = std::is_same<SIGOPS_CURVE, CurveK1>::value ? 0 : 1;
 
-// lanes of the stages that share an inversion: one per item up to STAGE_LANES
 static u32 stage_blocks(u32 n) { return ((n < STAGE_LANES ? n : STAGE_LANES) + 255) / 256; }
 
 hipError_t SIGOPS_CAT(launch_secp_recover_, SIGOPS_CURVE)(const SecpLaunch& L, const void* sigs, const void* digs,
@@ -30,11 +29,14 @@ hipError_t SIGOPS_CAT(launch_secp_recover_, SIGOPS_CURVE)(const SecpLaunch& L, c
                                                   (const uint4*)L.gtab8, (uint4*)L.lane_tab, L.slots, L.pend_list,
                                                   L.pend_count);
   } else {
+    const bool shared = n >= SECP_SHARED_FROM;
     const ItemScratch sc{(uint4*)L.scratch, L.scratch_stride};
-    k_secp_scalars<SIGOPS_CURVE, false><<<stage_blocks(n), 256, 0, s>>>((const uint4*)sigs, (const uint4*)digs, n, sc);
-    k_secp_points<SIGOPS_CURVE><<<g, 256, 0, s>>>((const uint4*)sigs, n, sc, (const uint4*)L.comb, (uint4*)L.lane_tab,
-                                                 L.slots, L.pend_list, L.pend_count);
-    k_secp_finish<SIGOPS_CURVE><<<stage_blocks(n), 256, 0, s>>>((uint4*)out, (u8*)status, n, sc);
+    if (shared)
+      k_secp_scalars<SIGOPS_CURVE, false><<<stage_blocks(n), 256, 0, s>>>((const uint4*)sigs, (const uint4*)digs, n, sc);
+    const auto points = shared ? k_secp_points<SIGOPS_CURVE, true> : k_secp_points<SIGOPS_CURVE, false>;
+    points<<<g, 256, 0, s>>>((const uint4*)sigs, (const uint4*)digs, (uint4*)out, (u8*)status, n, sc,
+                             (const uint4*)L.comb, (uint4*)L.lane_tab, L.slots, L.pend_list, L.pend_count);
+    if (shared) k_secp_finish<SIGOPS_CURVE><<<stage_blocks(n), 256, 0, s>>>((uint4*)out, (u8*)status, n, sc);
   }
   k_secp_careful<SIGOPS_CURVE><<<64, 64, 0, s>>>((const uint4*)sigs, (const uint4*)digs, (uint4*)out, (u8*)status,
                                                 (const uint4*)(L.gtab8 ? L.gtab8 : L.gtab), L.pend_list, L.pend_count);
@@ -50,12 +52,14 @@ hipError_t SIGOPS_CAT(launch_secp_verify_, SIGOPS_CURVE)(const SecpLaunch& L, co
     const hipError_t e = launch_quad_secp(CURVE_ID, true, L, sigs, digs, pubs, nullptr, status, n, s);
     if (e != hipSuccess) return e;
   } else {
-  const ItemScratch sc{(uint4*)L.scratch, L.scratch_stride};
-  k_fill_u32<<<1, 64, 0, s>>>(L.pend_count, 0u, 1u);
-  k_secp_scalars<SIGOPS_CURVE, true><<<stage_blocks(n), 256, 0, s>>>((const uint4*)sigs, (const uint4*)digs, n, sc);
-  k_secp_verify<SIGOPS_CURVE><<<g, 256, 0, s>>>((const uint4*)sigs, (const uint4*)pubs, (u8*)status, n, sc,
-                                               (const uint4*)L.comb, (uint4*)L.lane_tab, L.slots, L.pend_list,
-                                               L.pend_count);
+    const bool shared = n >= SECP_SHARED_FROM;
+    const ItemScratch sc{(uint4*)L.scratch, L.scratch_stride};
+    k_fill_u32<<<1, 64, 0, s>>>(L.pend_count, 0u, 1u);
+    if (shared)
+      k_secp_scalars<SIGOPS_CURVE, true><<<stage_blocks(n), 256, 0, s>>>((const uint4*)sigs, (const uint4*)digs, n, sc);
+    const auto verify = shared ? k_secp_verify<SIGOPS_CURVE, true> : k_secp_verify<SIGOPS_CURVE, false>;
+    verify<<<g, 256, 0, s>>>((const uint4*)sigs, (const uint4*)digs, (const uint4*)pubs, (u8*)status, n, sc,
+                             (const uint4*)L.comb, (uint4*)L.lane_tab, L.slots, L.pend_list, L.pend_count);
   }
   k_secp_verify_careful<SIGOPS_CURVE><<<64, 64, 0, s>>>((const uint4*)sigs, (const uint4*)digs, (const uint4*)pubs,
                                                        (u8*)status, (const uint4*)L.gtab, L.pend_list, L.pend_count);

@@ -46,8 +46,16 @@ hipError_t launch_secp_verify_CurveR1(const SecpLaunch& L, const void* sigs, con
 // most one per SIMD, and the call is as long as one item. Measured (us per device call, four lanes
 // against one lane per item): secp256k1 recovery 473 / 807 at 1,000 items, 551 / 812 at 16,384, 1,015
 // / 812 at 20,011; secp256r1 verification 563 / 1,140, 656 / 1,148, 1,255 / 1,148; Ed25519 with
-// messages up to 200 bytes 320 / 990, 543 / 1,000 (one lane per item with its bucketing).
+// messages up to 200 bytes 320 / 990, 543 / 1,000 (one lane per item with its bucketing). Beside other calls
+// four lanes take more of the GPU: on three streams secp256r1 recovery 386 us a call at 6,000 items, 598 at
+// 12,000 and 808 at 16,384, one lane per item 651 at each; the line is for calls alone.
 constexpr uint32_t QUAD_MAX_ITEMS = 16384;
+// Plain secp calls from this size on share their inversions between items, in a stage before and one after
+// the ladders (65,536 lanes; below that a lane has one item and shares nothing). us per call, shared / not:
+// secp256r1 recovery alone 1,282 / 1,245 at 20,011 items, 1,312 / 1,273 at 65,536, 2,284 / 2,278 at 131,072,
+// 9,089 / 9,196 at 524,288; secp256k1 3,077 / 3,165 at 200,000, 5,912 / 6,104 at 524,288. On three streams
+// secp256r1 852 / 654 at 20,011, 2,094 / 2,115 at 131,072, 3,302 / 3,370 at 200,000.
+constexpr uint32_t SECP_SHARED_FROM = 3u << 16;
 // the counters that keep point waves apart (kern_quad.hpp, QuadRole), zero at first
 constexpr uint32_t QUAD_LOAD_WORDS = 16 * 256 * 4;
 // pend_count is cleared; the careful pass is the caller's (launch_secp_*_careful)

@@ -345,6 +345,36 @@ DEV void secp_scalars_lane(u32 first, u32 step, u32 end, const Src& src, const I
   }
 }
 
+// u1 G + u2 P on the wide tables
+template <class C>
+DEV jac secp_ladder_wide(const secp_pro& pro, STabDev& tab, const CombDev& comb, bool& exc) {
+  const jacs Q = secp_ladder_s<C, 0>(pro, tab, comb, exc);
+  return s_to_jac<C>(secp_comb<C>(Q, pro, comb, exc));
+}
+
+// one recovery by itself, its inversions not shared: the status (ST_PENDING when the ladder met an
+// exceptional addition and the careful pass must redo the item) and the key X || Y (zeros unless
+// ST_OK)
+template <class C>
+DEV u32 secp_item(const u32 sr[16], const u32 dr[8], STabDev& tab, const CombDev& comb, u32 o[16]) {
+  secp_pro pro;
+  secp_prologue<C, true>(sr, dr, pro);
+  u32 st = pro.status;
+  if (st == ST_OK) {
+    bool exc = false;
+    const jac Q = secp_ladder_wide<C>(pro, tab, comb, exc);
+    if (exc)
+      st = ST_PENDING;
+    else
+      secp_output<C>(Q, o);
+  }
+  if (st != ST_OK) {
+#pragma unroll
+    for (int k = 0; k < 16; k++) o[k] = 0;
+  }
+  return st;
+}
+
 // Q = u1 G + u2 P of position p (u1, u2 from secp_scalars_lane)
 template <class C>
 DEV jac secp_point(u32 p, const fe& x, const fe& y, const ItemScratch& sc, STabDev& tab, const CombDev& comb,
@@ -358,8 +388,7 @@ DEV jac secp_point(u32 p, const fe& x, const fe& y, const ItemScratch& sc, STabD
     pro.u2[k] = w[8 + k];
   }
   secp_carriers<C, true>(pro, x, y);
-  const jacs Q = secp_ladder_s<C, 0>(pro, tab, comb, exc);
-  return s_to_jac<C>(secp_comb<C>(Q, pro, comb, exc));
+  return secp_ladder_wide<C>(pro, tab, comb, exc);
 }
 
 // the recovery at position p up to its Jacobian result, left in the scratch with the status
@@ -479,12 +508,12 @@ __global__ __launch_bounds__(256, SIGOPS_WAVES_PER_EU) void k_secp_finish(uint4*
                       PlainItems{nullptr, nullptr, out, status}, sc);
 }
 
-template <class C>
-__global__ __launch_bounds__(256, SIGOPS_WAVES_PER_EU) void k_secp_points(const uint4* __restrict__ sigs, u32 n,
-                                                                     ItemScratch sc, const uint4* __restrict__ comb,
-                                                                     uint4* __restrict__ rtab, u32 slots,
-                                                                     u32* __restrict__ pend_list,
-                                                                     u32* __restrict__ pend_count) {
+// SHARED: between k_secp_scalars and k_secp_finish, up to the Jacobian result; else the whole recovery
+template <class C, bool SHARED>
+__global__ __launch_bounds__(256, SIGOPS_WAVES_PER_EU) void k_secp_points(
+    const uint4* __restrict__ sigs, const uint4* __restrict__ digs, uint4* __restrict__ out, u8* __restrict__ status,
+    u32 n, ItemScratch sc, const uint4* __restrict__ comb, uint4* __restrict__ rtab, u32 slots,
+    u32* __restrict__ pend_list, u32* __restrict__ pend_count) {
   const u32 slot = blockIdx.x * blockDim.x + threadIdx.x;
   STabDev tab;
   tab.base = rtab;
@@ -492,20 +521,33 @@ __global__ __launch_bounds__(256, SIGOPS_WAVES_PER_EU) void k_secp_points(const 
   tab.slot = slot;
   const u32 stride = gridDim.x * blockDim.x;
   for (u32 i = slot; i < n; i += stride) {
-    u32 sr[16];
+    u32 sr[16], st;
     load_words(sigs + 4 * (u64)i, sr, 4);
-    if (secp_recover_point<C>(sr, i, sc, tab, CombDev{comb}) == ST_PENDING) pend_list[atomicAdd(pend_count, 1u)] = i;
+    if constexpr (SHARED) {
+      st = secp_recover_point<C>(sr, i, sc, tab, CombDev{comb});
+    } else {
+      u32 dr[8], o[16];
+      load_words(digs + 2 * (u64)i, dr, 2);
+      st = secp_item<C>(sr, dr, tab, CombDev{comb}, o);
+#pragma unroll
+      for (int c = 0; c < 4; c++) out[4 * (u64)i + c] = make_uint4(o[4 * c], o[4 * c + 1], o[4 * c + 2], o[4 * c + 3]);
+      status[i] = (u8)st;
+    }
+    if (st == ST_PENDING) pend_list[atomicAdd(pend_count, 1u)] = i;
   }
 }
 
-// ECDSA verification with a known key (fuel Signature::verify) after k_secp_scalars: the ladder with
-// the key in place of R and the projective x comparison in place of the affine output. Lanes that
-// meet an exceptional addition are finished by k_secp_verify_careful.
-template <class C>
-__global__ __launch_bounds__(256, SIGOPS_WAVES_PER_EU) void k_secp_verify(
-    const uint4* __restrict__ sigs, const uint4* __restrict__ pubs, u8* __restrict__ status, u32 n, ItemScratch sc,
-    const uint4* __restrict__ comb, uint4* __restrict__ rtab, u32 slots, u32* __restrict__ pend_list,
-    u32* __restrict__ pend_count) {
+// ECDSA verification with a known key (fuel Signature::verify): the ladder with the key in place of R
+// and the projective x comparison in place of the affine output. Lanes that meet an exceptional
+// addition are finished by k_secp_verify_careful. SHARED: after k_secp_scalars.
+// At most 2 wavefronts per SIMD: it needs 157-163 registers, and launches on three streams, whose
+// workgroups the dispatcher puts on the same compute units while they fit, met three to a SIMD
+// (20,011 items each: 2,964 us together, 2,080 so).
+template <class C, bool SHARED>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_secp_verify(
+    const uint4* __restrict__ sigs, const uint4* __restrict__ digs, const uint4* __restrict__ pubs,
+    u8* __restrict__ status, u32 n, ItemScratch sc, const uint4* __restrict__ comb, uint4* __restrict__ rtab, u32 slots,
+    u32* __restrict__ pend_list, u32* __restrict__ pend_count) {
   const u32 slot = blockIdx.x * blockDim.x + threadIdx.x;
   STabDev tab;
   tab.base = rtab;
@@ -516,12 +558,25 @@ __global__ __launch_bounds__(256, SIGOPS_WAVES_PER_EU) void k_secp_verify(
     u32 sr[16], pr[16];
     load_words(sigs + 4 * (u64)i, sr, 4);
     load_words(pubs + 4 * (u64)i, pr, 4);
-    secp_sig g;
+    secp_pro pro;
     fe x, y;
-    u32 st = secp_decode_verify<C>(sr, pr, g, x, y);
+    u32 st;
+    if constexpr (SHARED) {
+      secp_sig g;
+      st = secp_decode_verify<C>(sr, pr, g, x, y);
+    } else {
+      u32 dr[8];
+      load_words(digs + 2 * (u64)i, dr, 2);
+      secp_prologue_verify<C, true>(sr, dr, pr, pro);
+      st = pro.status;
+    }
     if (st == ST_OK) {
       bool exc = false;
-      const jac P = secp_point<C>(i, x, y, sc, tab, CombDev{comb}, exc);
+      jac P;
+      if constexpr (SHARED)
+        P = secp_point<C>(i, x, y, sc, tab, CombDev{comb}, exc);
+      else
+        P = secp_ladder_wide<C>(pro, tab, CombDev{comb}, exc);
       if (exc) {
         st = ST_PENDING;
         pend_list[atomicAdd(pend_count, 1u)] = i;
@@ -635,30 +690,6 @@ __global__ __launch_bounds__(64) void k_secp_verify_careful(const uint4* __restr
 
 static __global__ void k_fill_u32(u32* p, u32 v, u32 n) {
   for (u32 i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = v;
-}
-
-// one recovery by itself (the streamed kernel's tiles): the status (ST_PENDING when the ladder met an
-// exceptional addition and the careful pass must redo the item) and the key X || Y (zeros unless
-// ST_OK)
-template <class C>
-DEV u32 secp_item(const u32 sr[16], const u32 dr[8], STabDev& tab, const CombDev& comb, u32 o[16]) {
-  secp_pro pro;
-  secp_prologue<C, true>(sr, dr, pro);
-  u32 st = pro.status;
-  if (st == ST_OK) {
-    bool exc = false;
-    const jacs R = secp_ladder_s<C, 0>(pro, tab, comb, exc);
-    const jac Q = s_to_jac<C>(secp_comb<C>(R, pro, comb, exc));
-    if (exc)
-      st = ST_PENDING;
-    else
-      secp_output<C>(Q, o);
-  }
-  if (st != ST_OK) {
-#pragma unroll
-    for (int k = 0; k < 16; k++) o[k] = 0;
-  }
-  return st;
 }
 
 }  // namespace sigops

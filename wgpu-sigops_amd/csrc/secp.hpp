@@ -522,7 +522,7 @@ DEV u32 secp_decode_verify(const u32 sig_raw[16], const u32 pub_raw[16], secp_si
   return st;
 }
 
-template <class C>
+template <class C, bool WIDE = false>
 DEV void secp_prologue_verify(const u32 sig_raw[16], const u32 dig_raw[8], const u32 pub_raw[16], secp_pro& o) {
   typedef typename C::Fn Fn;
   secp_sig g;
@@ -533,7 +533,7 @@ DEV void secp_prologue_verify(const u32 sig_raw[16], const u32 dig_raw[8], const
   const fe sinv = finv<Fn>(to_mont<Fn>(fe_from_words(g.s)));
   const fe u1m = mont_mul<Fn>(to_mont<Fn>(fe_from_words(g.z)), sinv);
   const fe u2m = mont_mul<Fn>(to_mont<Fn>(fe_from_words(g.r)), sinv);
-  secp_scalars<C>(o, u1m, u2m, x, y);
+  secp_scalars<C, WIDE>(o, u1m, u2m, x, y);
 }
 
 // the verifier's final check on P = (X : Y : Z) (Jacobian) without an inversion: x(P) < p < 2n,
