@@ -240,7 +240,9 @@ int sigops_secp256r1_recover_address(sigops_ctx* ctx, const uint8_t* sigs, const
    batch and writes SIGOPS_STAGES durations in milliseconds: [0] bucketing (clear, histogram,
    scan, scatter), [1] a separate Ed25519 hashing pass, now always empty (the persistent kernel
    hashes each Ed25519 tile's challenges itself; the slot keeps the indices stable), [2] the
-   persistent verification kernel, [3] the careful pass for exceptional additions. ---- */
+   persistent verification kernel (with the stages before and after it that share inversions, where
+   the batch has them), [3] the careful pass for exceptional additions. A call of more than 2^22
+   items runs in pieces of that size; the durations are their sums. ---- */
 #define SIGOPS_STAGES 4
 int sigops_set_stage_timing(sigops_ctx* ctx, int on);
 int sigops_batch_stage_ms(sigops_ctx* ctx, float* ms);

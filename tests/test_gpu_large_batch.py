@@ -144,3 +144,47 @@ def test_sizes_where_the_launch_changes(rows):
         torch.cuda.synchronize()
         rows.check(at, dev[2].cpu().numpy(), dev[3].cpu().numpy(), n)
     ctx.close()
+
+
+def test_calls_in_pieces(rows):
+    """device calls of more than 2^22 items run in pieces of that size: results of ragged last pieces (1, 15
+    and 17 items and a larger one), and stage timing that covers every piece"""
+    piece = 1 << 22
+    ctx = sigops.Context(max_batch=piece + 30011)
+    s = torch.cuda.current_stream().cuda_stream
+    secp = [np.flatnonzero(rows.scheme == c) for c in (0, 1)]
+    cases = edge_cases.secp_verify_cases(1)
+    vst = np.array(edge_cases.secp_verify_expected(1, cases), np.uint8)
+    vcol = [torch.from_numpy(np.frombuffer(b"".join(c[j] for c in cases), np.uint8).reshape(len(cases), -1).copy()).cuda()
+            for j in (1, 2, 3)]
+    for curve, tail in ((0, 1), (1, 15), (1, 17), (0, 30011)):
+        n = piece + tail
+        print(f"pieces n={n}", flush=True)
+        out = torch.zeros(n, 64, dtype=torch.uint8, device="cuda")
+        st = torch.full((n,), 0xEE, dtype=torch.uint8, device="cuda")
+        at = torch.from_numpy(np.random.default_rng(tail).choice(secp[curve], n)).cuda()
+        sig, aux, want = (torch.from_numpy(x.copy()).cuda() for x in (rows.sig, rows.aux, rows.out))
+        sig, aux = sig[at], aux[at]
+        ctx.secp_recover_dev(curve, sig.data_ptr(), aux.data_ptr(), n, out.data_ptr(), st.data_ptr(), s)
+        torch.cuda.synchronize()
+        assert torch.equal(st, torch.from_numpy(rows.verdict).cuda()[at]) and torch.equal(out, want[at]), n
+        at = torch.from_numpy(np.random.default_rng(tail).integers(0, len(cases), n)).cuda()
+        v = [x[at] for x in vcol]
+        ctx.secp256r1_verify_dev(v[0].data_ptr(), v[1].data_ptr(), v[2].data_ptr(), n, st.data_ptr(), s)
+        torch.cuda.synchronize()
+        assert torch.equal(st, torch.from_numpy(vst).cuda()[at]), n
+        batch, at = rows.draw(n, tail, longest=60)
+        dev = _on_device(batch)
+        _enqueue(ctx, dev, s)
+        torch.cuda.synchronize()
+        rows.check(at, dev[2].cpu().numpy(), dev[3].cpu().numpy(), n)
+    # the larger piece is 140 times the last one, and so is its time
+    ctx.set_stage_timing(True)
+    _enqueue(ctx, dev, s)
+    whole = ctx.batch_stage_ms()["verify_kernel"]
+    ins, n, out, st = dev
+    _enqueue(ctx, (ins, tail, out, st), s)
+    part = ctx.batch_stage_ms()["verify_kernel"]
+    print(f"stage timing: {whole:.2f} ms, the last piece's items alone {part:.2f} ms", flush=True)
+    assert whole > 4 * part
+    ctx.close()

@@ -166,8 +166,11 @@ struct sigops_ctx {
   std::vector<uint8_t> s_bkt;      // bucket of every item
   void* noalloc_scratch = nullptr;  // device address of `scratch` on this context's device
   bool stage_timing = false;
-  bool stage_recorded = false;
-  hipEvent_t stage_ev[SIGOPS_STAGES + 1] = {};
+  struct StageEvents {
+    hipEvent_t ev[SIGOPS_STAGES + 1] = {};
+  };
+  std::vector<StageEvents> stage_ev;  // one for each piece of the longest timed call so far
+  size_t stage_pieces = 0;            // pieces of the last timed call
   std::vector<uint8_t> host_status;
   // host entry points: pinned staging of caller buffers, packed and unpacked by a thread pool
   std::unique_ptr<sigops_host::Pool> pool;
@@ -516,8 +519,9 @@ void sigops_destroy(sigops_ctx* c) {
   if (c->s_pin) (void)hipHostFree(c->s_pin);
   if (c->s_ctl) (void)hipHostFree(c->s_ctl);
   if (c->d_sctr) (void)hipFree(c->d_sctr);
-  for (hipEvent_t e : c->stage_ev)
-    if (e) (void)hipEventDestroy(e);
+  for (auto& p : c->stage_ev)
+    for (hipEvent_t e : p.ev)
+      if (e) (void)hipEventDestroy(e);
   for (void* p : {c->d_gtab_k1, c->d_gtab_r1, c->d_btab, c->d_scratch, c->d_lane_tab, (void*)c->d_pend, c->in.p, c->aux.p,
                   c->msg.p, c->off.p, c->out.p, c->st.p, c->sch.p, (void*)c->d_rank, (void*)c->d_work,
                   (void*)c->d_order, (void*)c->d_io, (void*)c->d_hq, (void*)c->d_horder, (void*)c->d_tlimbs,
@@ -738,23 +742,10 @@ int sigops_gen_ed25519_dev(sigops_ctx* c, uint64_t seed, size_t n, uint32_t corr
   return SIGOPS_OK;
 }
 
-int sigops_batch_dev(sigops_ctx* c, const void* d_schemes, const void* d_sigs, const void* d_aux, const void* d_msgs,
-                     const uint64_t* d_msg_off, size_t n, void* d_out, void* d_status, void* stream) {
-  if (!c) return SIGOPS_E_ARG;
-  if (n > c->max_batch) return fail(c, SIGOPS_E_ARG, "n exceeds max_batch");
-  if (n == 0) return SIGOPS_OK;
-  if (!d_schemes || !d_sigs || !d_aux || !d_msgs || !d_msg_off || !d_out || !d_status)
-    return fail(c, SIGOPS_E_ARG, "NULL buffer");
-  if (((uintptr_t)d_msgs & 3u) != 0) return fail(c, SIGOPS_E_ARG, "d_msgs must be 4-byte aligned");
-  if (n > STAGE_ITEMS) {
-    for (size_t a = 0; a < n; a += STAGE_ITEMS) {
-      const int rc = sigops_batch_dev(c, at(d_schemes, a), at(d_sigs, 64 * a), at(d_aux, 32 * a), d_msgs, d_msg_off + a,
-                                      std::min(n - a, STAGE_ITEMS), at(d_out, 64 * a), at(d_status, a), stream);
-      if (rc) return rc;
-    }
-    return SIGOPS_OK;
-  }
-  hipStream_t s = (hipStream_t)stream;
+// at most STAGE_ITEMS items of a call (arguments checked); first: its first piece
+static int batch_piece(sigops_ctx* c, bool first, const void* d_schemes, const void* d_sigs, const void* d_aux,
+                       const void* d_msgs, const uint64_t* d_msg_off, size_t n, void* d_out, void* d_status,
+                       hipStream_t s) {
   // the call's buffers and n go to device memory first (stream-ordered, by value at enqueue time),
   // so one captured graph serves every call and back-to-back enqueues do not race
   HIPCHK(c, sigops::launch_set_batch_io(c->d_io, {d_schemes, d_sigs, d_aux, d_msgs, d_msg_off, d_out, d_status,
@@ -792,9 +783,13 @@ int sigops_batch_dev(sigops_ctx* c, const void* d_schemes, const void* d_sigs, c
     return small ? sigops::launch_batch_small(L, on) : sigops::launch_batch(L, shared, on);
   };
   if (c->stage_timing) {
-    L.stage_ev = c->stage_ev;
+    if (first) c->stage_pieces = 0;
+    if (c->stage_ev.size() == c->stage_pieces) c->stage_ev.emplace_back();
+    for (hipEvent_t& e : c->stage_ev[c->stage_pieces].ev)
+      if (!e) HIPCHK(c, hipEventCreate(&e));
+    L.stage_ev = c->stage_ev[c->stage_pieces].ev;
     HIPCHK(c, launch(s));
-    c->stage_recorded = true;
+    c->stage_pieces++;
     return SIGOPS_OK;
   }
   if (!c->use_graph) {
@@ -818,6 +813,23 @@ int sigops_batch_dev(sigops_ctx* c, const void* d_schemes, const void* d_sigs, c
     }
   }
   HIPCHK(c, hipGraphLaunch(graph, s));
+  return SIGOPS_OK;
+}
+
+int sigops_batch_dev(sigops_ctx* c, const void* d_schemes, const void* d_sigs, const void* d_aux, const void* d_msgs,
+                     const uint64_t* d_msg_off, size_t n, void* d_out, void* d_status, void* stream) {
+  if (!c) return SIGOPS_E_ARG;
+  if (n > c->max_batch) return fail(c, SIGOPS_E_ARG, "n exceeds max_batch");
+  if (n == 0) return SIGOPS_OK;
+  if (!d_schemes || !d_sigs || !d_aux || !d_msgs || !d_msg_off || !d_out || !d_status)
+    return fail(c, SIGOPS_E_ARG, "NULL buffer");
+  if (((uintptr_t)d_msgs & 3u) != 0) return fail(c, SIGOPS_E_ARG, "d_msgs must be 4-byte aligned");
+  for (size_t a = 0; a < n; a += STAGE_ITEMS) {
+    const int rc = batch_piece(c, a == 0, at(d_schemes, a), at(d_sigs, 64 * a), at(d_aux, 32 * a), d_msgs,
+                               d_msg_off + a, std::min(n - a, STAGE_ITEMS), at(d_out, 64 * a), at(d_status, a),
+                               (hipStream_t)stream);
+    if (rc) return rc;
+  }
   return SIGOPS_OK;
 }
 
@@ -906,19 +918,25 @@ int sigops_set_fault(sigops_ctx* c, uint32_t flags) {
 int sigops_set_stage_timing(sigops_ctx* c, int on) {
   if (!c) return SIGOPS_E_ARG;
   HIPCHK(c, hipSetDevice(c->device));
-  if (on)
-    for (hipEvent_t& e : c->stage_ev)
-      if (!e) HIPCHK(c, hipEventCreate(&e));
   c->stage_timing = on != 0;
-  c->stage_recorded = false;
+  c->stage_pieces = 0;
   return SIGOPS_OK;
 }
 
 int sigops_batch_stage_ms(sigops_ctx* c, float* ms) {
   if (!c || !ms) return SIGOPS_E_ARG;
-  if (!c->stage_recorded) return fail(c, SIGOPS_E_ARG, "no timed batch since stage timing was switched on");
-  HIPCHK(c, hipEventSynchronize(c->stage_ev[SIGOPS_STAGES]));
-  for (int i = 0; i < SIGOPS_STAGES; i++) HIPCHK(c, hipEventElapsedTime(&ms[i], c->stage_ev[i], c->stage_ev[i + 1]));
+  if (!c->stage_pieces) return fail(c, SIGOPS_E_ARG, "no timed batch since stage timing was switched on");
+  float sum[SIGOPS_STAGES] = {};
+  for (size_t p = 0; p < c->stage_pieces; p++) {
+    hipEvent_t* ev = c->stage_ev[p].ev;
+    HIPCHK(c, hipEventSynchronize(ev[SIGOPS_STAGES]));
+    for (int i = 0; i < SIGOPS_STAGES; i++) {
+      float t = 0;
+      HIPCHK(c, hipEventElapsedTime(&t, ev[i], ev[i + 1]));
+      sum[i] += t;
+    }
+  }
+  memcpy(ms, sum, sizeof sum);
   return SIGOPS_OK;
 }
 
