@@ -899,4 +899,34 @@ DEV void secp_output(const jac& Q, u32 out_raw[16]) {
   secp_store_affine<C>(Q.X, Q.Y, finv<typename C::Fp>(Q.Z), out_raw);
 }
 
+// u1 G + u2 P on the wide tables (o from secp_carriers<C, true>)
+template <class C, class Tab, class Comb>
+DEV jac secp_ladder_wide(const secp_pro& pro, Tab& tab, const Comb& comb, bool& exc) {
+  const jacs Q = secp_ladder_s<C, 0>(pro, tab, comb, exc);
+  return s_to_jac<C>(secp_comb<C>(Q, pro, comb, exc));
+}
+
+// one recovery by itself, its inversions not shared: the status (ST_PENDING when the ladder met an
+// exceptional addition and the careful pass must redo the item) and the key X || Y (zeros unless
+// ST_OK)
+template <class C, class Tab, class Comb>
+DEV u32 secp_item(const u32 sr[16], const u32 dr[8], Tab& tab, const Comb& comb, u32 o[16]) {
+  secp_pro pro;
+  secp_prologue<C, true>(sr, dr, pro);
+  u32 st = pro.status;
+  if (st == ST_OK) {
+    bool exc = false;
+    const jac Q = secp_ladder_wide<C>(pro, tab, comb, exc);
+    if (exc)
+      st = ST_PENDING;
+    else
+      secp_output<C>(Q, o);
+  }
+  if (st != ST_OK) {
+#pragma unroll
+    for (int k = 0; k < 16; k++) o[k] = 0;
+  }
+  return st;
+}
+
 }  // namespace sigops
