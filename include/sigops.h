@@ -72,16 +72,20 @@ typedef struct {
   uint32_t bucket_order;    /* mixed batch: processing order of the buckets, 0 (default) secp256r1,
                                secp256k1, Ed25519 by decreasing SHA-512 block count; 1 secp256r1, Ed25519,
                                secp256k1; 2 secp256k1, secp256r1, Ed25519 */
-  uint32_t g_window;        /* every secp kernel: fixed-base window of the secp256k1 / secp256r1 G streams,
-                               8 or 9 bits (256 odd multiples of G in LDS, 4 fewer additions per
-                               secp256k1 item and 3 per secp256r1 item); 9 needs waves_per_simd 2; calls
-                               with a caller's generator table use 8. 0: 9 with two waves per SIMD
-                               (measured faster on the MI355X), 8 with one */
+  uint32_t g_window;        /* 0, 8 or 9 (9 not with waves_per_simd 1), without effect: it chose between two
+                               fixed-base tables that every call has since given up for wider ones
+                               (16-bit windows in HBM); calls with a caller's generator table use 8
+                               bits */
 } sigops_config;
 
 /* Creates a context on one GPU: uploads the fixed-base generator tables to HBM once (the
    reference re-uploads them on every call, src/secp256k1_ecdsa.rs:109) and allocates per-lane
-   scratch. cfg may be NULL. Returns NULL on failure. */
+   scratch. cfg may be NULL. Returns NULL on failure.
+   The first context on a device also builds the wide fixed-base tables (117 MB, shared by all of the
+   process's contexts there, about 7 ms); they are freed with the last one, so a process that creates
+   and destroys contexts one at a time builds them each time. Each context holds 112 bytes per item of
+   min(max_batch, 2^22), 470 MB by default: set max_batch to the largest call where many contexts
+   are kept. */
 sigops_ctx* sigops_create(const sigops_config* cfg);
 void sigops_destroy(sigops_ctx* ctx);
 /* text of the last error on this context ("" if none); valid until the next call */

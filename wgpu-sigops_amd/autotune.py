@@ -8,8 +8,6 @@ Candidates (each a Context setting; the library holds every variant's code):
                   atomics but a coarser tail at the end of the batch);
   * bucket_order: the processing order of the buckets (0: secp256r1, secp256k1, Ed25519 by
                   decreasing block count; 1: secp256r1, Ed25519, secp256k1; 2: secp256k1 first).
-  * g_window:     accepted and recorded, without effect: every kernel on the resident tables reads the
-                  16-bit windows, and a caller's table of G keeps 8 bits.
 blocks_per_cu follows waves (one 256-thread workgroup per SIMD wave): more workgroups than fit
 only queue behind the resident ones.
 
@@ -37,13 +35,10 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 TUNED_PATH = os.path.join(HERE, "tuned.json")
 # the library's defaults (a Context with no settings)
-DEFAULT = {"waves": 2, "tile_rounds": 1, "bucket_order": 0, "g_window": 9}
-# each knob changed alone, and the 8-bit windows with each of them (the one-wave kernel is built
-# with 8-bit windows only)
-_W8 = dict(DEFAULT, g_window=8)
-CANDIDATES = (DEFAULT, dict(DEFAULT, waves=1, g_window=8), dict(DEFAULT, tile_rounds=2), dict(DEFAULT, bucket_order=1),
-              dict(DEFAULT, bucket_order=2), _W8, dict(_W8, tile_rounds=2), dict(_W8, bucket_order=1),
-              dict(_W8, bucket_order=2))
+DEFAULT = {"waves": 2, "tile_rounds": 1, "bucket_order": 0}
+# each knob changed alone: no two candidates launch the same
+CANDIDATES = (DEFAULT, dict(DEFAULT, waves=1), dict(DEFAULT, tile_rounds=2), dict(DEFAULT, bucket_order=1),
+              dict(DEFAULT, bucket_order=2))
 
 
 def device_key(device=0):
@@ -66,8 +61,7 @@ def load(device=0, path=TUNED_PATH):
 
 
 def _name(c):
-    return (f"waves {c['waves']} tile_rounds {c['tile_rounds']} bucket_order {c['bucket_order']} "
-            f"g_window {c.get('g_window', 8)}")
+    return f"waves {c['waves']} tile_rounds {c['tile_rounds']} bucket_order {c['bucket_order']}"
 
 
 def tune(n=1 << 20, seed=2024, steps=5, rounds=3, candidates=CANDIDATES, write=True, path=TUNED_PATH, log=print):
