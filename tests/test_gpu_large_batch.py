@@ -188,3 +188,57 @@ def test_calls_in_pieces(rows):
     print(f"stage timing: {whole:.2f} ms, the last piece's items alone {part:.2f} ms", flush=True)
     assert whole > 4 * part
     ctx.close()
+
+
+def _rounds(ctx, rows, sizes, what):
+    for n in sizes:
+        print(f"{what} n={n}", flush=True)
+        batch, at = rows.draw(n, n, longest=300 if n > 200000 else 1 << 30)
+        dev = _on_device(batch)
+        _enqueue(ctx, dev, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        rows.check(at, dev[2].cpu().numpy(), dev[3].cpu().numpy(), (what, n))
+
+
+@pytest.mark.parametrize("order", [0, 1, 2])
+def test_tile_rounds(rows, order):
+    """tiles of 64 to 256 items in every bucket order, Ed25519 items of 1 to 40 blocks sharing them: tiles by
+    counter, by place and with shared inversions"""
+    for rounds in (1, 2, 3, 4):
+        ctx = sigops.Context(tuned=False, tile_rounds=rounds, bucket_order=order)
+        _rounds(ctx, rows, [25013, 70001, 200017] + ([786433] if rounds == 1 + order else []),
+                f"rounds={rounds} order={order}")
+        ctx.close()
+
+
+def test_one_wave_per_simd(rows):
+    """the persistent kernel built for one wavefront per SIMD shares inversions at every size"""
+    ctx = sigops.Context(tuned=False, waves=1)
+    _rounds(ctx, rows, [20481, 25013, 100003], "waves=1")
+    ctx.close()
+
+
+def test_graph_eager_and_timed_launches(rows):
+    """calls of every form in turn on one context, replayed from its graphs, launched eagerly and timed: on
+    four lanes per item, in one kernel, with shared inversions"""
+    sizes = (3000, 30011, 786433)
+    drawn = [rows.draw(n, n, longest=300) for n in sizes]
+    dev = [_on_device(b) for b, _ in drawn]
+    stream = torch.cuda.current_stream().cuda_stream
+    graph, eager = sigops.Context(), sigops.Context(use_graph=False)
+    for rep in range(3):
+        for ctx, timed in ((graph, False), (eager, False), (graph, True)):
+            ctx.set_stage_timing(timed)
+            for (_, at), d in zip(drawn, dev):
+                print(f"launch forms rep={rep} eager={ctx is eager} timed={timed} n={d[1]}", flush=True)
+                d[2].zero_()
+                d[3].fill_(0xEE)
+                _enqueue(ctx, d, stream)
+                if timed:
+                    ms = ctx.batch_stage_ms()
+                    assert all(v >= 0 for v in ms.values()) and ms["verify_kernel"] > 0
+                torch.cuda.synchronize()
+                rows.check(at, d[2].cpu().numpy(), d[3].cpu().numpy(), (rep, timed, d[1]))
+            ctx.set_stage_timing(False)
+    graph.close()
+    eager.close()
