@@ -85,7 +85,7 @@ template <class C, class Scratch, class Tab, class Comb>
 DEV u32 secp_recover_point(const u32 sr[16], u32 p, const Scratch& sc, Tab& tab, const Comb& comb) {
   secp_sig g;
   u32 st = secp_decode_sig<C>(sr, g);
-  u32 w[28] = {};  // an item without a point leaves zeros to secp_finish_lane
+  u32 w[28];  // without a point only the status is set (secp_finish_lane)
   if (st == ST_OK) {
     fe x, y;
     if (!secp_lift<C>(g.r, g.y_odd, x, y)) st = ST_NO_POINT;
@@ -148,11 +148,11 @@ DEV void secp_finish_lane(u32 first, u32 step, u32 end, const Dst& dst, const Sc
       before.v[8] = b2.x;
       const fe zi = mont_mul<F>(inv, before);
       inv = mont_mul<F>(inv, z_of(w));
+      const u32 keep = lane_mask(w[27] == ST_OK);
       fe X, Y;
 #pragma unroll
-      for (int k = 0; k < NL; k++) { X.v[k] = w[k]; Y.v[k] = w[9 + k]; }
+      for (int k = 0; k < NL; k++) { X.v[k] = w[k] & keep; Y.v[k] = w[9 + k] & keep; }
       secp_store_affine<C>(X, Y, zi, res);
-      const u32 keep = lane_mask(w[27] == ST_OK);
 #pragma unroll
       for (int c = 0; c < 4; c++)
         o[c] = make_uint4(res[4 * c] & keep, res[4 * c + 1] & keep, res[4 * c + 2] & keep, res[4 * c + 3] & keep);
