@@ -19,9 +19,9 @@ first one's. tuned.json (beside this file, keyed by the device) records the winn
 beats the default by more than the larger of 0.5 % and both candidates' spread; otherwise it
 records the default.
 
-Fixed by design rather than tuned: 29-bit limbs (one v_mad_u64_u32 per partial product with an
-even-aligned 64-bit accumulator), windows of 4 bits for per-lane tables, 8 bits for Ed25519's LDS
-table.
+Fixed by design rather than tuned: 29-bit limbs (one 64-bit multiply-add per partial product with
+an even-aligned accumulator), windows of 4 bits for per-lane tables, 16 bits for the fixed-base
+tables.
 
 Run on a GPU:  python wgpu-sigops_amd/autotune.py [--n 1048576] [--steps 5] [--rounds 3]
 """

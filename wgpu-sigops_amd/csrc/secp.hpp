@@ -155,8 +155,8 @@ DEV jac jmadd(const jac& P, const fe& x2, const fe& y2, bool& exc) {
 // Points carry W = 2Y in place of Y: the doubling's 4XY^2 = X W^2 and 8Y^4 = W^4 / 2 then need no
 // scaling, and W3 = 2 M (S - X3) - W^4 is a difference of two products that takes one reduction, as
 // the addition's W3 = 2 (r (V - X3) - W1 J) is. The subtractions of X3 and the factors 2 and 3 are
-// part of the products' carry chains. VALU instructions (secp256k1): doubling 1,015 against jdbl's
-// 1,280, mixed addition 1,760 against jmadd's 2,018.
+// part of the products' carry chains. VALU instructions (secp256k1): doubling 1,055 against jdbl's
+// 1,280, mixed addition 1,740 against jmadd's 2,018.
 struct jacs {
   sfe X, W, Z;
 };

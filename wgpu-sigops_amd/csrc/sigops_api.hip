@@ -95,10 +95,11 @@ void comb_release(int device) {
 constexpr size_t STAGE_ITEMS = 1u << 22;
 
 // Host batches from this size on are streamed unless the caller has chosen (sigops_set_streaming).
-// Streamed against copied, ms per call (messages up to 4 KB): 3.42 / 2.58 at 65,536 items, 3.62 / 3.27 at
-// 100,003, 5.36 / 5.08 at 200,000, 6.61 / 6.74 at 262,144, 9.36 / 9.76 at 400,000, 20.9 / 22.6 at 2^20: the
-// copied batch's tiles are placed (TileClaims) and its inversions shared, which below some four tiles
-// per wavefront saves more than the overlap with the copies.
+// Streamed / copied, ms per call: messages up to 4 KB on a fifth of the items (log-uniform lengths) 1.64 /
+// 1.52 at 20,000 items, 2.95 / 1.90 at 50,000, 5.19 / 4.98 at 200,000, 6.53 / 6.47 at 262,144; the same with
+// 4 KB each 4.36 / 2.69 at 50,000, 9.23 / 8.02 at 200,000; Ed25519 items only with 4 KB each, which moves
+// the most bytes an item, 8.56 / 5.65 at 50,000, 22.3 / 21.2 at 200,000; with 32 bytes each 2.16 / 1.41 and
+// 4.89 / 4.57: the copied form is the faster one below, whatever the messages.
 constexpr size_t STREAM_FROM = 1u << 18;
 
 constexpr uint8_t CANARY = 0xEE;
