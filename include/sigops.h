@@ -185,9 +185,10 @@ int sigops_ed25519_verify_strict_dev(sigops_ctx* ctx, const void* d_sigs, const 
 int sigops_batch(sigops_ctx* ctx, const uint8_t* schemes, const uint8_t* sigs, const uint8_t* aux,
                  const uint8_t* msgs, const uint64_t* msg_off, size_t n, uint8_t* out, uint8_t* status);
 /* How sigops_batch moves a host batch (no counterpart in the reference). Streamed (on = 1: for
-   n >= 4096; the default without a call: for n >= 262144): the host packs the batch into pinned, device-mapped memory chunk by chunk while
-   one persistent launch already processes the published chunks, reading them over PCIe, and the
-   results come back the same way as tiles finish, so packing, transfers and compute overlap.
+   n >= 4096; the default without a call: for n >= 262144): the host packs the batch into pinned,
+   device-mapped memory chunk by chunk while one persistent launch already processes the published
+   chunks, reading them over PCIe, and the results come back the same way as tiles finish, so
+   packing, transfers and compute overlap.
    Off: the whole batch is copied to the device, processed, and copied back. Both give the same
    results; a streamed launch that cannot take every chunk (its waits are bounded) is redone the
    other way. */

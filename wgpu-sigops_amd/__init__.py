@@ -256,8 +256,9 @@ class Context:
         return [(a, min(n, a + step)) for a in range(0, n, step)] or [(0, 0)]
 
     def set_streaming(self, on):
-        """host batches streamed through pinned memory while the kernel runs (default), or copied
-        to the device first (sigops_set_streaming); the results are the same"""
+        """host batches streamed through pinned memory while the kernel runs (from 4,096 items on; without
+        a call from 262,144 on), or copied to the device first (sigops_set_streaming); the results are
+        the same"""
         self._call(lib().sigops_set_streaming, 1 if on else 0)
 
     HOST_PHASES = ("head_packed_launched", "all_packed", "all_unpacked", "launch_done", "call_done", "launch_gpu_ms")
