@@ -202,7 +202,8 @@ int sigops_batch_host_ms(sigops_ctx* ctx, float* ms);
 
 /* device pointers (d_msgs non-NULL, 4-byte aligned and readable 16 bytes past the last message), enqueued
    on `stream`; the context's bucketing and lane scratch are shared, so calls on one context must
-   not overlap on the device */
+   not overlap on the device. A stream that is being captured records the call's kernels, for the
+   pointers and n given */
 int sigops_batch_dev(sigops_ctx* ctx, const void* d_schemes, const void* d_sigs, const void* d_aux,
                      const void* d_msgs, const uint64_t* d_msg_off, size_t n, void* d_out, void* d_status,
                      void* stream);

@@ -242,3 +242,35 @@ def test_graph_eager_and_timed_launches(rows):
             ctx.set_stage_timing(False)
     graph.close()
     eager.close()
+
+
+def test_calls_in_a_captured_graph(rows):
+    """calls of every form recorded into the caller's own graph, on a context that has run only one of them:
+    every replay, with eager calls on the same context between them, gives the oracle's results"""
+    ctx = sigops.Context()
+    s = torch.cuda.Stream()
+    warm, warm_at = rows.draw(1000, 1)
+    warm = _on_device(warm)
+    _enqueue(ctx, warm, s.cuda_stream)
+    torch.cuda.synchronize()
+    for n in (1000, 30011, 786433):
+        print(f"captured call n={n}", flush=True)
+        batch, at = rows.draw(n, n, longest=300)
+        dev = _on_device(batch)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            _enqueue(ctx, dev, s.cuda_stream)
+        for replay in range(4):
+            dev[2].zero_()
+            dev[3].fill_(0xEE)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            rows.check(at, dev[2].cpu().numpy(), dev[3].cpu().numpy(), (n, replay))
+            warm[3].fill_(0xEE)
+            _enqueue(ctx, warm, torch.cuda.current_stream().cuda_stream)
+            torch.cuda.synchronize()
+            rows.check(warm_at, warm[2].cpu().numpy(), warm[3].cpu().numpy(), (n, replay))
+        del graph
+    ctx.close()

@@ -793,7 +793,12 @@ static int batch_piece(sigops_ctx* c, bool first, const void* d_schemes, const v
     c->stage_pieces++;
     return SIGOPS_OK;
   }
-  if (!c->use_graph) {
+  // a caller who captures the stream gets the kernels in the graph captured: as a child graph the
+  // context's own gave right results on the first replay only (and its first use would be captured
+  // inside the caller's capture)
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  if (s) HIPCHK(c, hipStreamIsCapturing(s, &capturing));
+  if (!c->use_graph || capturing != hipStreamCaptureStatusNone) {
     HIPCHK(c, launch(s));
     return SIGOPS_OK;
   }
